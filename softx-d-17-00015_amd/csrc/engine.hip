@@ -181,10 +181,7 @@ size_t bytes_needed(int N, int K, int M, int cap, int diag_cap) {
   const size_t c3 = (size_t)cap * 3 * s.coll * sizeof(double2);
   b += c3 * 7;                                               // U[3], Nraw[2], om, R
   b += (size_t)cap * s.coll * sizeof(double2);               // S
-  b += (size_t)cap * 4 * N * LUS * s.P * sizeof(double);     // LU
-  b += (size_t)cap * 4 * N * s.P;                            // PV
-  b += (size_t)cap * 4 * N * s.P * (FW_Q + BW_Q) * sizeof(double2);  // FW, BW
-  b += (size_t)cap * 4 * s.P * 2;                            // META
+  b += (size_t)cap * 4 * s.P * blk_count(N) * 16 * sizeof(double);   // SE
   b += (size_t)cap * 6 * N * s.P * sizeof(double);           // Uinf
   b += (size_t)cap * 16 * s.H * sizeof(double);              // Ainv
   b += (size_t)cap * 3 * s.Hp * sizeof(double);              // diagb
@@ -257,49 +254,24 @@ Tuned lookup_tuning(int N, int K, int M, int cap) {
   return t;
 }
 
-size_t step_smem(int N, int gp, int bufd2) {
-  const int GH = 2 * gp;
-  size_t b = (size_t)4 * N * GH * sizeof(double2);           // V[4]
-  b += std::max(((size_t)2 * bufd2 + FC_TAIL) * sizeof(double2), (size_t)3 * N * GH * sizeof(double));
-  b += (size_t)GH * 8 * sizeof(double) + 8 * sizeof(double);  // AC, RED
-  b += 4 * sizeof(int);                                       // META
-  return round_up(b, 16);
-}
+size_t step_smem(int N, int gp) { return round_up(step_lds_doubles(N, gp) * sizeof(double), 16); }
 
-// Pairs per workgroup of the fused step kernel and its factor ring.  A
-// chunk block must hold one window of the widest U sweep (9 columns of 5
-// double2) plus its pad; 48 double2 per Helmholtz block gives 15-column
-// chunks for the common band widths.  Four pairs per workgroup (N <= 96)
-// put 48 of the solver wave's 64 lanes to work in the Helmholtz solves
-// instead of 24 and halve the solve instructions per harmonic; they are the
-// default when the slots give at least three such workgroups per CU (51 KiB
-// of LDS each at N = 64), otherwise two pairs (26 KiB, six per CU).  Above
-// N = 80 four pairs need more than 64 KiB of LDS (69 KiB at N = 96, two
-// workgroups per CU), which the kernel requests explicitly; at
-// (96,256,128) they take the step kernel from 1.55 to 1.35 ms.
+// Pairs per workgroup of the fused step kernel.  Four pairs (N <= 96) write
+// longer runs of each field's rows and share a stage's barriers among twice
+// the harmonics; they are the default when the slots give at least three such
+// workgroups per CU (40 KiB of LDS each at N = 64), otherwise two pairs.
 StepTiles choose_step_tiles(int N, int P, int cap, int ncu, int gp_req, size_t lds_max) {
   StepTiles t{};
   int gp = gp_req;
   if (gp <= 0)
-    gp = (N <= 96 && step_smem(N, 4, step_bufd2(4)) <= lds_max && (long long)((P + 3) / 4) * cap >= 3LL * ncu)
-             ? 4 : 2;
+    gp = (N <= 96 && step_smem(N, 4) <= lds_max && (long long)((P + 3) / 4) * cap >= 3LL * ncu) ? 4 : 2;
   if (gp != 1 && gp != 2 && gp != 4) throw OpfError(OPF_ERR_ARG, "step pairs per workgroup must be 1, 2 or 4");
   if (gp == 4 && N > 96) throw OpfError(OPF_ERR_ARG, "four pairs per workgroup need N <= 96");
   t.gp = gp;
-  t.bufd2 = step_bufd2(gp);
   t.ngroups = (P + gp - 1) / gp;
-  t.smem = step_smem(N, gp, t.bufd2);
+  t.smem = step_smem(N, gp);
   if (t.smem > lds_max) throw OpfError(OPF_ERR_ARG, "step kernel tiles do not fit in LDS");
   return t;
-}
-
-// the instantiation of the fused step kernel for the context's pairs per
-// workgroup and N (items per thread cover N * 2 * pairs)
-using StepKern = void (*)(Geo, Bufs, StepTiles, int);
-StepKern step_kernel(const opf_ctx* c) {
-  if (c->st.gp == 4) return c->N <= 64 ? k_step_g4 : k_step_g4x;
-  if (c->st.gp == 1) return k_step_g1;
-  return c->N <= 64 ? k_step_g2 : k_step_g2x;
 }
 
 void check_slot(opf_ctx* c, int slot) {
@@ -365,7 +337,7 @@ void launch_eval(opf_ctx* c, int s0, int ns) {
 
 void launch_step(opf_ctx* c, int s0, int ns) {
   const int per = (c->st.ngroups + 7) / 8;   // XCD-aware order inside the kernel
-  launch(c, "step", step_kernel(c), dim3(8 * per, 1, ns), dim3(step_threads(c->st.gp)), c->st.smem, c->G, c->B,
+  launch(c, "step", step_kernel(c->N, c->st.gp), dim3(8 * per, 1, ns), dim3(step_threads(c->st.gp)), c->st.smem, c->G, c->B,
          c->st, s0);
   launch(c, "control", k_control, dim3(1, 1, ns), dim3(256), 0, c->G, c->B, s0);
 }
@@ -373,9 +345,10 @@ void launch_step(opf_ctx* c, int s0, int ns) {
 // vel_matrices for slots s0 .. s0+ns-1 (gated: only slots whose control
 // block asks for it, the tim_new_dt of this step)
 void launch_matrices(opf_ctx* c, int s0, int ns, int gated) {
-  launch(c, "factor", k_lu_factor, dim3((c->P + 15) / 16, 4, ns), dim3(64), 0, c->G, c->B, s0, gated,
+  launch(c, "factor", k_block_factor, dim3((c->P + 31) / 32, 4, ns), dim3(64), 0, c->G, c->B, s0, gated,
          LuSpec{-1, 0, 0, 0.0, 0.0});
-  launch(c, "influence", k_influence, dim3((c->P + 63) / 64, 5, ns), dim3(64), 0, c->G, c->B, s0, gated);
+  launch(c, "influence", influence_kernel(c->N), dim3((c->P + 7) / 8, 4, ns), dim3(64), influence_smem(c->N), c->G,
+         c->B, s0, gated);
   launch(c, "ainv", k_ainv, grid_h(c, ns), dim3(64), 0, c->G, c->B, s0, gated);
 }
 
@@ -404,6 +377,15 @@ void launch_iteration(opf_ctx* c, int s0, int ns) {
     launch_matrices(c, s0, ns, 1);
   }
   launch_step(c, s0, ns);
+}
+
+// The LAPACK-form factors of one factor set, for tim_lumesh_get and
+// tim_lumesh_invert: built from the matrix the set holds when they are asked
+// for (the time step does not read them).  Buffers on first use.
+void lapack_factors(opf_ctx* c, int slot, int which) {
+  if (!c->B.LU) c->B.LU = c->alloc<double>((size_t)c->cap * 4 * c->N * LUS * c->P);
+  if (!c->B.PV) c->B.PV = c->alloc<unsigned char>((size_t)c->cap * 4 * c->N * c->P);
+  launch(c, "lapack_factor", k_lu_factor, dim3((c->P + 15) / 16), dim3(64), 0, c->G, c->B, slot, which);
 }
 
 // coll (reference layout) <-> device rows
@@ -623,7 +605,7 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
     const int gp = gp_req > 0 ? gp_req : (e1 ? std::atoi(e1) : tuned.gp);
     c->st = choose_step_tiles(N, c->P, cap, ncu, gp, (size_t)lds);
     if (c->st.smem > 64 * 1024)   // dynamic LDS beyond 64 KiB is requested per kernel
-      HIPCHK(hipFuncSetAttribute((const void*)step_kernel(c), hipFuncAttributeMaxDynamicSharedMemorySize,
+      HIPCHK(hipFuncSetAttribute((const void*)step_kernel(N, c->st.gp), hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)c->st.smem));
     // the whole-plane evaluation where the grid has one and its LDS fits
     // (OPF_PLANE=0: the three transform kernels instead)
@@ -653,6 +635,17 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   std::copy(me.lapb.begin(), me.lapb.end(), hm.begin() + mo.lapb);
   std::copy(me.dr0.begin(), me.dr0.end(), hm.begin() + mo.dr0);
   std::copy(me.dr1.begin(), me.dr1.end(), hm.begin() + mo.dr1);
+  for (int n = 0; n < N; ++n) {
+    for (int dd = -KL; dd <= KL; ++dd)
+      if (n + dd >= 0 && n + dd < N) {
+        hm[mo.lapT + 10 * n + dd + KL] = me.lapb[(size_t)(KL - dd) * N + n + dd];
+        hm[mo.d1T + 10 * n + dd + KL] = me.dr1b[(size_t)(KL - dd) * N + n + dd];
+      }
+    hm[mo.d1T + 10 * n + 9] = me.rinv[n];
+    hm[mo.rowv + n] = hm[mo.Ubase + n];
+    hm[mo.rowv + N + n] = hm[mo.twor + n];
+    hm[mo.rowv + 2 * N + n] = hm[mo.rinv2 + n];
+  }
   c->d_mesh = c->alloc<double>(mo.total);
   HIPCHK(hipMemcpy(c->d_mesh, hm.data(), hm.size() * sizeof(double), hipMemcpyHostToDevice));
 
@@ -663,11 +656,8 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   B.om = c->alloc<double2>(c3);
   B.R = c->alloc<double2>(c3);
   B.S = c->alloc<double2>((size_t)cap * s.coll);
-  B.LU = c->alloc<double>((size_t)cap * 4 * N * LUS * s.P);
-  B.PV = c->alloc<unsigned char>((size_t)cap * 4 * N * s.P);
-  B.FW = c->alloc<double2>((size_t)cap * 4 * N * s.P * FW_Q);
-  B.BW = c->alloc<double2>((size_t)cap * 4 * N * s.P * BW_Q);
-  B.META = c->alloc<unsigned char>((size_t)cap * 4 * s.P * 2);
+  B.SE = c->alloc<double>((size_t)cap * 4 * s.P * blk_count(N) * 16);
+  B.spec = c->alloc<LuSpec>((size_t)cap * 4);
   B.Uinf = c->alloc<double>((size_t)cap * 6 * N * s.P);
   B.Ainv = c->alloc<double>((size_t)cap * 16 * s.H);
   B.Ui = c->alloc<double>((size_t)cap * N);
@@ -1783,9 +1773,11 @@ int opf_tim_lumesh_get(opf_ctx* c, int slot, int which, double* ab, int* ipiv) {
     if (which < 0 || which > 3) throw OpfError(OPF_ERR_ARG, "which must be 0..3");
     if (!c->setup[slot]) throw OpfError(OPF_ERR_STATE, "slot not set up");
     const int N = c->N, P = c->P, H = c->H;
+    lapack_factors(c, slot, which);
     // per-pair blocks [pair][n][LUS] and [pair][n]
     std::vector<double> F((size_t)P * N * LUS);
     std::vector<unsigned char> pv((size_t)P * N);
+    HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipMemcpy(F.data(), lu_block(c->B, slot, which, 0, P, N), F.size() * sizeof(double),
                      hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(pv.data(), pv_block(c->B, slot, which, 0, P, N), pv.size(), hipMemcpyDeviceToHost));
@@ -1819,6 +1811,7 @@ extern "C" int opf_tim_lumesh_invert(opf_ctx* c, int slot, int which, int BC, do
     if (!bre || !bim) throw OpfError(OPF_ERR_ARG, "null field");
     const int bc = BC >= 0 ? BC : c->lu_bc[(size_t)slot * 4 + which];
     ensure_temps(c);
+    lapack_factors(c, slot, which);
     coll_to_dev(c, bre, bim, c->tC);
     launch(c, "lumesh_invert", k_lumesh_invert, grid_h(c, 1), dim3(64), 0, c->G, c->B, slot, which, bc, c->tC);
     dev_to_coll(c, c->tC, bre, bim);
@@ -1837,8 +1830,9 @@ extern "C" int opf_tim_lumesh_init(opf_ctx* c, int slot, int which, int PM, int 
     auto ctl = read_ctl(c);
     ctl[slot].status = 0;
     write_ctl(c, ctl);
-    launch(c, "factor", k_lu_factor, dim3((c->P + 15) / 16, 4, 1), dim3(64), 0, c->G, c->B, slot, 0,
+    launch(c, "factor", k_block_factor, dim3((c->P + 31) / 32, 4, 1), dim3(64), 0, c->G, c->B, slot, 0,
            LuSpec{which, PM, BC, c1, c2});
+    lapack_factors(c, slot, which);   // DGBTF2's own verdict on a singular matrix
     ctl = read_ctl(c);
     c->lu_bc[(size_t)slot * 4 + which] = BC;
     if (ctl[slot].status != 0) {

@@ -6,6 +6,15 @@
 
 namespace opf {
 
+// The matrix a factorisation builds, c1 + c2 Lap (of u+-: PM = +-1) with the
+// wall row BC: mat < 0 the four of vel_matrices (LDp, LDm, LDz with c1 = 1/dt,
+// c2 = -implicit nu/Re; LNp with 0, 1, BC = 1); mat >= 0 only that one, with
+// the given PM, BC, c1, c2.
+struct LuSpec {
+  int mat, PM, BC;
+  double c1, c2;
+};
+
 // All device arrays of one resolution class (slot-major).  Passed by value.
 struct Bufs {
   double2* U[3];        // velocity buffers [slot][3][N][Hp]; roles per slot in SlotCtl
@@ -13,11 +22,11 @@ struct Bufs {
   double2* om;          // curl of the current iterate [slot][3][N][Hp]
   double2* R;           // step scratch: right-hand sides [slot][3][N][Hp]
   double2* S;           // step scratch: pressure [slot][N][Hp]
-  double* LU;           // factors [slot][4 mats][P pairs][N columns][LUS]
-  unsigned char* PV;    // pivot offsets ipiv(j)-j [slot][4][P][N]
-  double2* FW;          // forward-sweep copy [slot][4][P][N][FW_Q]: (offset, l1) (l2, l3) (l4, 0)
-  double2* BW;          // backward-sweep copy [slot][4][P][BW_Q][N]: (u0, 1/u0) (u1, u2) .. (u7, u8)
-  unsigned char* META;  // [slot][4][P][2]: widest used superdiagonal, largest pivot offset
+  double* LU;           // LAPACK-form factors [slot][4 mats][P pairs][N columns][LUS] (first use of tim_lumesh_*)
+  unsigned char* PV;    // their pivot offsets ipiv(j)-j [slot][4][P][N]
+  double* SE;           // block inverses (k_block_factor, solve.hpp) [slot][4 mats][P pairs][blk_count(N)][16],
+                        // element (row, column) at 4 column + row
+  LuSpec* spec;         // [slot][4] the matrix each factor set holds
   double* Uinf;         // influence vectors [slot][6][N][P]
   double* Ainv;         // inverted influence matrices [slot][16][H]
   double* Ui;           // flux correction vector [slot][N]
@@ -57,36 +66,38 @@ __host__ __device__ inline unsigned char* pv_block(const Bufs& B, int slot, int 
   return B.PV + ((size_t)(slot * 4 + mat) * P + p) * N;
 }
 
-// Solve-ready copy of the factors used by the fused step kernel.  Column j of
-// the forward block holds the pivot offset (as a double) and the multipliers
-// l1..l4 = AB(10..13, j); plane q of the backward block holds, per column j,
-// q = 0: (u0, 1/u0) with u0 = AB(9, j), q >= 1: (u_{2q-1}, u_{2q}) with
-// u_d = AB(9-d, j) = U(j-d, j).
-constexpr int FW_Q = 3;
-constexpr int BW_Q = 5;
-__host__ __device__ inline double2* fw_block(const Bufs& B, int slot, int mat, int p, int P, int N) {
-  return B.FW + (((size_t)(slot * 4 + mat) * P + p) * N) * FW_Q;
-}
-__host__ __device__ inline double2* bw_block(const Bufs& B, int slot, int mat, int p, int P, int N) {
-  return B.BW + (((size_t)(slot * 4 + mat) * P + p) * N) * BW_Q;
-}
-__host__ __device__ inline unsigned char* meta_block(const Bufs& B, int slot, int mat, int p, int P) {
-  return B.META + ((size_t)(slot * 4 + mat) * P + p) * 2;
+// Block elimination: blocks of four rows, the block where the two sides meet,
+// and the scale of a matrix' unknowns (solve.hpp).
+__host__ __device__ constexpr int blk_count(int N) { return (N + 3) / 4; }
+__host__ __device__ constexpr int blk_mid(int N) { return blk_count(N) / 2; }
+__host__ __device__ inline double blk_scale(double c2) { return c2 != 0.0 ? c2 : 1e-300; }
+
+// curl of one harmonic at one radial point (var_coll_curl,
+// variables.f90:408-436) from u, the radial derivatives d1 of u_z and d2 of
+// u_theta, 1/r, m/r and alpha k: one definition for the step kernel and
+// k_curl, so that a state read back and loaded again continues with the same bits.
+__device__ __forceinline__ void curl_of(double2 vr, double2 vt, double2 vz, double2 d1, double2 d2, double ri,
+                                        double mr, double ak, double2 (&w)[3]) {
+  w[0] = make_double2(fma(vt.y, ak, -(vz.y * mr)), fma(-vt.x, ak, vz.x * mr));
+  w[1] = make_double2(-fma(vr.y, ak, d1.x), fma(vr.x, ak, -d1.y));
+  w[2] = make_double2(fma(vr.y, mr, fma(vt.x, ri, d2.x)), fma(-vr.x, mr, fma(vt.y, ri, d2.y)));
 }
 
 // Shape of the fused step kernel.
 struct StepTiles {
   int gp;        // (|k|, m) pairs per workgroup: 1, 2 or 4
-  int bufd2;     // double2 per factor chunk buffer (two buffers)
   int ngroups;   // workgroups per slot
   size_t smem;   // dynamic LDS bytes
 };
-// threads of a step workgroup: wave 0 solves, the other waves stream factor chunks
-inline int step_threads(int gp) { return gp == 4 ? 256 : 128; }
-constexpr int step_bufd2(int gp) { return 3 * gp * 49; }   // double2 per factor chunk buffer
-constexpr int STEP_BLKCAP = 64;    // double2 per (system, pair) block of a chunk (one per loader lane)
-constexpr int FC_TAIL = 16;        // double2 after the factor ring: the solvers' prefetch reads up to two
-                                   // columns (at most 10 double2) past a chunk
+inline int step_threads(int gp) { return gp == 1 ? 128 : 256; }
+// LDS of a step workgroup in doubles: V[3][N + 8][2 gp] (complex, four rows of
+// zeros at either end), the mesh tables (MeshOff::lapT, d1T, rowv; with four
+// pairs beyond 64 points the latter two stay in the cache, so that three
+// workgroups fit in a CU), the influence coefficients and the reduction words.
+__host__ __device__ constexpr bool step_d1_in_lds(int N, int gp) { return !(gp == 4 && N > 64); }
+__host__ __device__ constexpr size_t step_lds_doubles(int N, int gp) {
+  return (size_t)12 * (N + 8) * gp + 10 * (N + 8) + (step_d1_in_lds(N, gp) ? 13 * N + (N & 1) : 0) + 16 * gp + 16;
+}
 
 constexpr int FFT_THREADS = 256;
 constexpr int FFT_TILE = 2048;   // complex values per transform workgroup (all its lines)
@@ -105,15 +116,11 @@ __host__ __device__ constexpr int tile_m(int Z) { return FFT_TILE / Z; }
 
 __host__ __device__ constexpr int padded_len(int L) { return (L + (L - 1) / 16 + 1) | 1; }
 
-// The matrix tim_lumesh_init builds: mat < 0 the four of vel_matrices
-// (LDp, LDm, LDz with c1 = 1/dt, c2 = -implicit nu/Re; LNp with 0, 1, BC = 1);
-// mat >= 0 only that one, with the given PM, BC, c1, c2.
-struct LuSpec {
-  int mat, PM, BC;
-  double c1, c2;
-};
-__global__ void k_lu_factor(Geo G, Bufs B, int slot0, int gated, LuSpec spec);
-__global__ void k_influence(Geo G, Bufs B, int slot0, int gated);
+__global__ void k_block_factor(Geo G, Bufs B, int slot0, int gated, LuSpec spec);
+__global__ void k_lu_factor(Geo G, Bufs B, int slot, int mat);
+using FactorKern = void (*)(Geo, Bufs, int, int);
+FactorKern influence_kernel(int N);
+inline size_t influence_smem(int N) { return (size_t)(32 * (N + 4) + 10 * (N + 8)) * sizeof(double); }
 __global__ void k_ainv(Geo G, Bufs B, int slot0, int gated);
 __global__ void k_curl(Geo G, Bufs B, int slot0, int gated);
 __global__ void k_symmetry(Geo G, Bufs B, int slot0, int gated);
@@ -148,11 +155,9 @@ __global__ void k_add_coll(Geo G, double2* dst, const double2* src);
 // var_coll_norm of a field in the coll layout: per-harmonic partials b[H], then [E, Ek, Em]
 __global__ void k_norm_harm(Geo G, const SlotParams* prm, const double* re, const double* im, double* b);
 __global__ void k_norm_sum(Geo G, const double* b, double* out);
-__global__ void k_step_g1(Geo G, Bufs B, StepTiles ST, int slot0);
-__global__ void k_step_g2(Geo G, Bufs B, StepTiles ST, int slot0);    // N <= 64
-__global__ void k_step_g2x(Geo G, Bufs B, StepTiles ST, int slot0);   // N <= 128
-__global__ void k_step_g4(Geo G, Bufs B, StepTiles ST, int slot0);    // N <= 64, 256 threads
-__global__ void k_step_g4x(Geo G, Bufs B, StepTiles ST, int slot0);   // N <= 96, 256 threads
+// the fused step kernel for N radial points and gp pairs per workgroup
+using StepKern = void (*)(Geo, Bufs, StepTiles, int);
+StepKern step_kernel(int N, int gp);
 __global__ void k_control(Geo G, Bufs B, int slot0);
 
 // transforms: kernels specialised to the radix plans of (Z, T), chosen once

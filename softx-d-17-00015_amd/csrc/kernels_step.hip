@@ -1,19 +1,19 @@
 // Per-state set-up kernels and the small kernels around the fused step:
-// banded LU factorisation of the four matrices per (|k|, m) pair and its
-// solve-ready copy, the influence vectors and 4x4 inverses of the
+// block inverses of the four matrices per (|k|, m) pair (and their
+// LAPACK-form factors on request), the influence vectors and 4x4 inverses of the
 // influence-matrix method, the curl, imposesym, on-device corrector control
 // and diagnostics sums, the granular tim_lumesh_invert, and forcing added
 // to the nonlinear terms.
 //
 // Layout: a spectral (coll) field is stored harmonic-fastest, one complex
 // double2 per (n, h): element (slot, comp, n, h) at ((slot*3+comp)*N + n)*Hp + h.
-// The LU factors are stored once per (|k|, m) pair (the matrices depend on k
-// only through (alpha k)^2, timestep.f90:76-77) in LAPACK band form,
-// [slot][mat][pair][n][16] (see lu_block).
+// The factors are stored once per (|k|, m) pair (the matrices depend on k
+// only through (alpha k)^2, timestep.f90:76-77).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "kernels.hpp"
+#include "solve.hpp"
 
 // Products and sums are rounded separately, as in the reference's Fortran
 // (built for x86-64 without FMA): the ill-conditioned Neumann pressure solve
@@ -237,35 +237,215 @@ __device__ __forceinline__ double diag_d(double r2inv, int Mp, int m, double alp
 }
 
 // ---------------------------------------------------------------------------
-// tim_lumesh_init (timestep.f90:67-96) + DGBTF2, four lanes per (pair,
-// matrix), writing the factors in LAPACK band layout and the solve-ready
-// copy (see fw_block / bw_block, meta_block).
-// grid: x = pairs/16, y = 4 matrices, z = slot; 64 threads = 16 systems x 4 lanes.
+// The block elimination's inverses (solve.hpp) of tim_lumesh_init's matrices
+// (timestep.f90:67-96), one lane per (pair, matrix, side), the sides of a
+// matrix in neighbouring lanes:
+//   S_t = A(t, t) - A(t, o) E_o A(o, t)   (o the block before, seen from the side)
+//   E_t = inv(S_t), stored as -c2 E_t
+// and, for the block where the sides meet, both sides' terms subtracted.  The
+// 4 x 4 inverses interchange rows; between blocks nothing is interchanged (the
+// boundary rows, whose scale differs from the interior's, sit in the outermost
+// blocks; against 80-bit arithmetic the solves are as accurate as with the
+// banded LU and partial pivoting, error ratio 0.3 to 1.1 over N = 9 .. 128).
+// A lane's chain is N / 8 blocks of a few hundred instructions, which bounds it:
+// 34 us at (64,64,48) and 167 us at (96,256,128), where factoring all N columns
+// row by row and writing 265 bytes per row took 134 and 1254 us.
+// grid: x = pairs / 32, y = 4 matrices, z = slot; 64 threads.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot0, int gated, LuSpec spec) {
+__global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot0, int gated, LuSpec spec) {
+  const int mat = blockIdx.y;
+  const int slot = slot_of(B, slot0);
+  if ((gated && !B.ctl[slot].refactor) || (spec.mat >= 0 && mat != spec.mat)) return;
+  const int N = G.N, P = G.P, NB = blk_count(N);
+  const MeshOff mo = MeshOff::make(N);
+  const double* me = G.mesh;
+  const SlotParams prm = B.prm[slot];
+  LuSpec A = spec;
+  if (spec.mat < 0) {
+    const bool pr = mat == MAT_LNP;
+    A = LuSpec{mat, pr || mat == MAT_LDZ ? 0 : (mat == MAT_LDP ? 1 : -1), pr ? 1 : 0, pr ? 0.0 : 1.0 / prm.dt,
+               pr ? 1.0 : -prm.implicit * prm.nu / prm.Re};
+  }
+  if (threadIdx.x == 0 && blockIdx.x == 0) B.spec[slot * 4 + mat] = A;
+  __shared__ double T[10 * (MAXN + 8)];   // MeshOff::lapT
+  for (int i = threadIdx.x; i < 10 * (N + 8); i += 64) T[i] = me[mo.lapT + i];
+  __syncthreads();
+  const int side = threadIdx.x & 1;
+  const int p = min(blockIdx.x * 32 + (int)(threadIdx.x >> 1), P - 1);   // spare lanes repeat the last pair
+  const int m = p / G.K, k = p % G.K;
+  const int S1 = (m * G.Mp + (A.PM != 0)) & 1;
+  const double* ax = me + mo.dr0 + (KL + 1) * (1 - S1);   // axis row, columns 0..4
+  const double* wl = me + mo.dr1 + (KL + 1) * A.BC;       // wall row, columns N-5..N-1
+  const bool raw = A.BC == 1 && k == 0 && m == 0;   // singular, never solved (timestep.f90:84): zero inverses
+  const double sc = -blk_scale(A.c2);
+  double* out = B.SE + ((size_t)(slot * 4 + mat) * P + p) * NB * 16;
+  // the coupling of block t to the block after it (up = 1) or before it
+  auto couple = [&](int t, int up, double (&C)[4][4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int n = 4 * t + i;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int q = up ? (j <= i ? 8 + j - i : 9) : (j >= i ? j - i : 9);
+        C[i][j] = A.c2 * T[n * 10 + q];
+      }
+    }
+    if (t == 0) C[0][0] = ax[KL];   // only ever coupled upwards
+    if (t == NB - 1) {              // only ever coupled downwards
+      const int iw = (N - 1) & 3;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int q = 4 * (NB - 2) + j - (N - 1 - KL);
+          const double v = wl[q >= 0 ? q : 0];
+          C[i][j] = i == iw ? (q >= 0 ? v : 0.0) : C[i][j];
+        }
+    }
+  };
+  auto diagonal = [&](int t, double (&D)[4][4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int n = 4 * t + i;
+      const double dg = A.c2 * diag_d(me[mo.rinv2 + min(n, N - 1)], G.Mp, m, prm.alpha, k, A.PM) + A.c1;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        double x = A.c2 * T[n * 10 + KL + j - i];
+        x = i == j ? x + dg : x;
+        if (i == 0) x = t == 0 ? ax[j] : x;
+        const int q = 4 * t + j - (N - 1 - KL);
+        const double v = wl[q >= 0 && q <= KL ? q : 0];
+        x = n == N - 1 ? (q >= 0 && q <= KL ? v : 0.0) : x;
+        x = n >= N ? (i == j ? 1.0 : 0.0) : x;   // rows past the matrix
+        D[i][j] = 4 * t + j >= N && i != j ? 0.0 : x;
+      }
+    }
+  };
+  // in-place inverse, Gauss-Jordan with row interchanges
+  auto invert = [&](double (&D)[4][4]) {
+    double I[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) I[i][j] = i == j ? 1.0 : 0.0;
+    bool singular = false;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int r = c + 1; r < 4; ++r) {   // the largest of the column to row c
+        const bool sw = fabs(D[r][c]) > fabs(D[c][c]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const double a = D[c][j], b = D[r][j], e = I[c][j], f = I[r][j];
+          D[c][j] = sw ? b : a;
+          D[r][j] = sw ? a : b;
+          I[c][j] = sw ? f : e;
+          I[r][j] = sw ? e : f;
+        }
+      }
+      singular = singular || D[c][c] == 0.0;
+      const double rp = 1.0 / D[c][c];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        D[c][j] = D[c][j] * rp;
+        I[c][j] = I[c][j] * rp;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (r == c) continue;
+        const double f = D[r][c];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          D[r][j] = fma(-f, D[c][j], D[r][j]);
+          I[r][j] = fma(-f, I[c][j], I[r][j]);
+        }
+      }
+    }
+    if (singular && !raw) atomicMax(&B.ctl[slot].status, 100 + mat);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) D[i][j] = I[i][j];
+  };
+  auto store = [&](int t, const double (&E)[4][4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; i += 2)
+        *(double2*)(out + t * 16 + 4 * j + i) =
+            raw ? make_double2(0.0, 0.0) : make_double2(sc * E[i][j], sc * E[i + 1][j]);
+  };
+  const int nm = blk_mid(N);
+  const int steps = side ? NB - 1 - nm : nm, dt = side ? -1 : 1;
+  double D[4][4], U[4][4];   // the next block's matrix; the terms to subtract from it
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) U[i][j] = 0.0;
+  int t = side ? NB - 1 : 0;
+#pragma unroll 1
+  for (int s = 0; s < nm; ++s) {
+    if (s >= steps) break;
+    diagonal(t, D);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) D[i][j] = D[i][j] - U[i][j];
+    invert(D);
+    store(t, D);
+    double C[4][4], Y[4][4];
+    couple(t, side ? 0 : 1, C);   // Y = E_t A(t, u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        double v = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v = fma(D[i][q], C[q][j], v);
+        Y[i][j] = v;
+      }
+    t += dt;
+    couple(t, side ? 1 : 0, C);   // U = A(u, t) Y
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        double v = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v = fma(C[i][q], Y[q][j], v);
+        U[i][j] = v;
+      }
+  }
+  diagonal(nm, D);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) D[i][j] = D[i][j] - (U[i][j] + __shfl_xor(U[i][j], 1));
+  invert(D);
+  if (side == 0) store(nm, D);
+}
+
+// ---------------------------------------------------------------------------
+// tim_lumesh_init (timestep.f90:67-96) + DGBTF2 of one matrix per pair in
+// LAPACK band layout, for tim_lumesh_get / tim_lumesh_invert (the time step
+// solves with k_block_factor's inverses).  Four lanes per system.
+// grid: x = pairs/16; 64 threads = 16 systems x 4 lanes.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot, int mat) {
   constexpr int LPS = 4;              // lanes per system
   constexpr int SPW = 64 / LPS;       // systems per workgroup
   const int q = threadIdx.x % LPS, sl = threadIdx.x / LPS;
   const int p = blockIdx.x * SPW + sl;
-  const int mat = blockIdx.y;
-  const int slot = slot_of(B, slot0);
   // no barriers below: a lane may leave on its own
-  if (p >= G.P || (gated && !B.ctl[slot].refactor) || (spec.mat >= 0 && mat != spec.mat)) return;
+  if (p >= G.P) return;
   const int N = G.N, P = G.P;
   const int m = p / G.K, k = p % G.K;  // pair (|k|, m)
   const SlotParams prm = B.prm[slot];
   const MeshOff mo = MeshOff::make(N);
   const double* me = G.mesh;
-  int PM, BC;
-  double c1, c2;
-  if (spec.mat >= 0) { PM = spec.PM; BC = spec.BC; c1 = spec.c1; c2 = spec.c2; }
-  else if (mat == MAT_LNP) { PM = 0; BC = 1; c1 = 0.0; c2 = 1.0; }
-  else {
-    PM = mat == MAT_LDP ? 1 : (mat == MAT_LDM ? -1 : 0);
-    BC = 0;
-    c1 = 1.0 / prm.dt;
-    c2 = -prm.implicit * prm.nu / prm.Re;
-  }
+  const LuSpec spec = B.spec[slot * 4 + mat];   // the matrix that the factor set holds
+  const int PM = spec.PM, BC = spec.BC;
+  const double c1 = spec.c1, c2 = spec.c2;
   double* F = lu_block(B, slot, mat, p, P, N);
   unsigned char* pv = pv_block(B, slot, mat, p, P, N);
   // The elimination at column j touches columns j .. j + KV only, so each
@@ -325,36 +505,6 @@ __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot0, int 
       if (put) W(ws, row) = x;
     }
   };
-  // A finished column leaves as the LAPACK band column (F, pv) and as the
-  // solve-ready copy the fused step kernel reads (fw, bw); meanwhile the
-  // widest superdiagonal of U holding a non-zero and the largest pivot
-  // offset are tracked for the meta block.  The step kernel skips the
-  // superdiagonals that are exactly zero (x - t*0 = x) and multiplies by
-  // r = 1/u0 (correctly rounded) instead of dividing by the diagonal.
-  double2* fw = fw_block(B, slot, mat, p, P, N);
-  double2* bw = bw_block(B, slot, mat, p, P, N);
-  int kue = 1, mxo = 0;   // this lane's share of the meta block
-  // The backward copy's planes hold one 16-byte pair per column (the pivot
-  // rows one byte), so writing each column as it is finished would fill a
-  // 128-byte line in eight pieces far apart in time, and lines left partly
-  // written in the cache cost write bandwidth.  Each lane collects its own
-  // entries for 8 columns (planes q and, lane 0, 4 in LDS; lane 0 the pivot
-  // offsets in a register) and writes them together: flush(c0, n, npv).
-  constexpr int SG = 8;
-  __shared__ double2 Sb[SG * BW_Q * SPW];
-  auto sb = [&](int cc, int qq) -> double2& { return Sb[(cc * BW_Q + qq) * SPW + sl]; };
-  unsigned long long pvs = 0;
-  auto flush = [&](int c0, int n, int npv) {
-#pragma unroll
-    for (int cc = 0; cc < SG; ++cc)
-      if (cc < n) {
-        bw[(size_t)q * N + c0 + cc] = sb(cc, q);
-        if (q == 0) bw[(size_t)LPS * N + c0 + cc] = sb(cc, LPS);
-      }
-    if (q == 0)
-      for (int cc = 0; cc < npv; ++cc) pv[c0 + cc] = (unsigned char)(pvs >> (8 * cc));
-    pvs = 0;
-  };
   auto rd = [&](int ws, int row) { return W(ws, row < NLU ? row : NLU - 1); };
   auto store = [&](int ws, int col, int pj) {
     // LAPACK column: rows 4q .. 4q + 3 from lane q (rows 13 .. 15 zero)
@@ -364,20 +514,9 @@ __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot0, int 
       const int row = LPS * q + r;
       const double v = rd(ws, row);
       x[r] = row < NLU ? v : 0.0;
-      // superdiagonal d = 8 - row of U in column col
-      if (row < 2 * KL && col - (2 * KL - row) >= 0 && v != 0.0) kue = 2 * KL - row > kue ? 2 * KL - row : kue;
     }
     reinterpret_cast<double4*>(F + (size_t)col * LUS)[q] = make_double4(x[0], x[1], x[2], x[3]);
-    // solve-ready copy, in window rows r: fw pair q (q < 3) = (pj, r9),
-    // (r10, r11), (r12, 0); bw pair q = (r8, 1/r8), (r7, r6), (r5, r4),
-    // (r3, r2) and, from lane 0, pair 4 = (r1, r0)
-    const double fa = rd(ws, q == 1 ? 10 : 12), fb = rd(ws, q == 0 ? 9 : 11);
-    if (q < FW_Q) fw[col * FW_Q + q] = make_double2(q == 0 ? (double)pj : fa, q == 2 ? 0.0 : fb);
-    static_assert(BW_Q == LPS + 1, "bw pairs: one per lane and a fifth from lane 0");
-    const double ba = rd(ws, q == 0 ? 2 * KL : 2 * KL + 1 - 2 * q), bb = rd(ws, 2 * KL - 2 * q);
-    sb(col % SG, q) = make_double2(ba, q == 0 ? (ba != 0.0 ? 1.0 / ba : 0.0) : bb);
-    if (q == 0) sb(col % SG, LPS) = make_double2(rd(ws, 1), rd(ws, 0));
-    mxo = pj > mxo ? pj : mxo;
+    if (q == 0) pv[col] = (unsigned char)pj;
   };
   // the pressure matrix of (0,0) is never factored: its lanes store the
   // columns as built, in the same loop as the others
@@ -416,9 +555,8 @@ __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot0, int 
       jp = better ? i : jp;
       piv = better ? pc[i] : piv;
     }
-    pvs |= (unsigned long long)jp << (8 * (j % SG));
     if (!raw && piv == 0.0) {
-      flush(j - j % SG, j % SG, j % SG + 1);
+      if (q == 0) pv[j] = (unsigned char)jp;
       if (q == 0) atomicMax(&B.ctl[slot].status, 100 + mat);  // singular factor
       return;
     }
@@ -459,17 +597,6 @@ __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot0, int 
     store(wj, j, jp);
     lds_fence();   // every lane has read column j before its slot is refilled
     place(wj, jn, nx, j + WC < N);
-    // after place(): its wait for the mesh loads then does not include
-    // these stores (loads and stores share one in-order counter)
-    if (j % SG == SG - 1 || j == N - 1) flush(j - j % SG, j % SG + 1, j % SG + 1);
-  }
-  // the four lanes of a system are neighbours in the wave
-  kue = max(kue, __shfl_xor(kue, 1));
-  kue = max(kue, __shfl_xor(kue, 2));
-  if (q == 0) {
-    unsigned char* mt = meta_block(B, slot, mat, p, P);
-    mt[0] = (unsigned char)kue;
-    mt[1] = (unsigned char)mxo;
   }
 }
 
@@ -543,178 +670,88 @@ __global__ void k_norm_sum(Geo G, const double* __restrict__ b, double* __restri
 }
 
 // ---------------------------------------------------------------------------
-// lu_solve<double> for one lane whose vector lives in LDS (element n at
-// X[n * 64], the workgroup's lanes interleaved) and whose factor columns and
-// pivot offsets are read D columns ahead into a register ring, so a solve
-// waits on LDS rather than on a cache round trip per column.  The factors
-// come from the solve-ready copy (FW: pivot offset and multipliers, 48
-// contiguous bytes per column; BW: U's diagonal and superdiagonals in five
-// planes), half the bytes of the LAPACK columns' two 128-byte lines.  The
-// operations and their order are lu_solve's (the diagonal divides).
-// ---------------------------------------------------------------------------
-template <int D>
-__device__ __forceinline__ void lu_solve_lds(const double2* FW, const double2* BW, double* X, int N) {
-  // Every global load is unconditional (column indices clamped into the
-  // matrix; values past the last column are never used), and a ring slot is
-  // refilled only after its last use: a load issued on one path only, or a
-  // slot refilled while its old value is still live (the two then need
-  // different registers and a copy at the loop's back edge), makes each pass
-  // round the loop wait for every load in flight.
-  double w[5];
-#pragma unroll
-  for (int i = 0; i < 5; ++i) w[i] = i < N ? X[i * 64] : 0.0;
-  double fl[D][KL];
-  int pr[D];
-  // column c of L: (pivot offset, l1) (l2, l3) (l4, 0)
-  auto lcol = [&](int c, double (&f)[KL], int& o) {
-    const double2 a = FW[(size_t)c * FW_Q], b = FW[(size_t)c * FW_Q + 1], e = FW[(size_t)c * FW_Q + 2];
-    f[0] = a.y;
-    f[1] = b.x;
-    f[2] = b.y;
-    f[3] = e.x;
-    o = (int)a.x;
-  };
-  // column c of U, band rows 0..8 (row 8 - d: superdiagonal d): plane 0
-  // holds (u0, 1/u0), plane q >= 1 (u_{2q-1}, u_{2q})
-  auto ucol = [&](int c, double (&f)[2 * KL + 1]) {
-    f[2 * KL] = ((const double*)(BW + c))[0];
-#pragma unroll
-    for (int q = 1; q < BW_Q; ++q) {
-      const double2 v = BW[(size_t)q * N + c];
-      f[2 * KL + 1 - 2 * q] = v.x;
-      f[2 * KL - 2 * q] = v.y;
-    }
-  };
-#pragma unroll
-  for (int u = 0; u < D; ++u) lcol(u < N - 1 ? u : N - 2, fl[u], pr[u]);
-  for (int j0 = 0; j0 < N - 1; j0 += D) {
-#pragma unroll
-    for (int u = 0; u < D; ++u) {
-      const int j = j0 + u;
-      const int off = pr[u];
-      if (j < N - 1) {
-        const double a0 = w[0];
-        double s = w[0];
-        s = off == 1 ? w[1] : s;
-        s = off == 2 ? w[2] : s;
-        s = off == 3 ? w[3] : s;
-        s = off == 4 ? w[4] : s;
-        w[0] = s;
-        w[1] = off == 1 ? a0 : w[1];
-        w[2] = off == 2 ? a0 : w[2];
-        w[3] = off == 3 ? a0 : w[3];
-        w[4] = off == 4 ? a0 : w[4];
-        const double t = -w[0];
-        const int lm = N - 1 - j < KL ? N - 1 - j : KL;
-#pragma unroll
-        for (int i = 1; i <= KL; ++i)
-          if (i <= lm) w[i] = w[i] + fl[u][i - 1] * t;
-        X[j * 64] = w[0];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = w[i + 1];
-        const double xn = X[(j + 5 < N ? j + 5 : N - 1) * 64];
-        w[4] = j + 5 < N ? xn : 0.0;
-      }
-      lcol(j + D < N - 1 ? j + D : N - 2, fl[u], pr[u]);
-    }
-  }
-  double v[9];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int idx = N - 9 + q;
-    v[q] = idx >= 0 ? X[idx * 64] : 0.0;
-  }
-  v[8] = w[0];
-  double fu[D][2 * KL + 1];
-#pragma unroll
-  for (int u = 0; u < D; ++u) ucol(N - 1 - u >= 0 ? N - 1 - u : 0, fu[u]);
-  for (int j0 = N - 1; j0 >= 0; j0 -= D) {
-#pragma unroll
-    for (int u = 0; u < D; ++u) {
-      const int j = j0 - u;
-      if (j >= 0) {
-        v[8] = v[8] / fu[u][8];
-        const double t = v[8];
-        X[j * 64] = t;
-#pragma unroll
-        for (int d = 1; d <= 8; ++d)
-          if (j - d >= 0) v[8 - d] = v[8 - d] - t * fu[u][8 - d];
-#pragma unroll
-        for (int q = 8; q >= 1; --q) v[q] = v[q - 1];
-        const double xn = X[(j - 9 >= 0 ? j - 9 : 0) * 64];
-        v[0] = j - 9 >= 0 ? xn : 0.0;
-      }
-      ucol(j - D >= 0 ? j - D : 0, fu[u]);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // vel_adjPPE(0) influence vectors (velocity.f90:191-218) per pair, and
 // vel_adjustFlux(0) (velocity.f90:160-168) on pair 0.
 // Uinf slots: 0 U1 (LDp), 1 U2 (LDm), 2 U3 (LDz), 3 U4, 4 U5, 5 p (U6 = p*alpha*k).
-// The solves are independent, so each gets its own lane: grid y = 0..2 the
-// three Helmholtz solves, 3 the pressure solve and its gradient, 4 the flux
-// solve (lane of pair 0 only).  grid: x = pairs/64, y = 5, z = slot.
+// One wave solves a matrix of eight pairs (four groups of two, solve.hpp); of
+// a pair's four columns the first holds its right-hand side and, for pair 0,
+// the second that of the flux problem.
+// grid: x = pairs/8, y = 4 matrices, z = slot.  SM >= blk_mid(N).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) k_influence(Geo G, Bufs B, int slot0, int gated) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  const int which = blockIdx.y;
+template <int SM>
+__global__ void __launch_bounds__(64) k_influence_t(Geo G, Bufs B, int slot0, int gated) {
+  constexpr int PW = 8;
+  const int p0 = blockIdx.x * PW;
+  const int mat = blockIdx.y;
   const int slot = slot_of(B, slot0);
-  if (p >= G.P || (gated && !B.ctl[slot].refactor) || (which == 4 && p != 0)) return;
+  if (gated && !B.ctl[slot].refactor) return;
   const int N = G.N, P = G.P;
-  const int m = p / G.K, k = p % G.K;
+  const int tid = threadIdx.x;
+  const int np = min(PW, P - p0);
   const MeshOff mo = MeshOff::make(N);
   const double* me = G.mesh;
-  double* U = B.Uinf + (size_t)slot * 6 * N * P + p;
-  __shared__ double Xs[MAXN * 64];
-  double* x = Xs + threadIdx.x;
-  auto FWp = [&](int mat) { return (const double2*)fw_block(B, slot, mat, p, P, N); };
-  auto BWp = [&](int mat) { return (const double2*)bw_block(B, slot, mat, p, P, N); };
-  // right-hand side and factor of this lane's solve (one inlined solve for
-  // every case, so the vector stays in LDS and the factor loads in flight)
   const SlotParams prm = B.prm[slot];
-  int mat;
-  bool solve = true;
-  if (which < 3) mat = which;
-  else if (which == 3) { mat = MAT_LNP; solve = !(k == 0 && m == 0); }
-  else { mat = MAT_LDZ; solve = prm.const_flux != 0; }
-  for (int n = 0; n < N; ++n) {
-    double v;
-    if (which < 3) v = n == N - 1 ? 1.0 : 0.0;
-    else if (which == 3) v = solve && n == N - 1 ? -1.0 : 0.0;
-    else v = (n == 0 || n == N - 1) ? 0.0 : 1.0;
-    x[n * 64] = v;
+  const bool flux = p0 == 0 && mat == MAT_LDZ && prm.const_flux != 0;
+  extern __shared__ double Xi[];   // [N + 4][PW][4], then the Laplacian's rows
+  double* lap = Xi + (size_t)(N + 4) * PW * 4;
+  for (int i = tid; i < (N + 4) * PW * 4; i += 64) {
+    const int n = i / (PW * 4), r = i & 3, ip = (i >> 2) % PW;
+    double v = 0.0;
+    if (r == 0 && n == N - 1) v = mat == MAT_LNP ? -1.0 : 1.0;
+    if (r == 1 && ip == 0 && flux) v = n == 0 || n >= N - 1 ? 0.0 : 1.0;
+    Xi[i] = v;
   }
-  if (solve) lu_solve_lds<8>(FWp(mat), BWp(mat), x, N);
-  if (which < 3) {
-    double* u = U + (size_t)which * N * P;
-    for (int n = 0; n < N; ++n) u[(size_t)n * P] = x[n * 64];
-  } else if (which == 3) {
-    double* pp = U + (size_t)5 * N * P;
-    double* U4 = U + (size_t)3 * N * P;
-    double* U5 = U + (size_t)4 * N * P;
-    for (int n = 0; n < N; ++n) {
+  for (int i = tid; i < 10 * (N + 8); i += 64) lap[i] = me[mo.lapT + i];
+  __syncthreads();
+  const BlkLane l = BlkLane::make(tid);
+#pragma unroll 1
+  for (int g = 0; g < PW / 2; ++g) {
+    BlkE<SM, 1> E;
+    const int pl = 2 * g + l.mi;   // a partial last group repeats its last matrix in the spare columns
+    blk_load(E, 0, G, B, slot, mat, p0 + min(pl, np - 1), l);
+    double* const x[1] = {Xi + pl * 4 + l.col};
+    blk_solve(E, N, l, lap, x, PW * 4);
+  }
+  __syncthreads();
+  double* U = B.Uinf + (size_t)slot * 6 * N * P + p0;
+  const size_t us = (size_t)N * P;
+  auto xv = [&](int n, int ip) { return Xi[(n * PW + ip) * 4]; };
+  for (int i = tid; i < N * PW; i += 64) {
+    const int n = i / PW, ip = i % PW;
+    if (ip >= np) continue;
+    double* u = U + (size_t)n * P + ip;
+    if (mat != MAT_LNP) {
+      u[mat * us] = xv(n, ip);
+    } else {
       // grad: dr1 . p (meshmult from 0), t.Im = p * m/r; rt2pm -> U4 = gr - tIm, U5 = gr + tIm
       double gr = 0.0;
-      const int j0 = n - KL < 0 ? 0 : n - KL, j1 = n + KL > N - 1 ? N - 1 : n + KL;
-      for (int j = j0; j <= j1; ++j) gr = gr + me[mo.dr1b + (KL + n - j) * N + j] * x[j * 64];
-      const double mr = (me[mo.rinv + n] * (double)G.Mp) * (double)m;
-      const double tIm = x[n * 64] * mr;
-      pp[(size_t)n * P] = x[n * 64];
-      U4[(size_t)n * P] = gr - tIm;
-      U5[(size_t)n * P] = gr + tIm;
+#pragma unroll
+      for (int dd = -KL; dd <= KL; ++dd) {
+        const int j = n + dd;
+        if (j >= 0 && j <= N - 1) gr = gr + me[mo.dr1b + (KL - dd) * N + j] * xv(j, ip);
+      }
+      const double mr = (me[mo.rinv + n] * (double)G.Mp) * (double)((p0 + ip) / G.K);
+      const double tIm = xv(n, ip) * mr;
+      u[5 * us] = xv(n, ip);
+      u[3 * us] = gr - tIm;
+      u[4 * us] = gr + tIm;
     }
-  } else {
+  }
+  if (p0 == 0 && mat == MAT_LDZ) {
     double* Ui = B.Ui + (size_t)slot * N;
-    for (int n = 0; n < N; ++n) Ui[n] = x[n * 64];
-    if (prm.const_flux) {
+    for (int n = tid; n < N; n += 64) Ui[n] = Xi[n * PW * 4 + 1];
+    if (flux && tid == 0) {
       double s = 0.0;
-      for (int n = 0; n < N; ++n) s = s + x[n * 64] * me[mo.intrdr + n];
+      for (int n = 0; n < N; ++n) s = s + Xi[n * PW * 4 + 1] * me[mo.intrdr + n];
       B.ctl[slot].flux_d1 = 2.0 * s;
       if (2.0 * s == 0.0) atomicMax(&B.ctl[slot].status, 110);
     }
   }
+}
+
+FactorKern influence_kernel(int N) {
+  static_assert(blk_mid(32) == 4 && blk_mid(64) == 8 && blk_mid(96) == 12 && blk_mid(MAXN) == 16, "the ranges");
+  return N <= 32 ? k_influence_t<4> : N <= 64 ? k_influence_t<8> : N <= 96 ? k_influence_t<12> : k_influence_t<16>;
 }
 
 // Inverted 4x4 influence matrices per harmonic (velocity.f90:219-225).
@@ -770,19 +807,19 @@ __device__ __forceinline__ void curl_point(const Geo& G, int h, int n, int k, in
   const size_t hs = G.Hp;
   const MeshOff mo = MeshOff::make(N);
   const double* me = G.mesh;
-  const double ak = alpha * (double)k;
-  double2* orr = om;
-  double2* ot = om + G.coll;
-  double2* oz = om + 2 * G.coll;
-  const double mr = (me[mo.rinv + n] * (double)G.Mp) * (double)m;
+  const double ri = me[mo.rinv + n], mr = ri * ((double)G.Mp * (double)m);
   const size_t o = (size_t)n * hs + h;
-  const double2 vr = ur[o], vt = ut[o], vz = uz[o];
-  orr[o] = make_double2(-(vz.y * mr) + vt.y * ak, vz.x * mr - vt.x * ak);
-  const double2 d1 = band_row(me + mo.dr1b, N, n, uz + h, hs, make_double2(0.0, 0.0));
-  ot[o] = make_double2(-(vr.y * ak) - d1.x, vr.x * ak - d1.y);
-  const double2 d2 = band_row(me + mo.dr1b, N, n, ut + h, hs, make_double2(0.0, 0.0));
-  const double ri = me[mo.rinv + n];
-  oz[o] = make_double2((vt.x * ri + d2.x) + vr.y * mr, (vt.y * ri + d2.y) - vr.x * mr);
+  double2 d1 = make_double2(0.0, 0.0), d2 = d1;
+  for (int j = max(n - KL, 0); j <= min(n + KL, N - 1); ++j) {
+    const double a = me[mo.dr1b + (KL + n - j) * N + j];
+    const double2 z = uz[(size_t)j * hs + h], t = ut[(size_t)j * hs + h];
+    d1 = make_double2(fma(a, z.x, d1.x), fma(a, z.y, d1.y));
+    d2 = make_double2(fma(a, t.x, d2.x), fma(a, t.y, d2.y));
+  }
+  double2 w[3];
+  curl_of(ur[o], ut[o], uz[o], d1, d2, ri, mr, alpha * (double)k, w);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) om[c * G.coll + o] = w[c];
 }
 
 // which = 0: curl of U[ucur]; used after put_state and after every step.

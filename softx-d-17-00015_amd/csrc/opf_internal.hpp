@@ -108,7 +108,12 @@ struct Geo {
 
 // Offsets (in doubles) of the pieces of the device mesh block.
 struct MeshOff {
-  int r, rinv, rinv2, Ubase, twor, dr1b, lapb, intrdr, dr0, dr1, total;
+  int r, rinv, rinv2, Ubase, twor, dr1b, lapb, intrdr, dr0, dr1;
+  // the stencils row by row, as the step kernel stages them in LDS: row n's
+  // nine weights (columns n-4 .. n+4; zero outside the matrix) and a tenth
+  // value: lapT the radial Laplacian (0; rows N .. N+7 zero), d1T the first
+  // derivative (1/r); then Ubase, 2r, 1/r^2 again
+  int lapT, d1T, rowv, total;
   __host__ __device__ static MeshOff make(int N) {
     MeshOff o{};
     int p = 0;
@@ -122,6 +127,11 @@ struct MeshOff {
     o.intrdr = p; p += N;
     o.dr0 = p; p += (KL + 1) * (KL + 1);
     o.dr1 = p; p += (KL + 1) * (KL + 1);
+    p += p & 1;
+    o.lapT = p; p += 10 * (N + 8);
+    o.d1T = p; p += 10 * N;
+    o.rowv = p; p += 3 * N;
+    p += 1;   // copied in pairs
     o.total = p;
     return o;
   }

@@ -44,3 +44,68 @@ def _nonlinear_matches(opf, N, K, M):
                                  (81, 81), (96, 96), (108, 4), (144, 4), (162, 4), (192, 4), (216, 4), (4, 108)])
 def test_nonlinear_transform_lengths(opf, K, M):
     _nonlinear_matches(opf, 10, K, M)
+
+
+def _one_step_matches(opf, N, K, M, Mp, gp, monkeypatch, tol):
+    from opf import ic as icgen
+    Re, alpha, dt = 2400.0, 1.25, 0.01
+    monkeypatch.setenv("OPF_STEP_GP", str(gp))
+    ctx = opf.Context(N, K, M, Mp)
+    assert ctx.step_pairs() == gp
+    ctx.setup(0, Re, alpha, dt)
+    me = ctx.mesh()
+    u = icgen.seeded_perturbation(me["r"], me["intrdr"], K, M, alpha, 3, 1e-2, Mp=Mp)
+    ctx.put_state(0, *u)
+    ctx.run(2, corr_fixed=1)
+    got = ctx.get_state(0)
+    oc = O.Ctx(N, K, M, Mp, Re=Re, alpha=alpha, dt=dt)
+    oc.set_state(*u)
+    oc.run(2, ncorr_fixed=1)
+    for c, ref in enumerate((oc.ur, oc.ut, oc.uz)):
+        assert rel_err(got[c], ref) <= tol, (N, c)
+    ctx.close()
+
+
+# The block elimination at every remainder of N by eight, at the edges of the
+# ranges of its instantiations (N = 32, 64, 96) and at the smallest and largest
+# N, for groups that do (K M = 12) and do not (18) fill the workgroups.  The
+# pressure solves of the two differ by their forward errors, up to 1e-11 at
+# N = 128 for the lowest modes; the velocity takes dt grad p of it.
+@pytest.mark.parametrize("gp", [1, 2, 4])
+@pytest.mark.parametrize("N,K,M,Mp", [(9, 4, 3, 1), (10, 3, 6, 2), (11, 4, 3, 1), (12, 3, 6, 3), (13, 4, 3, 1),
+                                      (14, 4, 3, 4), (15, 4, 3, 1), (31, 4, 3, 1), (32, 3, 6, 1), (33, 4, 3, 2),
+                                      (63, 4, 3, 1), (64, 3, 6, 1), (65, 4, 3, 1), (96, 3, 6, 1), (97, 4, 3, 1),
+                                      (128, 3, 6, 1)])
+def test_step_radial_sizes(opf, N, K, M, Mp, gp, monkeypatch):
+    if gp == 4 and N > 96:
+        pytest.skip("four pairs per workgroup need N <= 96")
+    _one_step_matches(opf, N, K, M, Mp, gp, monkeypatch, 1e-12 if N <= 64 else 1e-11)
+
+
+def test_step_with_a_replaced_factor_set(opf):
+    """tim_lumesh_init into LDz (other c1, c2, the Neumann wall row): the next
+    steps solve with it, and tim_lumesh_get returns its LAPACK factors; then
+    vel_matrices rebuilds the set."""
+    from opf import ic as icgen
+    N, K, M, Re, alpha, dt = 20, 4, 3, 2400.0, 1.25, 0.01
+    ctx = opf.Context(N, K, M)
+    ctx.setup(0, Re, alpha, dt)
+    before = ctx.lumesh_get(0, opf.LDZ)
+    me = ctx.mesh()
+    u = icgen.seeded_perturbation(me["r"], me["intrdr"], K, M, alpha, 3, 1e-2)
+    ctx.lumesh_init(0, opf.LDZ, 0, 1, 130.0, -3e-4)
+    ctx.put_state(0, *u)
+    ctx.run(1, corr_fixed=1)
+    got = ctx.get_state(0)
+    oc = O.Ctx(N, K, M, Re=Re, alpha=alpha, dt=dt)
+    oc.LDz = oc.lumesh_init(0, 1, 130.0, -3e-4)
+    AB = oc.LDz[0][1:]
+    assert np.abs(ctx.lumesh_get(0, opf.LDZ)[0][1:] - AB).max() <= 1e-13 * np.abs(AB).max()
+    oc.set_state(*u)
+    oc.run(1, ncorr_fixed=1)
+    for c, ref in enumerate((oc.ur, oc.ut, oc.uz)):
+        # harmonic 0 has a singular system under BC = 1, which the time step never meets
+        assert rel_err(got[c][:, 1:], ref[:, 1:]) <= 1e-12, c
+    ctx.vel_matrices(0, dt)
+    after = ctx.lumesh_get(0, opf.LDZ)
+    assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
