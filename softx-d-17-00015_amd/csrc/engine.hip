@@ -148,7 +148,10 @@ struct opf_ctx {
     void* p = nullptr;
     const size_t b = round_up(std::max<size_t>(n, 1) * sizeof(T), 256);
     HIPCHK(hipMalloc(&p, b));
+    // the context's streams are non-blocking: they do not wait for this fill,
+    // which runs on the null stream and may outlast the call
     HIPCHK(hipMemset(p, 0, b));
+    HIPCHK(hipStreamSynchronize(nullptr));
     allocs.push_back(p);
     bytes += b;
     return (T*)p;
