@@ -356,7 +356,7 @@ int opf_server_pool(opf_server* srv, size_t* used, size_t* limit, int* blocks);
 /* ---- timing hooks --------------------------------------------------------- */
 
 /* Record HIP events around every launch of the named kernel on the
- * context's stream ("step", "zfwd", "theta", "zbwd", "curl", "control");
+ * context's stream ("step", "zfwd", "theta", "zbwd", "plane", "curl");
  * 0 disables.  opf_kernel_time returns the summed milliseconds and the
  * launch count since the last reset. */
 int opf_kernel_timing(opf_ctx* ctx, int enable);

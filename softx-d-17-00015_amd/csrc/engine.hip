@@ -182,13 +182,13 @@ size_t bytes_needed(int N, int K, int M, int cap, int diag_cap) {
   const Shape s = shape_of(N, K, M);
   size_t b = 0;
   const size_t c3 = (size_t)cap * 3 * s.coll * sizeof(double2);
-  b += c3 * 7;                                               // U[3], Nraw[2], om, R
-  b += (size_t)cap * s.coll * sizeof(double2);               // S
+  b += c3 * 6;                                               // U[3], Nraw[2], om
   b += (size_t)cap * 4 * s.P * blk_count(N) * 16 * sizeof(double);   // SE
   b += (size_t)cap * 6 * N * s.P * sizeof(double);           // Uinf
   b += (size_t)cap * 16 * s.H * sizeof(double);              // Ainv
   b += (size_t)cap * 3 * s.Hp * sizeof(double);              // diagb
   b += (size_t)cap * 3 * N * sizeof(unsigned long long);     // cflmax
+  b += (size_t)cap * arrive_words(s.P) * sizeof(unsigned long long);
   b += (size_t)cap * diag_cap * sizeof(DiagRec);
   b += (size_t)cap * N * s.Z * 9 * M * sizeof(double2);      // Yf + Yb
   return b;
@@ -342,7 +342,6 @@ void launch_step(opf_ctx* c, int s0, int ns) {
   const int per = (c->st.ngroups + 7) / 8;   // XCD-aware order inside the kernel
   launch(c, "step", step_kernel(c->N, c->st.gp), dim3(8 * per, 1, ns), dim3(step_threads(c->st.gp)), c->st.smem, c->G, c->B,
          c->st, s0);
-  launch(c, "control", k_control, dim3(1, 1, ns), dim3(256), 0, c->G, c->B, s0);
 }
 
 // vel_matrices for slots s0 .. s0+ns-1 (gated: only slots whose control
@@ -657,8 +656,6 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   for (int i = 0; i < 3; ++i) B.U[i] = c->alloc<double2>(c3);
   for (int i = 0; i < 2; ++i) B.Nraw[i] = c->alloc<double2>(c3);
   B.om = c->alloc<double2>(c3);
-  B.R = c->alloc<double2>(c3);
-  B.S = c->alloc<double2>((size_t)cap * s.coll);
   B.SE = c->alloc<double>((size_t)cap * 4 * s.P * blk_count(N) * 16);
   B.spec = c->alloc<LuSpec>((size_t)cap * 4);
   B.Uinf = c->alloc<double>((size_t)cap * 6 * N * s.P);
@@ -666,6 +663,7 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   B.Ui = c->alloc<double>((size_t)cap * N);
   B.diagb = c->alloc<double>((size_t)cap * 3 * s.Hp);
   B.cflmax = c->alloc<unsigned long long>((size_t)cap * 3 * N);
+  B.arrive = c->alloc<unsigned long long>((size_t)cap * arrive_words(s.P));
   B.diag = c->alloc<DiagRec>((size_t)cap * c->diag_cap);
   B.prm = c->alloc<SlotParams>(cap);
   B.ctl = c->alloc<SlotCtl>(cap);
@@ -768,7 +766,6 @@ void put_state(opf_ctx* c, int slot, const double* const* f, double t) {
   k.status = 0;
   k.ndiag = 0;
   k.active = 1;
-  k.dterr_bits = 0;
   k.corr_dt = 0.0;   // tim_corr_dt, tim_cfl_dt and tim_new_tstep's counter of a fresh run
   k.cfl_dt = 0.0;
   k.cfl_dir = 0;

@@ -20,8 +20,6 @@ struct Bufs {
   double2* U[3];        // velocity buffers [slot][3][N][Hp]; roles per slot in SlotCtl
   double2* Nraw[2];     // nonlinear terms without base-flow terms [slot][3][N][Hp]
   double2* om;          // curl of the current iterate [slot][3][N][Hp]
-  double2* R;           // step scratch: right-hand sides [slot][3][N][Hp]
-  double2* S;           // step scratch: pressure [slot][N][Hp]
   double* LU;           // LAPACK-form factors [slot][4 mats][P pairs][N columns][LUS] (first use of tim_lumesh_*)
   unsigned char* PV;    // their pivot offsets ipiv(j)-j [slot][4][P][N]
   double* SE;           // block inverses (k_block_factor, solve.hpp) [slot][4 mats][P pairs][blk_count(N)][16],
@@ -33,6 +31,8 @@ struct Bufs {
   double* diagb;        // per-harmonic energy partials [slot][3][Hp]
   unsigned long long* cflmax;  // [slot][3][N] per-plane max of |u_r|, |u_t|, |u_z + 1 - r^2| on the
                                // physical grid of the last evaluation (bit patterns, vel_maxtstep)
+  unsigned long long* arrive;  // [slot][arrive_words(P)] arrivals of the step kernel's workgroups (0 between
+                        // launches), one word per 128 bytes, then each workgroup's max |du|^2 (bit pattern)
   DiagRec* diag;        // diagnostics records [slot][diag_cap]
   SlotParams* prm;      // [slot]
   SlotCtl* ctl;         // [slot]
@@ -89,6 +89,8 @@ struct StepTiles {
   int ngroups;   // workgroups per slot
   size_t smem;   // dynamic LDS bytes
 };
+constexpr int ARRIVE_WORDS = 16;
+__host__ __device__ constexpr size_t arrive_words(int P) { return 16 * ARRIVE_WORDS + (size_t)P; }
 inline int step_threads(int gp) { return gp == 1 ? 128 : 256; }
 // LDS of a step workgroup in doubles: V[3][N + 8][2 gp] (complex, four rows of
 // zeros at either end), the mesh tables (MeshOff::lapT, d1T, rowv; with four
@@ -158,7 +160,6 @@ __global__ void k_norm_sum(Geo G, const double* b, double* out);
 // the fused step kernel for N radial points and gp pairs per workgroup
 using StepKern = void (*)(Geo, Bufs, StepTiles, int);
 StepKern step_kernel(int N, int gp);
-__global__ void k_control(Geo G, Bufs B, int slot0);
 
 // transforms: kernels specialised to the radix plans of (Z, T), chosen once
 // per context by fft_kernels (generic kernels for other lengths)

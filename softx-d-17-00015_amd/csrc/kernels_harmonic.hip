@@ -92,6 +92,96 @@ __device__ __forceinline__ double pr0_of(const double2* uz0, size_t hs, int N, c
   return s / (-2.0);
 }
 
+// ---------------------------------------------------------------------------
+// tim_check_cgce (timestep.f90:214-253), buffer roles, time and step counters
+// of one slot: one thread, on the slot's control block, after every
+// workgroup's part of the step.  Pr0 and Pr0_hpf are another workgroup's to
+// write.  dt2: max |du|^2 of a corrector; E, Ek0, Em0: var_coll_norm of a
+// diagnostics step.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void control_decide(SlotCtl* c, const SlotParams& prm, DiagRec* recs, bool diag_now,
+                                               double dt2, double E, double Ek0, double Em0) {
+  SlotCtl k = *c;
+  c->arrived = 0u;
+  if (k.mode == MODE_PRED) {
+    if (diag_now) {
+      DiagRec* rec = recs + (k.ndiag % k.diag_cap);
+      rec->E = E;
+      rec->Ek0 = Ek0;
+      rec->Em0 = Em0;
+      rec->ncorr = -1.0;
+      rec->dterr = 0.0;
+      c->ndiag = k.ndiag + 1;
+    }
+    // vel_predictor done: u_ := old current, N_ := this evaluation's raw N
+    c->ubase = k.ucur;
+    c->ucur = k.unext;
+    c->unext = k.ubase;
+    c->npred = k.ncur;
+    c->ncur = 1 - k.ncur;
+    c->it = 1;
+    c->ncorr = 0;
+    c->lasterr = 1e99;
+    c->mode = MODE_CORR;
+    return;
+  }
+  // corrector done
+  const double dterr = sqrt(dt2);
+  const int ncorr = k.ncorr + 1;
+  c->ncorr = ncorr;
+  c->ucur = k.unext;
+  c->unext = k.ucur;
+  c->last_dterr = dterr;
+  if (k.host_driven) return;   // the caller applies tim_check_cgce itself
+  int it = k.it;
+  if (it == 1) {
+    c->corr_dt = prm.dt * sqrt(prm.dterr_tol / dterr);
+    c->lasterr = k.lasterr = 1e99;
+  }
+  int fail = OPF_FAIL_NONE;
+  if (!(dterr == dterr)) {
+    fail = OPF_FAIL_NAN;
+    it = 0;
+  } else if (prm.dt < 1e-9 && k.step > 30) {
+    fail = OPF_FAIL_DT0;
+    it = 0;
+  } else if (it > 10) {
+    fail = OPF_FAIL_ITS;
+    it = 0;
+  } else if (dterr > k.lasterr) {
+    if (dterr > 2.0 * prm.dterr_tol) fail = OPF_FAIL_INCERR;
+    else c->corr_dt = prm.dt / (10.0 * prm.courant);
+    it = 0;
+  } else if (dterr > prm.dterr_tol) {
+    c->lasterr = dterr;
+    it = it + 1;
+  } else {
+    it = 0;
+  }
+  if (k.corr_fixed > 0) it = ncorr >= k.corr_fixed ? 0 : (it == 0 ? 1 : it);
+  if (fail != OPF_FAIL_NONE && k.corr_fixed <= 0) {
+    c->status = fail;
+    c->active = 0;
+    return;
+  }
+  c->it = it;
+  if (it == 0) {
+    // step complete: tim_t += dt, tim_step += 1 (main.f90:43-44)
+    if (k.diag_every > 0 && k.ndiag > 0) {
+      DiagRec* rec = recs + ((k.ndiag - 1) % k.diag_cap);
+      if ((int)rec->step == k.step) {
+        rec->ncorr = ncorr;
+        rec->dterr = dterr;
+      }
+    }
+    c->last_ncorr = ncorr;
+    c->t = k.t + prm.dt;
+    c->step = k.step + 1;
+    c->mode = MODE_PRED;
+    if (k.target_steps >= 0 && k.step + 1 >= k.target_steps) c->active = 0;
+  }
+}
+
 // IT: (radial point, harmonic) items per thread in the parallel stages,
 // N * 2 * GP <= IT * THR; THR: threads of the workgroup; SM >= blk_mid(N).
 template <int GP, int IT, int THR, int SM>
@@ -346,6 +436,7 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
         for (int n = 0; n < N; ++n) bsum = bsum + EN[c * NI + n * GH + l] * me[mo.intrdr + n];
         if (Sd.h00) bsum = 0.5 * bsum;
         B.diagb[(size_t)slot * 3 * G.Hp + (size_t)(cc + c) * G.Hp + Sd.h] = bsum;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");   // for the workgroup that sums them
       }
       __syncthreads();
     }
@@ -547,21 +638,50 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
     }
   }
   double dmax = 0.0;
+  if (corr) {
+#pragma unroll
+    for (int q = 0; q < IT; ++q) {
+      if (n0 + q * DN >= N || !S.valid) continue;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double dx = old[q][c].x - nu[q][c].x, dy = old[q][c].y - nu[q][c].y;
+        dmax = fmax(dmax, fma(dx, dx, dy * dy));
+      }
+    }
+    for (int off = 32; off >= 1; off >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, off));
+    if ((tid & 63) == 0) RED[1 + wave] = dmax;
+  }
+  __syncthreads();
+
+  // This workgroup's maximum, and its arrival: the last one to arrive takes
+  // the control step (control_decide).  An arrival follows the return of its
+  // workgroup's exchange, and both round trips run behind the stores and the
+  // curl.  Arrivals at one word cost about 3 ns each, so many workgroups
+  // arrive at ARRIVE_WORDS words first, and the last at each of those at the
+  // slot's.  A kernel of its own for the control step took 4.6 us per
+  // evaluation; this takes about CTLCOST.
+  unsigned long long* arr = B.arrive + (size_t)slot * arrive_words(P);
+  const int nsub = ST.ngroups > 2 * ARRIVE_WORDS ? ARRIVE_WORDS : 1;
+  const int sub = grp % nsub;
+  unsigned long long prev = 0ull, cnt = 0ull;
+  if (tid == 0 && corr) {
+#pragma unroll
+    for (int w = 1; w < THR / 64; ++w) dmax = fmax(dmax, RED[1 + w]);
+    prev = __hip_atomic_exchange(arr + 16 * ARRIVE_WORDS + grp, (unsigned long long)__double_as_longlong(dmax),
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 #pragma unroll
   for (int q = 0; q < IT; ++q) {
     const int n = n0 + q * DN;
     if (n >= N || !S.valid) continue;
     const unsigned o = (unsigned)n * rb + ho;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      *(double2*)(un + (size_t)(c * cb) + o) = nu[q][c];
-      if (corr) {
-        const double dx = old[q][c].x - nu[q][c].x, dy = old[q][c].y - nu[q][c].y;
-        dmax = fmax(dmax, fma(dx, dx, dy * dy));
-      }
-    }
+    for (int c = 0; c < 3; ++c) *(double2*)(un + (size_t)(c * cb) + o) = nu[q][c];
   }
-  __syncthreads();
+  if (tid == 0) {
+    asm volatile("" ::"v"(prev) : "memory");
+    cnt = __hip_atomic_fetch_add(arr + 16 * sub, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 
   // ---- stage 7: curl of the new velocity for the next evaluation ---------
 #pragma unroll
@@ -588,17 +708,66 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
 #pragma unroll
     for (int c = 0; c < 3; ++c) *(double2*)(om + (size_t)(c * cb) + o) = cw[c];
   }
-  if (corr) {
-    // max is order independent and the bit pattern of a non-negative double
-    // orders like its value: an integer atomic max is exact.  One atomic per
-    // workgroup (all of them target the slot's one word).
-    for (int off = 32; off >= 1; off >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, off));
-    if ((tid & 63) == 0) RED[1 + (tid >> 6)] = dmax;
-    __syncthreads();
-    if (tid == 0) {
-      for (int w = 1; w < THR / 64; ++w) dmax = fmax(dmax, RED[1 + w]);
-      atomicMax(&ctl->dterr_bits, (unsigned long long)__double_as_longlong(dmax));
+  if (tid == 0) {
+    bool last = cnt == (unsigned long long)((ST.ngroups - sub + nsub - 1) / nsub - 1);
+    if (last) {
+      arr[16 * sub] = 0ull;
+      if (nsub > 1)
+        last = __hip_atomic_fetch_add(&ctl->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsub - 1u;
     }
+    RED[0] = last ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  if (RED[0] == 0.0) return;
+  DiagRec* recs = B.diag + (size_t)slot * ct.diag_cap;
+  double* ws = (double*)V;   // [wave][3]
+  if (corr) {
+    dmax = 0.0;
+    for (int i = tid; i < ST.ngroups; i += 4 * THR) {
+      unsigned long long w4[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)   // past the end: the last one again
+        w4[u] = __hip_atomic_load(arr + 16 * ARRIVE_WORDS + min(i + u * THR, ST.ngroups - 1), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) dmax = fmax(dmax, __longlong_as_double((long long)w4[u]));
+    }
+    for (int off = 32; off >= 1; off >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, off));
+    if ((tid & 63) == 0) ws[wave] = dmax;
+    __syncthreads();
+    for (int w = 1; w < THR / 64; ++w) dmax = fmax(dmax, ws[w]);
+  }
+  if (!want_diag) {
+    if (tid == 0) control_decide(ctl, prm, recs, false, dmax, 0.0, 0.0, 0.0);
+    return;
+  }
+  // var_coll_norm (variables.f90:727-749) from the harmonics' partials
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  constexpr int DTN = 128;   // summing threads: the same sums for every THR
+  double en[3] = {0.0, 0.0, 0.0};   // E, E of k = 0, E of m = 0
+  for (int c = 0; c < 3 && tid < DTN; ++c) {
+    const double* db = B.diagb + ((size_t)slot * 3 + c) * G.Hp;
+    for (int h0 = tid; h0 < G.H; h0 += 8 * DTN) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = h0 + u * DTN < G.H ? db[h0 + u * DTN] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int h = h0 + u * DTN;
+        en[0] = en[0] + v[u];
+        if (h == 0 || (h >= K && (h - K) % (2 * K - 1) == K - 1)) en[1] = en[1] + v[u];
+        if (h < K) en[2] = en[2] + v[u];
+      }
+    }
+  }
+  for (int i = 0; i < 3; ++i) {
+    for (int off = 32; off >= 1; off >>= 1) en[i] = en[i] + __shfl_xor(en[i], off);
+    if ((tid & 63) == 0) ws[wave * 3 + i] = en[i];
+  }
+  __syncthreads();
+  if (tid == 0) {
+    for (int i = 0; i < 3; ++i) en[i] = en[i] + ws[3 + i];
+    control_decide(ctl, prm, recs, true, 0.0, en[0], en[1], en[2]);
   }
 }
 

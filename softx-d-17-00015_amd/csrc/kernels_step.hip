@@ -1233,7 +1233,6 @@ __global__ void k_admit(Bufs B, int slot, int phase, int nsteps, int corr_fixed)
     k.it = 0;
     k.ncorr = 0;
     k.ndiag = 0;
-    k.dterr_bits = 0;
     k.corr_dt = 0.0;
     k.cfl_dt = 0.0;
     k.cfl_dir = 0;
@@ -1259,170 +1258,6 @@ __global__ void k_imposesym(Geo G, Bufs B, int slot0) {
   u[o] = make_double2(0.0, 0.0);
   u[G.coll + o].y = 0.0;
   u[2 * G.coll + o].y = 0.0;
-}
-
-// ---------------------------------------------------------------------------
-// Control: tim_check_cgce (timestep.f90:214-253) per slot, buffer roles,
-// time and step counters, and the reduction of the diagnostics partials in
-// var_coll_norm's blocks (variables.f90:727-749).
-// One workgroup per slot.
-// ---------------------------------------------------------------------------
-// The decisions of the control step on a register copy of the slot's
-// control block (recs: the slot's diagnostics records).
-__device__ __forceinline__ void control_decide(SlotCtl& k, const SlotParams& prm, DiagRec* recs, bool diag_now,
-                                               double E, double Ek0, double Em0) {
-  if (diag_now) {
-    DiagRec* rec = recs + (k.ndiag % k.diag_cap);
-    rec->E = E;
-    rec->Ek0 = Ek0;
-    rec->Em0 = Em0;
-    rec->ncorr = -1.0;
-    rec->dterr = 0.0;
-  }
-  if (k.mode == MODE_PRED) {
-    // vel_predictor done: u_ := old current, N_ := this evaluation's raw N
-    const int old_base = k.ubase;
-    k.ubase = k.ucur;
-    k.ucur = k.unext;
-    k.unext = old_base;
-    k.npred = k.ncur;
-    k.ncur = 1 - k.ncur;
-    k.it = 1;
-    k.ncorr = 0;
-    k.lasterr = 1e99;
-    k.mode = MODE_CORR;
-    if (diag_now) k.ndiag = k.ndiag + 1;
-    return;
-  }
-  // corrector done
-  const double dterr = sqrt(__longlong_as_double((long long)k.dterr_bits));
-  k.dterr_bits = 0ull;
-  k.ncorr = k.ncorr + 1;
-  const int old_cur = k.ucur;
-  k.ucur = k.unext;
-  k.unext = old_cur;
-  k.last_dterr = dterr;
-  if (k.host_driven) return;   // the caller applies tim_check_cgce itself
-  int it = k.it;
-  if (it == 1) {
-    k.corr_dt = prm.dt * sqrt(prm.dterr_tol / dterr);
-    k.lasterr = 1e99;
-  }
-  int fail = OPF_FAIL_NONE;
-  if (!(dterr == dterr)) {
-    fail = OPF_FAIL_NAN;
-    it = 0;
-  } else if (prm.dt < 1e-9 && k.step > 30) {
-    fail = OPF_FAIL_DT0;
-    it = 0;
-  } else if (it > 10) {
-    fail = OPF_FAIL_ITS;
-    it = 0;
-  } else if (dterr > k.lasterr) {
-    if (dterr > 2.0 * prm.dterr_tol) fail = OPF_FAIL_INCERR;
-    else k.corr_dt = prm.dt / (10.0 * prm.courant);
-    it = 0;
-  } else if (dterr > prm.dterr_tol) {
-    k.lasterr = dterr;
-    it = it + 1;
-  } else {
-    it = 0;
-  }
-  if (k.corr_fixed > 0) it = k.ncorr >= k.corr_fixed ? 0 : (it == 0 ? 1 : it);
-  if (fail != OPF_FAIL_NONE && k.corr_fixed <= 0) {
-    k.status = fail;
-    k.active = 0;
-    return;
-  }
-  k.it = it;
-  if (it == 0) {
-    // step complete: tim_t += dt, tim_step += 1 (main.f90:43-44)
-    if (k.diag_every > 0 && k.ndiag > 0) {
-      DiagRec* rec = recs + ((k.ndiag - 1) % k.diag_cap);
-      if ((int)rec->step == k.step) {
-        rec->ncorr = k.ncorr;
-        rec->dterr = dterr;
-      }
-    }
-    k.last_ncorr = k.ncorr;
-    k.t = k.t + prm.dt;
-    k.step = k.step + 1;
-    k.mode = MODE_PRED;
-    if (k.target_steps >= 0 && k.step >= k.target_steps) k.active = 0;
-  }
-}
-
-__global__ void k_control(Geo G, Bufs B, int slot0) {
-  const int slot = slot_of(B, slot0);
-  const SlotCtl k0 = B.ctl[slot];   // one batch of loads
-  if (!k0.active) return;
-  const SlotParams prm = B.prm[slot];
-  __shared__ double Em[3][256];
-  __shared__ double Ekm[3][256];   // the k = 0 term of each m block (the Ek(0) sum)
-  __shared__ double chunk[4096];
-  const bool diag_now = k0.mode == MODE_PRED && k0.diag_every > 0 && (k0.step % k0.diag_every) == 0;
-  if (diag_now) {
-    // Em(m) accumulates the block of m.  Whole m blocks are staged through
-    // LDS by all threads (coalesced), then one wave per block sums it as a
-    // tree (the reference sums in harmonic order; the two differ by
-    // rounding, about 1e-16 relative).
-    const int K = G.K, M = G.M, bl = 2 * K - 1;
-    auto hstart = [&](int m) { return m == 0 ? 0 : K + (m - 1) * bl; };
-    auto hend = [&](int m) { return m == 0 ? K : K + m * bl; };
-    for (int comp = 0; comp < 3; ++comp) {
-      const double* db = B.diagb + ((size_t)slot * 3 + comp) * G.Hp;
-      for (int m0 = 0; m0 < M;) {
-        int m1 = m0 + 1;
-        while (m1 < M && hend(m1) - hstart(m0) <= 4096) ++m1;
-        const int h0 = hstart(m0), nh = hend(m1 - 1) - h0;
-        // all of a thread's loads of the chunk in one batch (one round trip)
-        for (int b0 = 0; b0 < nh; b0 += 16 * (int)blockDim.x) {
-          double v[16];
-#pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            const int i = b0 + u * (int)blockDim.x + (int)threadIdx.x;
-            v[u] = i < nh ? db[h0 + i] : 0.0;
-          }
-#pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            const int i = b0 + u * (int)blockDim.x + (int)threadIdx.x;
-            if (i < nh) chunk[i] = v[u];
-          }
-        }
-        __syncthreads();
-        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
-        for (int m = m0 + wave; m < m1; m += nw) {
-          const int a = hstart(m) - h0, n = hend(m) - hstart(m);
-          double sm = 0.0;
-          for (int i = lane; i < n; i += 64) sm = sm + chunk[a + i];
-          for (int off = 32; off >= 1; off >>= 1) sm = sm + __shfl_xor(sm, off);
-          if (lane == 0 && m < 256) {
-            Em[comp][m] = sm;
-            Ekm[comp][m] = chunk[(m == 0 ? 0 : hstart(m) + (K - 1)) - h0];
-          }
-        }
-        __syncthreads();
-        m0 = m1;
-      }
-    }
-  }
-  if (threadIdx.x != 0) return;
-  double E = 0.0, Ek0 = 0.0, Em0 = 0.0;
-  if (diag_now) {
-    for (int comp = 0; comp < 3; ++comp) {
-      double e = 0.0, ek = 0.0;   // Ek(0): harmonics with k = 0 in order, m = 0..M-1
-      for (int m = 0; m < G.M; ++m) {
-        e = e + Em[comp][m];
-        ek = ek + Ekm[comp][m];
-      }
-      E = E + e;
-      Ek0 = Ek0 + ek;
-      Em0 = Em0 + Em[comp][0];
-    }
-  }
-  SlotCtl k = k0;
-  control_decide(k, prm, B.diag + (size_t)slot * k.diag_cap, diag_now, E, Ek0, Em0);
-  B.ctl[slot] = k;   // one batch of stores
 }
 
 // ---------------------------------------------------------------------------

@@ -54,8 +54,8 @@ struct SlotParams {
 // Slot modes for the next step kernel.
 enum { MODE_PRED = 0, MODE_CORR = 1 };
 
-// Per-slot control block (device resident).  The step and control kernels
-// advance it; the host reads it back to follow progress.
+// Per-slot control block (device resident).  The step kernel advances it; the
+// host reads it back to follow progress.
 struct SlotCtl {
   int active;          // slot integrates
   int mode;            // MODE_PRED / MODE_CORR for the next step kernel
@@ -78,8 +78,8 @@ struct SlotCtl {
   int cfl_dir;         // tim_cfl_dir
   double cfl_dt;       // tim_cfl_dt
   double t, dterr, lasterr, corr_dt, Pr0, Pr0_hpf, last_dterr;
-  unsigned long long dterr_bits;  // max |du|^2 of the running corrector (bit pattern)
   double flux_d1;      // vel_adjustFlux(0) d1
+  unsigned arrived;    // arrivals of the running step kernel (0 between launches)
 };
 
 // One diagnostics record, the content of io_write_energy / io_write_friction.
