@@ -86,7 +86,7 @@ struct opf_ctx {
   Geo G{};
   FftTiles tiles{};
   StepTiles st{};
-  size_t smem_z = 0, smem_t = 0;
+
   FftKerns fk{};
   PlaneKern plane = nullptr;   // whole-plane evaluation, where the grid has one
   size_t smem_plane = 0;
@@ -190,7 +190,7 @@ size_t bytes_needed(int N, int K, int M, int cap, int diag_cap) {
   b += (size_t)cap * 3 * N * sizeof(unsigned long long);     // cflmax
   b += (size_t)cap * arrive_words(s.P) * sizeof(unsigned long long);
   b += (size_t)cap * diag_cap * sizeof(DiagRec);
-  b += (size_t)cap * N * s.Z * 9 * M * sizeof(double2);      // Yf + Yb
+  b += (size_t)cap * N * ((s.Z + 3) / 4 * 4) * 9 * M * sizeof(double2);   // Yf + Yb
   return b;
 }
 
@@ -318,24 +318,30 @@ dim3 grid_hn(opf_ctx* c, int nslots) {
 // blocks of k_zfwd_t / k_zbwd_t: their (m tile, n, field) tiles, 6 or 3
 // fields, rounded up to 8 XCDs
 unsigned ztile_blocks(const opf_ctx* c, int nfield) {
-  const int gx = (c->M + c->tiles.tm - 1) / c->tiles.tm;
+  const int gx = (c->M + c->fk.t.tm - 1) / c->fk.t.tm;
   return (unsigned)(8 * ((gx * nfield * c->N + 7) / 8));
+}
+
+// vel_transform's z transforms; the theta transforms, products and the way back
+void launch_zfwd(opf_ctx* c, int s0, int ns) {
+  launch(c, "zfwd", c->fk.zfwd, dim3(ztile_blocks(c, 6), 1, ns), dim3(c->fk.zn), c->fk.zfs, c->G, c->B, c->fk.t, s0);
+}
+void launch_back(opf_ctx* c, int s0, int ns) {
+  const int gz = (c->Z + c->fk.t.tz - 1) / c->fk.t.tz;
+  launch(c, "theta", c->fk.theta, dim3(8 * ((gz * c->N + 7) / 8), 1, ns), dim3(c->fk.tn), c->fk.ts, c->G,
+         c->B, c->fk.t, s0);
+  launch(c, "zbwd", c->fk.zbwd, dim3(ztile_blocks(c, 3), 1, ns), dim3(c->fk.zn), c->fk.zbs, c->G, c->B, c->fk.t, s0);
 }
 
 // One evaluation (vel_transform + vel_nonlinear without the base-flow
 // terms) for slots [s0, s0+ns).
 void launch_eval(opf_ctx* c, int s0, int ns) {
-  const FftTiles& t = c->tiles;
   if (c->plane) {   // one workgroup per radial plane, the intermediates in LDS
-    launch(c, "plane", c->plane, dim3(c->N, 1, ns), dim3(PLANE_THREADS), c->smem_plane, c->G, c->B, t, s0);
+    launch(c, "plane", c->plane, dim3(c->N, 1, ns), dim3(PLANE_THREADS), c->smem_plane, c->G, c->B, c->fk.t, s0);
     return;
   }
-  launch(c, "zfwd", c->fk.zfwd, dim3(ztile_blocks(c, 6), 1, ns), dim3(FFT_THREADS), c->smem_z, c->G, c->B, t,
-         s0);
-  launch(c, "theta", c->fk.theta, dim3((c->Z + t.tz - 1) / t.tz, c->N, ns), dim3(FFT_THREADS), c->smem_t,
-         c->G, c->B, t, s0);
-  launch(c, "zbwd", c->fk.zbwd, dim3(ztile_blocks(c, 3), 1, ns), dim3(FFT_THREADS), c->smem_z,
-         c->G, c->B, t, s0);
+  launch_zfwd(c, s0, ns);
+  launch_back(c, s0, ns);
 }
 
 void launch_step(opf_ctx* c, int s0, int ns) {
@@ -411,9 +417,10 @@ void dev_to_coll(opf_ctx* c, const double2* src, double* re, double* im) {
     }
 }
 
+size_t y_one(const opf_ctx* c) { return (size_t)c->N * c->G.ZQ * c->M; }   // z-transformed planes of one field
 void ensure_temps(opf_ctx* c) {
   if (c->tY) return;
-  c->tY = c->alloc<double2>((size_t)c->N * c->Z * c->M);
+  c->tY = c->alloc<double2>(y_one(c));
   c->tP = c->alloc<double>((size_t)c->N * c->Z * c->T);
   c->tC = c->alloc<double2>(c->G.coll);
 }
@@ -422,26 +429,26 @@ void ensure_temps(opf_ctx* c) {
 // (stride N*Z*T) on device buffers for the plugins (tra_spec2phys /
 // tra_phys2spec, transform.fftw3.f90:65-147), one launch per stage with the
 // field as grid z; physical fields in the plugins' layout [n][z][theta].
-int lines_per_block(const opf_ctx* c) { return std::max(1, FFT_TILE / padded_len(c->T)); }
+// one coll field to / from the planes Y of its z transform (nf fields)
+void launch_zfwd_one(opf_ctx* c, const double2* src, double2* Y, int nf) {
+  launch(c, "zfwd1", c->fk.zfwd1, dim3(ztile_blocks(c, 1), 1, nf), dim3(c->fk.zn), c->fk.zfs, c->G, c->B, c->fk.t, src,
+         Y, (size_t)c->G.coll, y_one(c));
+}
+void launch_zbwd_one(opf_ctx* c, const double2* Y, double2* dst, int nf) {
+  launch(c, "zbwd1", c->fk.zbwd1, dim3(ztile_blocks(c, 1), 1, nf), dim3(c->fk.zn), c->fk.zbs, c->G, c->B, c->fk.t, Y,
+         dst, y_one(c), (size_t)c->G.coll);
+}
+dim3 grid_lines(const opf_ctx* c, int nf) { return dim3((c->Z + 2 * c->fk.bt - 1) / (2 * c->fk.bt), c->N, nf); }
 void coll2phys_dev(opf_ctx* c, const double2* src, double* dst, int nf) {
-  const FftTiles& t = c->tiles;
-  const int BT = lines_per_block(c);
-  const size_t fy = (size_t)c->N * c->Z * c->M, fp = (size_t)c->N * c->Z * c->T;
-  launch(c, "zfwd1", k_zfwd_one, dim3((c->M + t.tm - 1) / t.tm, c->N, nf), dim3(FFT_THREADS), c->smem_z, c->G,
-         c->B, t, src, c->nnY, (size_t)c->G.coll, fy);
-  launch(c, "c2r_lines", k_c2r_lines, dim3((c->Z + 2 * BT - 1) / (2 * BT), c->N, nf), dim3(FFT_THREADS),
-         ((size_t)BT * padded_len(c->T) + c->T) * sizeof(double2), c->G, c->B, t, BT, (const double2*)c->nnY, dst,
-         fy, fp);
+  launch_zfwd_one(c, src, c->nnY, nf);
+  launch(c, "c2r_lines", c->fk.c2r, grid_lines(c, nf), dim3(c->fk.ln), c->fk.c2rs, c->G, c->B, c->fk.t, c->fk.bt,
+         (const double2*)c->nnY, dst, y_one(c), (size_t)c->N * c->Z * c->T);
 }
 void phys2coll_dev(opf_ctx* c, const double* src, double2* dst, int nf) {
-  const FftTiles& t = c->tiles;
-  const int BT = lines_per_block(c);
-  const size_t fy = (size_t)c->N * c->Z * c->M, fp = (size_t)c->N * c->Z * c->T;
   HIPCHK(hipMemsetAsync(dst, 0, sizeof(double2) * c->G.coll * nf, c->stream));
-  launch(c, "r2c_lines", k_r2c_lines, dim3((c->Z + 2 * BT - 1) / (2 * BT), c->N, nf), dim3(FFT_THREADS),
-         ((size_t)BT * padded_len(c->T) + c->T) * sizeof(double2), c->G, c->B, t, BT, src, c->nnY, fp, fy);
-  launch(c, "zbwd1", k_zbwd_one, dim3((c->M + t.tm - 1) / t.tm, c->N, nf), dim3(FFT_THREADS), c->smem_z, c->G,
-         c->B, t, (const double2*)c->nnY, dst, fy, (size_t)c->G.coll);
+  launch(c, "r2c_lines", c->fk.r2c, grid_lines(c, nf), dim3(c->fk.ln), c->fk.r2cs, c->G, c->B, c->fk.t, c->fk.bt, src,
+         c->nnY, (size_t)c->N * c->Z * c->T, y_one(c));
+  launch_zbwd_one(c, c->nnY, dst, nf);
 }
 
 // The variable-viscosity plugins share their transforms: the gradient
@@ -453,7 +460,7 @@ NnPhys visc_fields(opf_ctx* c) {
   const size_t np = (size_t)c->N * c->Z * c->T;
   if (!c->nnP) c->nnP = c->alloc<double>(16 * np);
   if (!c->nnC) c->nnC = c->alloc<double2>(4 * c->G.coll);
-  if (!c->nnY) c->nnY = c->alloc<double2>(3 * (size_t)c->N * c->Z * c->M);
+  if (!c->nnY) c->nnY = c->alloc<double2>(3 * y_one(c));
   NnPhys P{};
   for (int i = 0; i < 9; ++i) P.S[i] = c->nnP + (size_t)i * np;
   P.nu = c->nnP + 9 * np;
@@ -576,7 +583,6 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   c->H = s.H; c->Hp = s.Hp; c->P = s.P; c->Z = s.Z; c->T = s.T;
   build_mesh(N, r, c->mesh);
   c->tiles = choose_tiles(c->Z, c->T, M);
-  c->fk = fft_kernels(c->tiles.pz, c->tiles.pt);
   const Tuned tuned = lookup_tuning(N, K, M, cap);
   c->use_graph = tuned.graph;
   c->use_streams = tuned.streams > 0 ? tuned.streams : 2;
@@ -612,14 +618,20 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
     // the whole-plane evaluation where the grid has one and its LDS fits
     // (OPF_PLANE=0: the three transform kernels instead)
     const char* e2 = std::getenv("OPF_PLANE");
-    c->plane = plane_kernel(c->tiles.pz, c->tiles.pt, &c->smem_plane);
+    c->plane = plane_kernel(c->Z, c->T, &c->smem_plane);
     if (c->plane && ((e2 && std::atoi(e2) == 0) || c->smem_plane > (size_t)lds)) c->plane = nullptr;
     if (c->plane && c->smem_plane > 64 * 1024)
       HIPCHK(hipFuncSetAttribute((const void*)c->plane, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)c->smem_plane));
   }
-  c->smem_z = ((size_t)c->tiles.tm * padded_len(c->Z) + c->Z) * sizeof(double2);       // data + twiddles
-  c->smem_t = ((size_t)3 * c->tiles.tz * padded_len(c->T) + c->T) * sizeof(double2);
+  c->fk = fft_kernels(c->tiles.pz, c->tiles.pt, c->tiles, M);
+  const std::pair<const void*, size_t> lds_of[] = {
+      {(const void*)c->fk.zfwd, c->fk.zfs},  {(const void*)c->fk.zfwd1, c->fk.zfs}, {(const void*)c->fk.zbwd, c->fk.zbs},
+      {(const void*)c->fk.zbwd1, c->fk.zbs}, {(const void*)c->fk.theta, c->fk.ts},  {(const void*)c->fk.c2r, c->fk.c2rs},
+      {(const void*)c->fk.r2c, c->fk.r2cs}};
+  for (const auto& k : lds_of)
+    if (k.second > 64 * 1024)
+      HIPCHK(hipFuncSetAttribute(k.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.second));
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   // device mesh block
   const MeshOff mo = MeshOff::make(N);
@@ -667,8 +679,8 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   B.diag = c->alloc<DiagRec>((size_t)cap * c->diag_cap);
   B.prm = c->alloc<SlotParams>(cap);
   B.ctl = c->alloc<SlotCtl>(cap);
-  B.Yf = c->alloc<double2>((size_t)cap * N * s.Z * 6 * M);
-  B.Yb = c->alloc<double2>((size_t)cap * N * s.Z * 3 * M);
+  B.Yf = c->alloc<double2>((size_t)cap * N * ((s.Z + 3) / 4 * 4) * 6 * M);
+  B.Yb = c->alloc<double2>((size_t)cap * N * ((s.Z + 3) / 4 * 4) * 3 * M);
   B.twZ = c->alloc<double2>(s.Z);
   B.twT = c->alloc<double2>(s.T);
   B.smap = nullptr;
@@ -678,7 +690,7 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   HIPCHK(hipMemcpy(B.twT, tt.data(), tt.size() * sizeof(double2), hipMemcpyHostToDevice));
 
   Geo& G = c->G;
-  G.N = N; G.K = K; G.M = M; G.Mp = Mp; G.H = s.H; G.Hp = s.Hp; G.P = s.P; G.Z = s.Z; G.T = s.T;
+  G.N = N; G.K = K; G.M = M; G.Mp = Mp; G.H = s.H; G.Hp = s.Hp; G.P = s.P; G.Z = s.Z; G.T = s.T; G.ZQ = (s.Z + 3) / 4 * 4;
   G.coll = s.coll;
   G.mesh = c->d_mesh;
 
@@ -1450,9 +1462,7 @@ int opf_vel_imposesym(opf_ctx* c, int slot) {
 int opf_vel_transform(opf_ctx* c, int slot) {
   return guard([&] {
     with_active(c, slot, -1, [&] {
-      const FftTiles& t = c->tiles;
-      launch(c, "zfwd", c->fk.zfwd, dim3(ztile_blocks(c, 6), 1, 1), dim3(FFT_THREADS), c->smem_z, c->G, c->B, t,
-             slot);
+      launch_zfwd(c, slot, 1);
     });
   });
 }
@@ -1460,11 +1470,7 @@ int opf_vel_transform(opf_ctx* c, int slot) {
 int opf_vel_nonlinear(opf_ctx* c, int slot) {
   return guard([&] {
     with_active(c, slot, -1, [&] {
-      const FftTiles& t = c->tiles;
-      launch(c, "theta", c->fk.theta, dim3((c->Z + t.tz - 1) / t.tz, c->N, 1), dim3(FFT_THREADS), c->smem_t, c->G,
-             c->B, t, slot);
-      launch(c, "zbwd", c->fk.zbwd, dim3(ztile_blocks(c, 3), 1, 1), dim3(FFT_THREADS), c->smem_z, c->G,
-             c->B, t, slot);
+      launch_back(c, slot, 1);
       if (c->nn[slot].on) launch_nonnewtonian(c, slot);   // var_null(2)
       if (c->les[slot].on) launch_les(c, slot);
     });
@@ -1707,8 +1713,7 @@ int opf_get_phys(opf_ctx* c, int slot, int which, double* phys) {
     const double2* src = which < 3 ? c->B.U[ctl[slot].ucur] + (size_t)slot * 3 * c->G.coll + (size_t)which * c->G.coll
                                    : c->B.om + (size_t)slot * 3 * c->G.coll + (size_t)(which - 3) * c->G.coll;
     const FftTiles& t = c->tiles;
-    launch(c, "zfwd1", k_zfwd_one, dim3((c->M + t.tm - 1) / t.tm, c->N, 1), dim3(FFT_THREADS), c->smem_z, c->G,
-           c->B, t, src, c->tY, (size_t)0, (size_t)0);
+    launch_zfwd_one(c, src, c->tY, 1);
     launch(c, "c2r", k_theta_c2r, dim3((c->Z + 1) / 2, c->N, 1), dim3(FFT_THREADS),
            (padded_len(c->T) + c->T) * sizeof(double2), c->G, c->B, t, (const double2*)c->tY, c->tP);
     HIPCHK(hipMemcpyAsync(phys, c->tP, sizeof(double) * c->N * c->Z * c->T, hipMemcpyDeviceToHost, c->stream));
@@ -1743,8 +1748,7 @@ int opf_tra_coll2phys(opf_ctx* c, const double* cre, const double* cim, double* 
     ensure_temps(c);
     coll_to_dev(c, cre, cim, c->tC);
     const FftTiles& t = c->tiles;
-    launch(c, "zfwd1", k_zfwd_one, dim3((c->M + t.tm - 1) / t.tm, c->N, 1), dim3(FFT_THREADS), c->smem_z, c->G,
-           c->B, t, (const double2*)c->tC, c->tY, (size_t)0, (size_t)0);
+    launch_zfwd_one(c, c->tC, c->tY, 1);
     launch(c, "c2r", k_theta_c2r, dim3((c->Z + 1) / 2, c->N, 1), dim3(FFT_THREADS), (padded_len(c->T) + c->T) * sizeof(double2), c->G,
            c->B, t, (const double2*)c->tY, c->tP);
     HIPCHK(hipMemcpyAsync(phys, c->tP, sizeof(double) * c->N * c->Z * c->T, hipMemcpyDeviceToHost, c->stream));
@@ -1761,8 +1765,7 @@ int opf_tra_phys2coll(opf_ctx* c, const double* phys, double* cre, double* cim) 
     HIPCHK(hipMemsetAsync(c->tC, 0, sizeof(double2) * c->G.coll, c->stream));
     launch(c, "r2c", k_theta_r2c, dim3((c->Z + 1) / 2, c->N, 1), dim3(FFT_THREADS), (padded_len(c->T) + c->T) * sizeof(double2), c->G,
            c->B, t, (const double*)c->tP, c->tY);
-    launch(c, "zbwd1", k_zbwd_one, dim3((c->M + t.tm - 1) / t.tm, c->N, 1), dim3(FFT_THREADS), c->smem_z, c->G,
-           c->B, t, (const double2*)c->tY, c->tC, (size_t)0, (size_t)0);
+    launch_zbwd_one(c, c->tY, c->tC, 1);
     dev_to_coll(c, c->tC, cre, cim);
   });
 }

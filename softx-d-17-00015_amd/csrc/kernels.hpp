@@ -36,8 +36,8 @@ struct Bufs {
   DiagRec* diag;        // diagnostics records [slot][diag_cap]
   SlotParams* prm;      // [slot]
   SlotCtl* ctl;         // [slot]
-  double2* Yf;          // forward intermediates [slot][N][Z][6][M]
-  double2* Yb;          // backward intermediates [slot][N][Z][3][M]
+  double2* Yf;          // forward intermediates [slot][N][ZQ/4][6][M][4] (z, field, m, z % 4)
+  double2* Yb;          // backward intermediates [slot][N][ZQ/4][3][M][4]
   double2* twZ;         // twiddles exp(2 pi i q / Z), q < Z
   double2* twT;         // twiddles exp(2 pi i q / T), q < T
   const int* smap;      // null: grid z counts slots from slot0; else the slots of a
@@ -149,10 +149,6 @@ __global__ void k_les_visc(NnPhys P, size_t np, int N, int ZT, int model, double
                            unsigned long long* numax_slot);
 __global__ void k_les_nur(Bufs B, int slot, const unsigned long long* numax);
 __global__ void k_les_force(NnPhys P, size_t np, Bufs B, int slot);
-__global__ void k_c2r_lines(Geo G, Bufs B, FftTiles T, int BT, const double2* Y, double* phys, size_t fy,
-                            size_t fp);
-__global__ void k_r2c_lines(Geo G, Bufs B, FftTiles T, int BT, const double* phys, double2* Y, size_t fp,
-                            size_t fy);
 __global__ void k_add_coll(Geo G, double2* dst, const double2* src);
 // var_coll_norm of a field in the coll layout: per-harmonic partials b[H], then [E, Ek, Em]
 __global__ void k_norm_harm(Geo G, const SlotParams* prm, const double* re, const double* im, double* b);
@@ -162,22 +158,31 @@ using StepKern = void (*)(Geo, Bufs, StepTiles, int);
 StepKern step_kernel(int N, int gp);
 
 // transforms: kernels specialised to the radix plans of (Z, T), chosen once
-// per context by fft_kernels (generic kernels for other lengths)
+// per context by fft_kernels (run-time plans for other lengths)
 using FftKern = void (*)(Geo, Bufs, FftTiles, int);
+using ZOneKern = void (*)(Geo, Bufs, FftTiles, const double2*, double2*, size_t, size_t);
+using C2rKern = void (*)(Geo, Bufs, FftTiles, int, const double2*, double*, size_t, size_t);
+using R2cKern = void (*)(Geo, Bufs, FftTiles, int, const double*, double2*, size_t, size_t);
 struct FftKerns {
   FftKern zfwd, theta, zbwd;
+  ZOneKern zfwd1, zbwd1;   // one coll field to / from its z-transformed plane, a batch of fields as grid z
+  C2rKern c2r;             // theta lines of such planes to / from phys[n][z][theta], two lines per transform
+  R2cKern r2c;
+  FftTiles t;       // the tiles asked for, at most those that the kernels hold
+  int zn, tn, ln;   // threads of the z, theta and line kernels
+  int bt;           // transforms per workgroup of the line kernels
+  size_t zfs, zbs, ts, c2rs, r2cs;   // dynamic LDS bytes (zfwd1, zbwd1: as zfwd, zbwd)
 };
-FftKerns fft_kernels(const FftPlan& pz, const FftPlan& pt);
+FftKerns fft_kernels(const FftPlan& pz, const FftPlan& pt, const FftTiles& t, int M);
 // whole-plane evaluation (z, theta, products, theta, z in one workgroup per
-// radial plane) for the plan pairs that have one; nullptr otherwise.
+// radial plane) for the grids that have one; nullptr otherwise.
 // smem: its dynamic LDS bytes.
 constexpr int PLANE_THREADS = 1024;
-using PlaneKern = void (*)(Geo, Bufs, FftTiles, int);
-PlaneKern plane_kernel(const FftPlan& pz, const FftPlan& pt, size_t* smem);
-// materialise physical fields / transform arbitrary coll fields (granular API)
-__global__ void k_zfwd_one(Geo G, Bufs B, FftTiles T, const double2* a, double2* Y, size_t fa, size_t fy);
+using PlaneKern = FftKern;
+PlaneKern plane_kernel(int Z, int T, size_t* smem);
+// phys of one coll field by theta lines with z fastest (granular API), from the
+// z transforms' output
 __global__ void k_theta_c2r(Geo G, Bufs B, FftTiles T, const double2* Y, double* phys);
 __global__ void k_theta_r2c(Geo G, Bufs B, FftTiles T, const double* phys, double2* Y);
-__global__ void k_zbwd_one(Geo G, Bufs B, FftTiles T, const double2* Y, double2* a, size_t fy, size_t fa);
 
 }  // namespace opf

@@ -102,6 +102,7 @@ struct Geo {
   int Hp;         // row stride of a spectral field (H rounded up to 64)
   int P;          // unique (|k|, m) pairs = K*M
   int Z, T;       // physical grid 3K x 3M
+  int ZQ;         // Z rounded up to 4
   size_t coll;    // doubles2 per component of one slot: N*Hp
   const double* mesh;   // device mesh block, see MeshOff
 };
