@@ -350,14 +350,10 @@ void launch_step(opf_ctx* c, int s0, int ns) {
          c->st, s0);
 }
 
-// vel_matrices for slots s0 .. s0+ns-1 (gated: only slots whose control
-// block asks for it, the tim_new_dt of this step)
-void launch_matrices(opf_ctx* c, int s0, int ns, int gated) {
-  launch(c, "factor", k_block_factor, dim3((c->P + 31) / 32, 4, ns), dim3(64), 0, c->G, c->B, s0, gated,
-         LuSpec{-1, 0, 0, 0.0, 0.0});
-  launch(c, "influence", influence_kernel(c->N), dim3((c->P + 7) / 8, 4, ns), dim3(64), influence_smem(c->N), c->G,
-         c->B, s0, gated);
-  launch(c, "ainv", k_ainv, grid_h(c, ns), dim3(64), 0, c->G, c->B, s0, gated);
+// vel_matrices for slots s0 .. s0+ns-1 (gate: k_matrices_t)
+void launch_matrices(opf_ctx* c, int s0, int ns, int gate) {
+  launch(c, "matrices", matrices_kernel(c->N), dim3((c->P + 7) / 8, 1, ns), dim3(256), matrices_smem(c->N), c->G, c->B,
+         s0, gate);
 }
 
 // One iteration.  With adaptive slots, the predictor's evaluation is
@@ -381,8 +377,7 @@ void launch_iteration(opf_ctx* c, int s0, int ns) {
       if (c->les[s].on) launch_les(c, s);
     }
   if (c->n_adaptive > 0) {
-    launch(c, "newdt", k_newdt, dim3(1, 1, ns), dim3(64), 0, c->G, c->B, s0, 0);
-    launch_matrices(c, s0, ns, 1);
+    launch_matrices(c, s0, ns, 2);
   }
   launch_step(c, s0, ns);
 }
@@ -509,7 +504,7 @@ void launch_nonnewtonian(opf_ctx* c, int slot) {
   visc_add(c, slot, P);
 }
 
-void launch_matrices(opf_ctx* c, int s0, int ns, int gated);
+void launch_matrices(opf_ctx* c, int s0, int ns, int gate);
 
 // util(2) of the LES plugin for one slot (LES.f90:100-320): get_nu with the
 // slot's eddy-viscosity model, update_nu_r before a predictor (vel_matrices
@@ -1351,7 +1346,7 @@ int opf_vel_maxtstep(opf_ctx* c, int slot, double* cfl_dt, int* cfl_dir) {
   return guard([&] {
     check_slot(c, slot);
     if (!c->occupied[slot]) throw OpfError(OPF_ERR_STATE, "slot holds no state");
-    launch(c, "newdt", k_newdt, dim3(1, 1, 1), dim3(64), 0, c->G, c->B, slot, 1);
+    launch(c, "maxtstep", k_maxtstep, dim3(1), dim3(64), 0, c->G, c->B, slot);
     HIPCHK(hipStreamSynchronize(c->stream));
     auto ctl = read_ctl(c);
     if (cfl_dt) *cfl_dt = ctl[slot].cfl_dt;
@@ -1833,7 +1828,7 @@ extern "C" int opf_tim_lumesh_init(opf_ctx* c, int slot, int which, int PM, int 
     auto ctl = read_ctl(c);
     ctl[slot].status = 0;
     write_ctl(c, ctl);
-    launch(c, "factor", k_block_factor, dim3((c->P + 31) / 32, 4, 1), dim3(64), 0, c->G, c->B, slot, 0,
+    launch(c, "factor", k_block_factor, dim3((c->P + 31) / 32), dim3(64), 0, c->G, c->B, slot,
            LuSpec{which, PM, BC, c1, c2});
     lapack_factors(c, slot, which);   // DGBTF2's own verdict on a singular matrix
     ctl = read_ctl(c);

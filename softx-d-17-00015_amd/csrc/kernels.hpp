@@ -6,10 +6,8 @@
 
 namespace opf {
 
-// The matrix a factorisation builds, c1 + c2 Lap (of u+-: PM = +-1) with the
-// wall row BC: mat < 0 the four of vel_matrices (LDp, LDm, LDz with c1 = 1/dt,
-// c2 = -implicit nu/Re; LNp with 0, 1, BC = 1); mat >= 0 only that one, with
-// the given PM, BC, c1, c2.
+// The matrix a factorisation builds for set `mat`: c1 + c2 Lap (of u+-: PM =
+// +-1) with the wall row BC.
 struct LuSpec {
   int mat, PM, BC;
   double c1, c2;
@@ -22,7 +20,7 @@ struct Bufs {
   double2* om;          // curl of the current iterate [slot][3][N][Hp]
   double* LU;           // LAPACK-form factors [slot][4 mats][P pairs][N columns][LUS] (first use of tim_lumesh_*)
   unsigned char* PV;    // their pivot offsets ipiv(j)-j [slot][4][P][N]
-  double* SE;           // block inverses (k_block_factor, solve.hpp) [slot][4 mats][P pairs][blk_count(N)][16],
+  double* SE;           // block inverses (block_factor, solve.hpp) [slot][4 mats][P pairs][blk_count(N)][16],
                         // element (row, column) at 4 column + row
   LuSpec* spec;         // [slot][4] the matrix each factor set holds
   double* Uinf;         // influence vectors [slot][6][N][P]
@@ -118,15 +116,14 @@ __host__ __device__ constexpr int tile_m(int Z) { return FFT_TILE / Z; }
 
 __host__ __device__ constexpr int padded_len(int L) { return (L + (L - 1) / 16 + 1) | 1; }
 
-__global__ void k_block_factor(Geo G, Bufs B, int slot0, int gated, LuSpec spec);
+__global__ void k_block_factor(Geo G, Bufs B, int slot, LuSpec A);
 __global__ void k_lu_factor(Geo G, Bufs B, int slot, int mat);
-using FactorKern = void (*)(Geo, Bufs, int, int);
-FactorKern influence_kernel(int N);
-inline size_t influence_smem(int N) { return (size_t)(32 * (N + 4) + 10 * (N + 8)) * sizeof(double); }
-__global__ void k_ainv(Geo G, Bufs B, int slot0, int gated);
+using MatricesKern = void (*)(Geo, Bufs, int, int);
+MatricesKern matrices_kernel(int N);
+inline size_t matrices_smem(int N) { return (size_t)(10 * (N + 8) + 40 * (N + 4) + 48 * (KL + 1)) * sizeof(double); }
 __global__ void k_curl(Geo G, Bufs B, int slot0, int gated);
 __global__ void k_symmetry(Geo G, Bufs B, int slot0, int gated);
-__global__ void k_newdt(Geo G, Bufs B, int slot0, int what);
+__global__ void k_maxtstep(Geo G, Bufs B, int slot);
 __global__ void k_imposesym(Geo G, Bufs B, int slot0);
 __global__ void k_admit(Bufs B, int slot, int phase, int nsteps, int corr_fixed);
 __global__ void k_shift(Geo G, Bufs B, int slot0, const double2* __restrict__ tab);

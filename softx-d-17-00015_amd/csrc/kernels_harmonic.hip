@@ -388,7 +388,7 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   const int ps = p0 + min(wave, np - 1);   // a missing pair of the last group repeats a factor on zeros
   const int lhs = wave + GP * (bl.col >> 1);
   BlkE<SM, 1> EP;
-  if (solver) blk_load(EP, 0, G, B, slot, MAT_LNP, ps, bl);
+  if (solver) blk_load(EP, 0, G, B, slot, B.spec[slot * 4 + MAT_LNP], MAT_LNP, ps, bl);
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < IT; ++q) {
@@ -478,8 +478,8 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   }
   BlkE<SM, 2> EH;
   if (solver) {
-    blk_load(EH, 0, G, B, slot, MAT_LDP + bl.mi, ps, bl);
-    blk_load(EH, 1, G, B, slot, MAT_LDZ, ps, bl);
+    blk_load(EH, 0, G, B, slot, B.spec[slot * 4 + MAT_LDP + bl.mi], MAT_LDP + bl.mi, ps, bl);
+    blk_load(EH, 1, G, B, slot, B.spec[slot * 4 + MAT_LDZ], MAT_LDZ, ps, bl);
   }
   __syncthreads();
 

@@ -247,31 +247,20 @@ __device__ __forceinline__ double diag_d(double r2inv, int Mp, int m, double alp
 // boundary rows, whose scale differs from the interior's, sit in the outermost
 // blocks; against 80-bit arithmetic the solves are as accurate as with the
 // banded LU and partial pivoting, error ratio 0.3 to 1.1 over N = 9 .. 128).
-// A lane's chain is N / 8 blocks of a few hundred instructions, which bounds it:
-// 34 us at (64,64,48) and 167 us at (96,256,128), where factoring all N columns
-// row by row and writing 265 bytes per row took 134 and 1254 us.
-// grid: x = pairs / 32, y = 4 matrices, z = slot; 64 threads.
+// A lane's chain is N / 8 blocks of a few hundred instructions, which bounds it.
+// T: MeshOff::lapT in LDS.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot0, int gated, LuSpec spec) {
-  const int mat = blockIdx.y;
-  const int slot = slot_of(B, slot0);
-  if ((gated && !B.ctl[slot].refactor) || (spec.mat >= 0 && mat != spec.mat)) return;
+// the matrices of vel_matrices (velocity.f90:85-100)
+__device__ __forceinline__ LuSpec matrix_spec(int mat, const SlotParams& prm) {
+  const bool pr = mat == MAT_LNP;
+  return LuSpec{mat, pr || mat == MAT_LDZ ? 0 : (mat == MAT_LDP ? 1 : -1), pr ? 1 : 0, pr ? 0.0 : 1.0 / prm.dt,
+                pr ? 1.0 : -prm.implicit * prm.nu / prm.Re};
+}
+__device__ __forceinline__ void block_factor(const Geo& G, const Bufs& B, int slot, const LuSpec& A, int mat, int p,
+                                             int side, double alpha, const double* T) {
   const int N = G.N, P = G.P, NB = blk_count(N);
   const MeshOff mo = MeshOff::make(N);
   const double* me = G.mesh;
-  const SlotParams prm = B.prm[slot];
-  LuSpec A = spec;
-  if (spec.mat < 0) {
-    const bool pr = mat == MAT_LNP;
-    A = LuSpec{mat, pr || mat == MAT_LDZ ? 0 : (mat == MAT_LDP ? 1 : -1), pr ? 1 : 0, pr ? 0.0 : 1.0 / prm.dt,
-               pr ? 1.0 : -prm.implicit * prm.nu / prm.Re};
-  }
-  if (threadIdx.x == 0 && blockIdx.x == 0) B.spec[slot * 4 + mat] = A;
-  __shared__ double T[10 * (MAXN + 8)];   // MeshOff::lapT
-  for (int i = threadIdx.x; i < 10 * (N + 8); i += 64) T[i] = me[mo.lapT + i];
-  __syncthreads();
-  const int side = threadIdx.x & 1;
-  const int p = min(blockIdx.x * 32 + (int)(threadIdx.x >> 1), P - 1);   // spare lanes repeat the last pair
   const int m = p / G.K, k = p % G.K;
   const int S1 = (m * G.Mp + (A.PM != 0)) & 1;
   const double* ax = me + mo.dr0 + (KL + 1) * (1 - S1);   // axis row, columns 0..4
@@ -307,7 +296,7 @@ __global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot0, i
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * t + i;
-      const double dg = A.c2 * diag_d(me[mo.rinv2 + min(n, N - 1)], G.Mp, m, prm.alpha, k, A.PM) + A.c1;
+      const double dg = A.c2 * diag_d(me[mo.rinv2 + min(n, N - 1)], G.Mp, m, alpha, k, A.PM) + A.c1;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         double x = A.c2 * T[n * 10 + KL + j - i];
@@ -425,10 +414,21 @@ __global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot0, i
   if (side == 0) store(nm, D);
 }
 
+// one factor set of its own matrix (tim_lumesh_init).  grid: x = pairs / 32; 64 threads.
+__global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot, LuSpec A) {
+  __shared__ double T[10 * (MAXN + 8)];
+  for (int i = threadIdx.x; i < 10 * (G.N + 8); i += 64) T[i] = G.mesh[MeshOff::make(G.N).lapT + i];
+  if (threadIdx.x == 0 && blockIdx.x == 0) B.spec[slot * 4 + A.mat] = A;
+  __syncthreads();
+  // spare lanes repeat the last pair
+  block_factor(G, B, slot, A, A.mat, min((int)blockIdx.x * 32 + (int)(threadIdx.x >> 1), G.P - 1), threadIdx.x & 1,
+               B.prm[slot].alpha, T);
+}
+
 // ---------------------------------------------------------------------------
 // tim_lumesh_init (timestep.f90:67-96) + DGBTF2 of one matrix per pair in
 // LAPACK band layout, for tim_lumesh_get / tim_lumesh_invert (the time step
-// solves with k_block_factor's inverses).  Four lanes per system.
+// solves with block_factor's inverses).  Four lanes per system.
 // grid: x = pairs/16; 64 threads = 16 systems x 4 lanes.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot, int mat) {
@@ -670,132 +670,227 @@ __global__ void k_norm_sum(Geo G, const double* __restrict__ b, double* __restri
 }
 
 // ---------------------------------------------------------------------------
-// vel_adjPPE(0) influence vectors (velocity.f90:191-218) per pair, and
-// vel_adjustFlux(0) (velocity.f90:160-168) on pair 0.
+// vel_maxtstep (velocity.f90:438-481) from the per-plane maxima that the
+// theta kernel recorded for the last evaluation, and tim_new_tstep
+// (timestep.f90:259-278): cfl and its direction, and the new dt, nw whether
+// vel_matrices follows.  Every lane of a wave takes the planes n = lane,
+// lane + 64, ..; the minima are exact, so their order is free.
+// ---------------------------------------------------------------------------
+struct NewStep {
+  double cfl, dt;
+  int dir, ntc;
+  bool nw;
+};
+__device__ __forceinline__ NewStep new_tstep(const Geo& G, const Bufs& B, int slot, const SlotCtl& c,
+                                             const SlotParams& prm, int lane) {
+  const int N = G.N;
+  const MeshOff mo = MeshOff::make(N);
+  const double* r = G.mesh + mo.r;
+  const unsigned long long* mx = B.cflmax + (size_t)slot * 3 * N;
+  const double dth = (2.0 * D_PI) / (double)(G.T * G.Mp);
+  const double dz = (2.0 * D_PI) / (prm.alpha * (double)G.Z);
+  double t1 = 1e99, t2 = 1e99, t3 = 1e99;
+  for (int n = lane; n < N; n += 64) {
+    double d;
+    if (n == 0) d = r[1] - r[0];
+    else if (n == N - 1) d = r[N - 1] - r[N - 2];
+    else d = fmin(r[n] - r[n - 1], r[n + 1] - r[n]);
+    const double a = __longlong_as_double((long long)mx[n]);
+    const double b = __longlong_as_double((long long)mx[N + n]);
+    const double e = __longlong_as_double((long long)mx[2 * N + n]);
+    if (a != 0.0) t1 = fmin(t1, d / a);
+    if (b != 0.0) t2 = fmin(t2, dth / b);
+    if (e != 0.0) t3 = fmin(t3, dz / e);
+  }
+  for (int off = 32; off >= 1; off >>= 1) {
+    t1 = fmin(t1, __shfl_xor(t1, off));
+    t2 = fmin(t2, __shfl_xor(t2, off));
+    t3 = fmin(t3, __shfl_xor(t3, off));
+  }
+  NewStep s;
+  s.cfl = fmin(t1, fmin(t2, t3));
+  s.dir = c.cfl_dir;
+  if (s.cfl == t1) s.dir = 1;
+  if (s.cfl == t2) s.dir = 2;
+  if (s.cfl == t3) s.dir = 3;
+  // tim_new_tstep
+  const double dt0 = prm.dt;
+  double dt = fmin(dt0 * 1.11, prm.maxdt);
+  if (c.step == 0 && c.corr_dt == 0.0) dt = fmin(dt, s.cfl * 0.1);
+  if (s.cfl > 0.0) dt = fmin(dt, s.cfl * prm.courant);
+  if (c.corr_dt > 0.0) dt = fmin(dt, c.corr_dt * 0.95);
+  const int i = c.ntc - 1;
+  s.nw = dt < dt0 * 0.95 || (dt > dt0 * 1.10 && i < 0) || (dt == prm.maxdt && dt0 < dt && i < 0);
+  s.ntc = (s.nw && dt >= dt0) ? 99 : i;
+  s.dt = s.nw ? dt : dt0;
+  return s;
+}
+// vel_maxtstep alone (one wave)
+__global__ void k_maxtstep(Geo G, Bufs B, int slot) {
+  SlotCtl* c = &B.ctl[slot];
+  const NewStep s = new_tstep(G, B, slot, *c, B.prm[slot], threadIdx.x);
+  if (threadIdx.x != 0) return;
+  c->cfl_dt = s.cfl;
+  c->cfl_dir = s.dir;
+}
+
+// ---------------------------------------------------------------------------
+// vel_matrices (velocity.f90:85-100) of eight pairs per workgroup: the four
+// matrices' inverses (block_factor, all 64 lanes of wave 0), the influence
+// vectors of vel_adjPPE(0) (velocity.f90:191-218; wave w solves matrix w) with
+// vel_adjustFlux(0) (:160-168) on pair 0, and the inverted influence matrices
+// of the pairs' harmonics (:219-225).
 // Uinf slots: 0 U1 (LDp), 1 U2 (LDm), 2 U3 (LDz), 3 U4, 4 U5, 5 p (U6 = p*alpha*k).
-// One wave solves a matrix of eight pairs (four groups of two, solve.hpp); of
-// a pair's four columns the first holds its right-hand side and, for pair 0,
-// the second that of the flux problem.
-// grid: x = pairs/8, y = 4 matrices, z = slot.  SM >= blk_mid(N).
+// gate: 0 always; 1 where ctl.refactor asks for it; 2 a slot of the device
+// loop about to run a predictor with an adaptive time step: tim_new_tstep first,
+// and the rest where it changed dt.
+// One launch, since most launches find nothing to do and cost their few
+// microseconds all the same (an adaptive step of (48,48,24) spent 28 of its 115
+// us on four of them per evaluation; 106 now), and a set-up is a chain of
+// latencies: 41 us in three launches and 29 in this one at (32,24,12), 75 and
+// 57 at (64,64,48).
+// grid: x = pairs/8, z = slot.  SM >= blk_mid(N).
 // ---------------------------------------------------------------------------
 template <int SM>
-__global__ void __launch_bounds__(64) k_influence_t(Geo G, Bufs B, int slot0, int gated) {
-  constexpr int PW = 8;
+__global__ void __launch_bounds__(256) k_matrices_t(Geo G, Bufs B, int slot0, int gate) {
+  constexpr int PW = 8, XS = PW + 2;   // right-hand sides: the pairs', the flux problem's, and zeros
   const int p0 = blockIdx.x * PW;
-  const int mat = blockIdx.y;
   const int slot = slot_of(B, slot0);
-  if (gated && !B.ctl[slot].refactor) return;
-  const int N = G.N, P = G.P;
-  const int tid = threadIdx.x;
+  const int N = G.N, P = G.P, K = G.K;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int np = min(PW, P - p0);
+  SlotCtl* ctl = &B.ctl[slot];
+  SlotParams prm = B.prm[slot];
+  if (gate == 1 && !ctl->refactor) return;
+  if (gate == 2) {
+    const SlotCtl c = *ctl;
+    if (!(c.active && c.mode == MODE_PRED && prm.adaptive)) return;
+    const NewStep s = new_tstep(G, B, slot, c, prm, lane);
+    __syncthreads();
+    // every workgroup has read what the last one to arrive here writes
+    if (tid == 0 &&
+        __hip_atomic_fetch_add(&ctl->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+      ctl->arrived = 0u;
+      ctl->cfl_dt = s.cfl;
+      ctl->cfl_dir = s.dir;
+      ctl->ntc = s.ntc;
+      B.prm[slot].dt = s.dt;
+    }
+    if (!s.nw) return;
+    prm.dt = s.dt;
+  }
   const MeshOff mo = MeshOff::make(N);
   const double* me = G.mesh;
-  const SlotParams prm = B.prm[slot];
+  extern __shared__ double lap[];          // the Laplacian's rows
+  double* X = lap + 10 * (N + 8);          // [4][N + 4][XS]
+  double* W = X + 4 * (N + 4) * XS;        // [6][PW][KL + 1]: the vectors' rows at the wall
+  const int mat = wave;
   const bool flux = p0 == 0 && mat == MAT_LDZ && prm.const_flux != 0;
-  extern __shared__ double Xi[];   // [N + 4][PW][4], then the Laplacian's rows
-  double* lap = Xi + (size_t)(N + 4) * PW * 4;
-  for (int i = tid; i < (N + 4) * PW * 4; i += 64) {
-    const int n = i / (PW * 4), r = i & 3, ip = (i >> 2) % PW;
+  double* Xi = X + mat * (N + 4) * XS;
+  for (int i = tid; i < 10 * (N + 8); i += 256) lap[i] = me[mo.lapT + i];
+  for (int i = lane; i < (N + 4) * XS; i += 64) {
+    const int n = i / XS, r = i - n * XS;
     double v = 0.0;
-    if (r == 0 && n == N - 1) v = mat == MAT_LNP ? -1.0 : 1.0;
-    if (r == 1 && ip == 0 && flux) v = n == 0 || n >= N - 1 ? 0.0 : 1.0;
+    if (r < PW && n == N - 1) v = mat == MAT_LNP ? -1.0 : 1.0;
+    if (r == PW && flux) v = n == 0 || n >= N - 1 ? 0.0 : 1.0;
     Xi[i] = v;
   }
-  for (int i = tid; i < 10 * (N + 8); i += 64) lap[i] = me[mo.lapT + i];
   __syncthreads();
-  const BlkLane l = BlkLane::make(tid);
+  if (wave == 0) {
+    const int fm = lane >> 4, fp = (lane >> 1) & 7;
+    const LuSpec A = matrix_spec(fm, prm);
+    if (p0 == 0 && (lane & 15) == 0) B.spec[slot * 4 + fm] = A;
+    block_factor(G, B, slot, A, fm, p0 + min(fp, np - 1), lane & 1, prm.alpha, lap);   // spare lanes repeat the last pair
+  }
+  __syncthreads();
+  const BlkLane l = BlkLane::make(lane);
+  const LuSpec A = matrix_spec(mat, prm);
 #pragma unroll 1
   for (int g = 0; g < PW / 2; ++g) {
     BlkE<SM, 1> E;
-    const int pl = 2 * g + l.mi;   // a partial last group repeats its last matrix in the spare columns
-    blk_load(E, 0, G, B, slot, mat, p0 + min(pl, np - 1), l);
-    double* const x[1] = {Xi + pl * 4 + l.col};
-    blk_solve(E, N, l, lap, x, PW * 4);
+    const int pl = 2 * g + l.mi;
+    blk_load(E, 0, G, B, slot, A, mat, p0 + min(pl, np - 1), l);
+    double* const x[1] = {Xi + (l.col == 0 ? pl : l.col == 1 && pl == 0 ? PW : PW + 1)};
+    blk_solve(E, N, l, lap, x, XS);
   }
   __syncthreads();
   double* U = B.Uinf + (size_t)slot * 6 * N * P + p0;
   const size_t us = (size_t)N * P;
-  auto xv = [&](int n, int ip) { return Xi[(n * PW + ip) * 4]; };
-  for (int i = tid; i < N * PW; i += 64) {
-    const int n = i / PW, ip = i % PW;
+  for (int i = lane; i < N * PW; i += 64) {
+    const int n = i / PW, ip = i % PW, wr = n - (N - 1 - KL);
     if (ip >= np) continue;
     double* u = U + (size_t)n * P + ip;
+    double* w = W + ip * (KL + 1) + wr;
+    auto put = [&](int f, double v) {
+      u[f * us] = v;
+      if (wr >= 0) w[f * PW * (KL + 1)] = v;
+    };
+    const double x = Xi[n * XS + ip];
     if (mat != MAT_LNP) {
-      u[mat * us] = xv(n, ip);
+      put(mat, x);
     } else {
       // grad: dr1 . p (meshmult from 0), t.Im = p * m/r; rt2pm -> U4 = gr - tIm, U5 = gr + tIm
       double gr = 0.0;
 #pragma unroll
       for (int dd = -KL; dd <= KL; ++dd) {
         const int j = n + dd;
-        if (j >= 0 && j <= N - 1) gr = gr + me[mo.dr1b + (KL - dd) * N + j] * xv(j, ip);
+        if (j >= 0 && j <= N - 1) gr = gr + me[mo.dr1b + (KL - dd) * N + j] * Xi[j * XS + ip];
       }
-      const double mr = (me[mo.rinv + n] * (double)G.Mp) * (double)((p0 + ip) / G.K);
-      const double tIm = xv(n, ip) * mr;
-      u[5 * us] = xv(n, ip);
-      u[3 * us] = gr - tIm;
-      u[4 * us] = gr + tIm;
+      const double mr = (me[mo.rinv + n] * (double)G.Mp) * (double)((p0 + ip) / K);
+      const double tIm = x * mr;
+      put(5, x);
+      put(3, gr - tIm);
+      put(4, gr + tIm);
     }
   }
   if (p0 == 0 && mat == MAT_LDZ) {
     double* Ui = B.Ui + (size_t)slot * N;
-    for (int n = tid; n < N; n += 64) Ui[n] = Xi[n * PW * 4 + 1];
-    if (flux && tid == 0) {
+    for (int n = lane; n < N; n += 64) Ui[n] = Xi[n * XS + PW];
+    if (flux && lane == 0) {
       double s = 0.0;
-      for (int n = 0; n < N; ++n) s = s + Xi[n * PW * 4 + 1] * me[mo.intrdr + n];
-      B.ctl[slot].flux_d1 = 2.0 * s;
-      if (2.0 * s == 0.0) atomicMax(&B.ctl[slot].status, 110);
+      for (int n = 0; n < N; ++n) s = s + Xi[n * XS + PW] * me[mo.intrdr + n];
+      ctl->flux_d1 = 2.0 * s;
+      if (2.0 * s == 0.0) atomicMax(&ctl->status, 110);
     }
   }
-}
-
-FactorKern influence_kernel(int N) {
-  static_assert(blk_mid(32) == 4 && blk_mid(64) == 8 && blk_mid(96) == 12 && blk_mid(MAXN) == 16, "the ranges");
-  return N <= 32 ? k_influence_t<4> : N <= 64 ? k_influence_t<8> : N <= 96 ? k_influence_t<12> : k_influence_t<16>;
-}
-
-// Inverted 4x4 influence matrices per harmonic (velocity.f90:219-225).
-__global__ void k_ainv(Geo G, Bufs B, int slot0, int gated) {
-  const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  const int slot = slot_of(B, slot0);
-  if (h >= G.H || (gated && !B.ctl[slot].refactor)) return;
-  int k, m;
-  harmonic_km(h, G.K, k, m);
+  __syncthreads();
+  // harmonics +k and -k of the pairs
+  const int ip = tid & (PW - 1), p = p0 + ip, m = p / K, ka = p - m * K, k = tid & PW ? -ka : ka;
+  if (tid >= 2 * PW || ip >= np || (k < 0 && m == 0) || (tid >= PW && ka == 0)) return;
+  const int h = m == 0 ? k : K + (m - 1) * (2 * K - 1) + k + K - 1;
   double* Ai = B.Ainv + (size_t)slot * 16 * G.H + h;
-  if (k == 0 && m == 0) {
+  if (p == 0) {
     for (int q = 0; q < 16; ++q) Ai[(size_t)q * G.H] = 0.0;
     return;
   }
-  const int N = G.N, P = G.P;
-  const int p = m * G.K + (k < 0 ? -k : k);
-  const SlotParams prm = B.prm[slot];
-  const MeshOff mo = MeshOff::make(N);
-  const double* me = G.mesh;
-  const double* U = B.Uinf + (size_t)slot * 6 * N * P + p;
   const double ak = prm.alpha * (double)k;
-  const double d = me[mo.rinv + N - 1];
-  const double m_ = (double)(m * G.Mp);
-  double A[16];
+  double M4[16];
   for (int j = 0; j < 4; ++j) {
     double2 up[KL + 1], um[KL + 1], uz[KL + 1];
     for (int i = 0; i <= KL; ++i) {
-      const size_t n = (size_t)(N - 1 - KL + i) * P;
+      const double* w = W + ip * (KL + 1) + i;
+      constexpr int fs = PW * (KL + 1);
       up[i] = um[i] = uz[i] = make_double2(0.0, 0.0);
-      if (j == 0) up[i].x = U[n];
-      if (j == 1) um[i].x = U[(size_t)N * P + n];
-      if (j == 2) uz[i].y = U[(size_t)2 * N * P + n];
+      if (j == 0) up[i].x = w[0];
+      if (j == 1) um[i].x = w[fs];
+      if (j == 2) uz[i].y = w[2 * fs];
       if (j == 3) {
-        up[i].x = U[(size_t)3 * N * P + n];
-        um[i].x = U[(size_t)4 * N * P + n];
-        uz[i].y = U[(size_t)5 * N * P + n] * ak;
+        up[i].x = w[3 * fs];
+        um[i].x = w[4 * fs];
+        uz[i].y = w[5 * fs] * ak;
       }
     }
     double BRe[4], BIm[4];
-    eval_bc(up, um, uz, me + mo.dr1 + (KL + 1), d, m_, ak, BRe, BIm);
-    for (int i = 0; i < 4; ++i) A[i * 4 + j] = BRe[i];
+    eval_bc(up, um, uz, me + mo.dr1 + (KL + 1), me[mo.rinv + N - 1], (double)(m * G.Mp), ak, BRe, BIm);
+    for (int i = 0; i < 4; ++i) M4[i * 4 + j] = BRe[i];
   }
-  if (!inv4(A)) atomicMax(&B.ctl[slot].status, 120);
-  for (int q = 0; q < 16; ++q) Ai[(size_t)q * G.H] = A[q];
+  if (!inv4(M4)) atomicMax(&ctl->status, 120);
+  for (int q = 0; q < 16; ++q) Ai[(size_t)q * G.H] = M4[q];
+}
+
+MatricesKern matrices_kernel(int N) {
+  static_assert(blk_mid(32) == 4 && blk_mid(64) == 8 && blk_mid(96) == 12 && blk_mid(MAXN) == 16, "the ranges");
+  return N <= 32 ? k_matrices_t<4> : N <= 64 ? k_matrices_t<8> : N <= 96 ? k_matrices_t<12> : k_matrices_t<16>;
 }
 
 // ---------------------------------------------------------------------------
@@ -1258,73 +1353,6 @@ __global__ void k_imposesym(Geo G, Bufs B, int slot0) {
   u[o] = make_double2(0.0, 0.0);
   u[G.coll + o].y = 0.0;
   u[2 * G.coll + o].y = 0.0;
-}
-
-// ---------------------------------------------------------------------------
-// vel_maxtstep (velocity.f90:438-481) from the per-plane maxima that the
-// theta kernel recorded for the last evaluation, and tim_new_tstep
-// (timestep.f90:259-278).  what = 0: the device loop: for adaptive slots
-// about to run a predictor, both, with tim_new_dt left in `refactor` for the
-// gated vel_matrices launches that follow (every other slot: refactor = 0);
-// what = 1: vel_maxtstep only.  One wave per slot: lane l takes the planes
-// n = l, l+64, ...; the minima are exact, so their order is free.
-// ---------------------------------------------------------------------------
-__global__ void k_newdt(Geo G, Bufs B, int slot0, int what) {
-  const int slot = slot_of(B, slot0);
-  SlotCtl* c = &B.ctl[slot];
-  SlotParams* prm = &B.prm[slot];
-  const int lane = threadIdx.x;
-  if (what == 0) {
-    const bool act = c->active && c->mode == MODE_PRED && prm->adaptive;
-    if (!act) {
-      if (lane == 0) c->refactor = 0;
-      return;
-    }
-  }
-  const int N = G.N;
-  const MeshOff mo = MeshOff::make(N);
-  const double* r = G.mesh + mo.r;
-  const unsigned long long* mx = B.cflmax + (size_t)slot * 3 * N;
-  const double dth = (2.0 * D_PI) / (double)(G.T * G.Mp);
-  const double dz = (2.0 * D_PI) / (prm->alpha * (double)G.Z);
-  double t1 = 1e99, t2 = 1e99, t3 = 1e99;
-  for (int n = lane; n < N; n += 64) {
-    double d;
-    if (n == 0) d = r[1] - r[0];
-    else if (n == N - 1) d = r[N - 1] - r[N - 2];
-    else d = fmin(r[n] - r[n - 1], r[n + 1] - r[n]);
-    const double a = __longlong_as_double((long long)mx[n]);
-    const double b = __longlong_as_double((long long)mx[N + n]);
-    const double e = __longlong_as_double((long long)mx[2 * N + n]);
-    if (a != 0.0) t1 = fmin(t1, d / a);
-    if (b != 0.0) t2 = fmin(t2, dth / b);
-    if (e != 0.0) t3 = fmin(t3, dz / e);
-  }
-  for (int off = 32; off >= 1; off >>= 1) {
-    t1 = fmin(t1, __shfl_xor(t1, off));
-    t2 = fmin(t2, __shfl_xor(t2, off));
-    t3 = fmin(t3, __shfl_xor(t3, off));
-  }
-  if (lane != 0) return;
-  const double cfl = fmin(t1, fmin(t2, t3));
-  int dir = c->cfl_dir;
-  if (cfl == t1) dir = 1;
-  if (cfl == t2) dir = 2;
-  if (cfl == t3) dir = 3;
-  c->cfl_dt = cfl;
-  c->cfl_dir = dir;
-  if (what == 1) return;
-  // tim_new_tstep
-  const double dt0 = prm->dt;
-  double dt = fmin(dt0 * 1.11, prm->maxdt);
-  if (c->step == 0 && c->corr_dt == 0.0) dt = fmin(dt, cfl * 0.1);
-  if (cfl > 0.0) dt = fmin(dt, cfl * prm->courant);
-  if (c->corr_dt > 0.0) dt = fmin(dt, c->corr_dt * 0.95);
-  const int i = c->ntc - 1;
-  const bool nw = dt < dt0 * 0.95 || (dt > dt0 * 1.10 && i < 0) || (dt == prm->maxdt && dt0 < dt && i < 0);
-  c->ntc = (nw && dt >= dt0) ? 99 : i;
-  if (nw) prm->dt = dt;
-  c->refactor = nw ? 1 : 0;
 }
 
 // tim_lumesh_invert (timestep.f90:102-123) of one coll field x[n][Hp] with

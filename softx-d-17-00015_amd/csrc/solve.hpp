@@ -72,10 +72,11 @@ struct BlkE {
   double rs[NG];      // scale of the solution, -1 / c2
 };
 
-// Loads of group g: matrix `mat` of pair p (this lane's), its m for the parity.
+// Loads of group g: the set `mat` of pair p (this lane's), holding the matrix s;
+// p's m gives the parity.
 template <int SM, int NG>
-__device__ __forceinline__ void blk_load(BlkE<SM, NG>& R, int g, const Geo& G, const Bufs& B, int slot, int mat, int p,
-                                         const BlkLane& l) {
+__device__ __forceinline__ void blk_load(BlkE<SM, NG>& R, int g, const Geo& G, const Bufs& B, int slot, const LuSpec& s,
+                                         int mat, int p, const BlkLane& l) {
   const int N = G.N;
   const BlkSweep sw = BlkSweep::make(N, l.side);
   const char* base = (const char*)(B.SE + (size_t)slot * 4 * G.P * sw.NB * 16);
@@ -87,7 +88,6 @@ __device__ __forceinline__ void blk_load(BlkE<SM, NG>& R, int g, const Geo& G, c
       R.e[g][i] = *(const double*)(base + (o + (unsigned)t * 128u));
     }
   R.e[g][SM] = *(const double*)(base + (o + (unsigned)sw.S * 128u));
-  const LuSpec s = B.spec[slot * 4 + mat];
   R.rs[g] = -1.0 / blk_scale(s.c2);
   // row 0 reaches one column of block 1, dr0(5, 1 - S); row N-1 the columns
   // N-5 .. of block NB-2
