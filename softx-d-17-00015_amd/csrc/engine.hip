@@ -259,15 +259,19 @@ Tuned lookup_tuning(int N, int K, int M, int cap) {
 
 size_t step_smem(int N, int gp) { return round_up(step_lds_doubles(N, gp) * sizeof(double), 16); }
 
-// Pairs per workgroup of the fused step kernel.  Four pairs (N <= 96) write
-// longer runs of each field's rows and share a stage's barriers among twice
-// the harmonics; they are the default when the slots give at least three such
-// workgroups per CU (40 KiB of LDS each at N = 64), otherwise two pairs.
+// Pairs per workgroup of the fused step kernel.  Two pairs where their
+// workgroups are all resident at once (three per CU; up to N = 32, where the
+// kernel is short, one per CU), otherwise four (N <= 96), which write longer
+// runs of each field's rows and need half the rounds.  us per launch with two
+// and four, and workgroups of two per CU: (48,48,32) 23.6 24.8, 3; (64,48,32)
+// 27.8 28.1, 3; (64,64,36) 42.9 35.0, 4.5; (64,64,48) 48.9 37.1, 6; (80,48,32)
+// 32.5 35.0, 3; (96,64,48) 84.9 77.4, 6; (32,24,12) 13.1 13.8, 0.6; (32,32,24)
+// 16.6 15.9, 1.5.
 StepTiles choose_step_tiles(int N, int P, int cap, int ncu, int gp_req, size_t lds_max) {
   StepTiles t{};
   int gp = gp_req;
   if (gp <= 0)
-    gp = (N <= 96 && step_smem(N, 4) <= lds_max && (long long)((P + 3) / 4) * cap >= 3LL * ncu) ? 4 : 2;
+    gp = (N <= 96 && step_smem(N, 4) <= lds_max && (long long)((P + 1) / 2) * cap > (N <= 32 ? 1LL : 3LL) * ncu) ? 4 : 2;
   if (gp != 1 && gp != 2 && gp != 4) throw OpfError(OPF_ERR_ARG, "step pairs per workgroup must be 1, 2 or 4");
   if (gp == 4 && N > 96) throw OpfError(OPF_ERR_ARG, "four pairs per workgroup need N <= 96");
   t.gp = gp;

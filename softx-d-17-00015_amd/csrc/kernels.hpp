@@ -91,12 +91,10 @@ constexpr int ARRIVE_WORDS = 16;
 __host__ __device__ constexpr size_t arrive_words(int P) { return 16 * ARRIVE_WORDS + (size_t)P; }
 inline int step_threads(int gp) { return gp == 1 ? 128 : 256; }
 // LDS of a step workgroup in doubles: V[3][N + 8][2 gp] (complex, four rows of
-// zeros at either end), the mesh tables (MeshOff::lapT, d1T, rowv; with four
-// pairs beyond 64 points the latter two stay in the cache, so that three
-// workgroups fit in a CU), the influence coefficients and the reduction words.
-__host__ __device__ constexpr bool step_d1_in_lds(int N, int gp) { return !(gp == 4 && N > 64); }
+// zeros at either end), the mesh tables (MeshOff::lapT, d1T, rowv), the
+// influence coefficients and the reduction words.
 __host__ __device__ constexpr size_t step_lds_doubles(int N, int gp) {
-  return (size_t)12 * (N + 8) * gp + 10 * (N + 8) + (step_d1_in_lds(N, gp) ? 13 * N + (N & 1) : 0) + 16 * gp + 16;
+  return (size_t)12 * (N + 8) * gp + 10 * (N + 8) + 13 * N + (N & 1) + 16 * gp + 16;
 }
 
 constexpr int FFT_THREADS = 256;

@@ -25,7 +25,9 @@
 // checks, and the sums are fused multiply-adds.  Against the row-by-row solves
 // with their LDS ring of factors, and separately rounded stencils, this took a
 // launch from 69 to 41 us at (64,64,48) (148 MB, 3.6 TB/s), 1395 to 860 us at
-// (96,256,128), 26.5 to 11.7 us at (32,24,12) and 21.8 to 10.9 us at (16,6,4).
+// (96,256,128), 26.5 to 11.7 us at (32,24,12) and 21.8 to 10.9 us at (16,6,4);
+// without spilled registers 37 and 723 us at the larger two, the control step
+// included.
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
@@ -223,17 +225,15 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   // LDS (step_lds_doubles): V, rows -4 .. N+3; LT, the Laplacian's rows; DT,
   // the first derivative's, and Ubase, 2r, 1/r^2; the influence coefficients;
   // reduction words
-  constexpr bool DWL = !(GP == 4 && IT > 2);   // = step_d1_in_lds
   extern __shared__ double2 lds2[];
   const int VC = (N + 8) * GH;      // double2 per field
   double2* V = lds2 + KL * GH;      // V[c * VC + n * GH + lh]
   double* LT = (double*)(lds2 + 3 * VC);
   double* DT = LT + 10 * (N + 8);
-  double* AC = DT + (DWL ? 13 * N + (N & 1) : 0);   // [GH][8]
-  double* RED = AC + GH * 8;                        // [16]
+  double* AC = DT + 13 * N + (N & 1);   // [GH][8]
+  double* RED = AC + GH * 8;            // [16]
   double* EN = (double*)(V + 2 * VC);               // energy terms [2][N][GH] in V's third field
-  const double* D1 = DWL ? DT : me + mo.d1T;
-  const double* RV = DWL ? DT + 10 * N : me + mo.rowv;
+  const double* RV = DT + 10 * N;
 
   const double th = prm.implicit, th1 = 1.0 - prm.implicit;
   const double c1 = 1.0 / prm.dt;
@@ -262,8 +262,8 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   // ---- stage 0: loads ------------------------------------------------------
   // the mesh tables first (one batch, ahead of the state loads)
   constexpr int WMAX = DN * IT;   // N <= WMAX
-  constexpr int TT = ((10 * (WMAX + 8) + (DWL ? 13 * WMAX + 1 : 0)) / 2 + THR - 1) / THR;
-  const int ntab = (10 * (N + 8) + (DWL ? 13 * N : 0) + 1) / 2;   // d1T and rowv follow lapT
+  constexpr int TT = ((23 * WMAX + 81) / 2 + THR - 1) / THR;
+  const int ntab = (10 * (N + 8) + 13 * N + 1) / 2;   // d1T and rowv follow lapT
   double2 tab[TT];
 #pragma unroll
   for (int u = 0; u < TT; ++u) {
@@ -282,17 +282,30 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
       vn[q][c] = *(const double2*)(Nc + (size_t)(c * cb) + o);
     }
   }
+  auto load_np = [&]() {
+#pragma unroll
+    for (int q = 0; q < IT; ++q) {
+      const int n = n0 + q * DN;
+      const unsigned o = n < N && S.valid ? (unsigned)n * rb + ho : 0u;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) vp[q][c] = *(const double2*)(Np + (size_t)(c * cb) + o);
+    }
+  };
+  // Registers: with two items, a thread's loads of N_ wait for the others and
+  // the influence loads stand behind the Helmholtz solve, which leaves three
+  // waves a SIMD without spills (44.8 us with 21 spilled registers, 37.1 without,
+  // at (64,64,48)); with three, two waves of 256 registers are better than
+  // three of 168 (886 to 723 us at (96,256,128)).
+  constexpr bool LATE_NP = IT == 2;
   if (corr) {
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
       const int n = n0 + q * DN;
       const unsigned o = n < N && S.valid ? (unsigned)n * rb + ho : 0u;
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        vc[q][c] = *(const double2*)(uc + (size_t)(c * cb) + o);
-        vp[q][c] = *(const double2*)(Np + (size_t)(c * cb) + o);
-      }
+      for (int c = 0; c < 3; ++c) vc[q][c] = *(const double2*)(uc + (size_t)(c * cb) + o);
     }
+    if (!LATE_NP) load_np();
   }
   // the mean flow's pressure gradients of both iterates (harmonic (0,0))
   double prc = 0.0, prb = 0.0;
@@ -336,7 +349,6 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
 #pragma unroll
   for (int q = 0; q < IT; ++q) {
     const int n = n0 + q * DN;
-    res[q][0] = res[q][1] = res[q][2] = make_double2(0.0, 0.0);
     if (n >= N || !S.valid) continue;
     const double a = ak * RV[n];
     const double b = RV[N + n];
@@ -346,6 +358,23 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
     nt = make_double2(fma(a, uct.y, nt.x), fma(-a, uct.x, nt.y));
     nz = make_double2(fma(b, ucr.x, fma(a, ucz.y, nz.x)), fma(b, ucr.y, fma(-a, ucz.x, nz.y)));
     if (S.h00) nz.x = nz.x + (4.0 * prc) / prm.Re;
+    vn[q][0] = nr;
+    vn[q][1] = nt;
+    vn[q][2] = nz;
+  }
+  if (LATE_NP && corr) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_np();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int q = 0; q < IT; ++q) {
+    const int n = n0 + q * DN;
+    res[q][0] = res[q][1] = res[q][2] = make_double2(0.0, 0.0);
+    if (n >= N || !S.valid) continue;
+    const double a = ak * RV[n];
+    const double b = RV[N + n];
+    double2 nr = vn[q][0], nt = vn[q][1], nz = vn[q][2];
     if (corr) {
       const double2 bur = vb[q][0], but = vb[q][1], buz = vb[q][2];
       double2 pr = vp[q][0], pt = vp[q][1], pz = vp[q][2];
@@ -451,7 +480,7 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
     double2 dv = make_double2(0.0, 0.0);
     if (S.valid && !S.h00 && n != 0 && n != N - 1) {
       double w[10];
-      row10(D1 + 10 * n, w);
+      row10(DT + 10 * n, w);
       const double2* v = V + (n - KL) * GH + lh;
       double2 d = make_double2(0.0, 0.0);
 #pragma unroll
@@ -491,7 +520,7 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
     double2 r0 = make_double2(0.0, 0.0), r1 = r0, r2 = r0;
     if (n != 0 && n != N - 1) {
       double w[10];
-      row10(D1 + 10 * n, w);
+      row10(DT + 10 * n, w);
       const double2* v = V + 2 * VC + (n - KL) * GH + lh;
       double2 gr = make_double2(0.0, 0.0);
 #pragma unroll
@@ -551,7 +580,7 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
       for (int j = 0; j < 4; ++j) ai[j] = B.Ainv[(size_t)slot * 16 * G.H + (size_t)(ci * 4 + j) * G.H + CS.h];
     }
   };
-  constexpr bool EARLY = IT * 24 + SM * 8 <= 112;
+  constexpr bool EARLY = IT != 2;
   if (EARLY || !solver) influence_loads();
   if (solver) {
     double* xp = (double*)(V + lhs) + (bl.col & 1);
@@ -689,7 +718,7 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
     const int n = n0 + q * DN;
     if (n >= N || !S.valid) continue;
     double w[10];
-    row10(D1 + 10 * n, w);
+    row10(DT + 10 * n, w);
     const double2* v = V + (n - KL) * GH + lh;
     double2 d1 = make_double2(0.0, 0.0), d2 = d1;
 #pragma unroll
@@ -783,10 +812,10 @@ StepKern step_kernel(int N, int gp) {
   static_assert(blk_mid(32) == 4 && blk_mid(64) == 8 && blk_mid(96) == 12 && blk_mid(MAXN) == 16, "the ranges");
   const int r = N <= 32 ? 0 : N <= 64 ? 1 : N <= 96 ? 2 : 3;
   static const StepKern g1[] = {k_step_t<1, 1, 128, 4, 3>, k_step_t<1, 1, 128, 8, 3>, k_step_t<1, 2, 128, 12, 3>,
-                                k_step_t<1, 2, 128, 16, 3>};
+                                k_step_t<1, 2, 128, 16, 2>};
   static const StepKern g2[] = {k_step_t<2, 1, 256, 4, 3>, k_step_t<2, 1, 256, 8, 3>, k_step_t<2, 2, 256, 12, 3>,
                                 k_step_t<2, 2, 256, 16, 2>};
-  static const StepKern g4[] = {k_step_t<4, 1, 256, 4, 3>, k_step_t<4, 2, 256, 8, 3>, k_step_t<4, 3, 256, 12, 3>};
+  static const StepKern g4[] = {k_step_t<4, 1, 256, 4, 3>, k_step_t<4, 2, 256, 8, 3>, k_step_t<4, 3, 256, 12, 2>};
   return gp == 1 ? g1[r] : gp == 2 ? g2[r] : g4[r];
 }
 
