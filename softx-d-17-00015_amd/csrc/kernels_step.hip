@@ -614,6 +614,49 @@ __global__ void k_add_coll(Geo G, double2* dst, const double2* src) {
 }
 
 // ---------------------------------------------------------------------------
+// Device rows u[comp][n][Hp] <-> the reference's coll planes, of a component
+// re[h][n] then im[h][n] (r fastest), through LDS tiles of 32 x 32 so that both
+// sides move whole lines.  The host's loops over both layouts took 100 ms for
+// the 300 MB of a (96,256,128) state, whose copy needs 11.
+// grid: x = 32-harmonic tiles of a row (Hp, the padding included: zeros), y =
+// 32-point tiles, z = component; 256 threads.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) k_rows_to_planes(Geo G, const double2* __restrict__ rows,
+                                                        double* __restrict__ planes) {
+  __shared__ double2 t[32][33];
+  const int h0 = blockIdx.x * 32, n0 = blockIdx.y * 32, lo = threadIdx.x & 31, hi = threadIdx.x >> 5;
+  const size_t nh = (size_t)G.N * G.H;
+  rows += blockIdx.z * G.coll;
+  planes += blockIdx.z * 2 * nh;
+  for (int i = hi; i < 32; i += 8)
+    if (n0 + i < G.N && h0 + lo < G.H) t[i][lo] = rows[(size_t)(n0 + i) * G.Hp + h0 + lo];
+  __syncthreads();
+  for (int i = hi; i < 32; i += 8)
+    if (n0 + lo < G.N && h0 + i < G.H) {
+      const double2 v = t[lo][i];
+      const size_t o = (size_t)(h0 + i) * G.N + n0 + lo;
+      planes[o] = v.x;
+      planes[nh + o] = v.y;
+    }
+}
+__global__ void __launch_bounds__(256) k_planes_to_rows(Geo G, const double* __restrict__ planes,
+                                                        double2* __restrict__ rows) {
+  __shared__ double2 t[32][33];
+  const int h0 = blockIdx.x * 32, n0 = blockIdx.y * 32, lo = threadIdx.x & 31, hi = threadIdx.x >> 5;
+  const size_t nh = (size_t)G.N * G.H;
+  rows += blockIdx.z * G.coll;
+  planes += blockIdx.z * 2 * nh;
+  for (int i = hi; i < 32; i += 8) {
+    const size_t o = (size_t)(h0 + i) * G.N + n0 + lo;
+    const bool in = n0 + lo < G.N && h0 + i < G.H;
+    t[lo][i] = in ? make_double2(planes[o], planes[nh + o]) : make_double2(0.0, 0.0);
+  }
+  __syncthreads();
+  for (int i = hi; i < 32; i += 8)
+    if (n0 + i < G.N && h0 + lo < G.Hp) rows[(size_t)(n0 + i) * G.Hp + h0 + lo] = t[i][lo];
+}
+
+// ---------------------------------------------------------------------------
 // var_coll_norm (variables.f90:718-751) of a field in the reference's coll
 // layout (re, im: N x H, r fastest).  Pass 1, one thread per harmonic:
 // b(h) = sum_n f(n) intrdr(n) with f = w (re^2 + im^2), w = 4 pi^2 / alpha,
