@@ -122,6 +122,7 @@ struct opf_ctx {
   double* normBuf = nullptr;     // opf_var_coll_norm: field, partials and sums (first use)
   double* stage[2] = {nullptr, nullptr};   // pinned pieces of fields on their way to or from the host (first use)
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
+  double* dterrHost = nullptr;   // pinned: tim_dterr of the last host-driven call (first use)
   SlotParams* prmHost = nullptr; // pinned parameters of asynchronous admissions (first use)
   std::vector<int> lu_bc;        // BC of each factor set [slot][4] (tim_lumesh_invert's (0,0) rule)
   int device = 0;                // HIP device of the context
@@ -1184,23 +1185,19 @@ void orbit_finish(opf_ctx* c, const std::vector<int>& sel, const std::vector<dou
 }  // namespace
 
 namespace {
-// run `fn` with the slot marked active (kernels skip inactive slots)
-template <typename F> void with_active(opf_ctx* c, int slot, int mode, F&& fn) {
+// run `fn` with the slot marked active (kernels skip inactive slots); returns
+// tim_dterr.  The marks are kernels on the stream: reading the control block
+// back and writing it, before and after, cost more than the work of most calls
+// (a host's loop over (48,48,24) took 625 us per step, 110 of it in kernels).
+template <typename F> double with_active(opf_ctx* c, int slot, int mode, F&& fn) {
   check_slot(c, slot);
   if (!c->occupied[slot]) throw OpfError(OPF_ERR_STATE, "slot holds no state");
-  auto ctl = read_ctl(c);
-  ctl[slot].active = 1;
-  ctl[slot].target_steps = -1;
-  if (mode >= 0) ctl[slot].mode = mode;
-  ctl[slot].diag_every = 0;
-  ctl[slot].corr_fixed = 0;
-  ctl[slot].host_driven = 1;
-  write_ctl(c, ctl);
+  if (!c->dterrHost) HIPCHK(hipHostMalloc((void**)&c->dterrHost, sizeof(double), hipHostMallocDefault));
+  launch(c, "host_call", k_host_call, dim3(1), dim3(1), 0, c->B, slot, 1, mode, c->dterrHost);
   fn();
+  launch(c, "host_call", k_host_call, dim3(1), dim3(1), 0, c->B, slot, 0, mode, c->dterrHost);
   HIPCHK(hipStreamSynchronize(c->stream));
-  ctl = read_ctl(c);
-  ctl[slot].active = 0;
-  write_ctl(c, ctl);
+  return *c->dterrHost;
 }
 }  // namespace
 
@@ -1245,6 +1242,7 @@ int opf_ctx_destroy(opf_ctx* c) {
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   if (c->stream2) (void)hipStreamDestroy(c->stream2);
   if (c->prmHost) (void)hipHostFree(c->prmHost);
+  if (c->dterrHost) (void)hipHostFree(c->dterrHost);
   for (int b = 0; b < 2; ++b) {
     if (c->stage[b]) (void)hipHostFree(c->stage[b]);
     if (c->stage_ev[b]) (void)hipEventDestroy(c->stage_ev[b]);
@@ -1522,7 +1520,6 @@ int opf_vel_imposesym(opf_ctx* c, int slot) {
              0);
       launch(c, "curl", k_curl, grid_hn(c, 1), dim3(64), 0, c->G, c->B, slot, 0);
     });
-    HIPCHK(hipStreamSynchronize(c->stream));
   });
 }
 
@@ -1551,10 +1548,8 @@ int opf_vel_predictor(opf_ctx* c, int slot) {
 
 int opf_vel_corrector(opf_ctx* c, int slot, double* dterr) {
   return guard([&] {
-    with_active(c, slot, MODE_CORR, [&] { launch_step(c, slot, 1); });
-    auto ctl = read_ctl(c);
-    if (dterr) *dterr = ctl[slot].last_dterr;
-
+    const double d = with_active(c, slot, MODE_CORR, [&] { launch_step(c, slot, 1); });
+    if (dterr) *dterr = d;
   });
 }
 

@@ -1385,6 +1385,25 @@ __global__ void k_admit(Bufs B, int slot, int phase, int nsteps, int corr_fixed)
   B.ctl[slot] = k;
 }
 
+// A host-driven call on one slot, in stream order (one thread): begin marks the
+// slot active, for the launches between, as a single procedure of the host's
+// own loop (mode < 0: as it is); the end clears the mark and reports tim_dterr
+// to host memory.
+__global__ void k_host_call(Bufs B, int slot, int begin, int mode, double* dterr) {
+  SlotCtl* c = &B.ctl[slot];
+  if (begin) {
+    c->active = 1;
+    c->target_steps = -1;
+    if (mode >= 0) c->mode = mode;
+    c->diag_every = 0;
+    c->corr_fixed = 0;
+    c->host_driven = 1;
+  } else {
+    c->active = 0;
+    *dterr = c->last_dterr;
+  }
+}
+
 // var_imposesym(0) (variables.f90:611-616) on harmonic 0 of U[ucur].
 __global__ void k_imposesym(Geo G, Bufs B, int slot0) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
