@@ -112,8 +112,8 @@ struct opf_ctx {
   double* lesD = nullptr;      // per slot [Delta, Delta_r, L_theta, coef] x N
   unsigned long long* lesMax = nullptr;   // per slot nu_max (bit pattern)
   double* nnP = nullptr;       // non-Newtonian physical fields (16 of N*Z*T), first use
-  double2* nnC = nullptr;      // non-Newtonian coll temporaries (4 of coll), first use
-  double2* nnY = nullptr;      // their z-transform intermediates (3 fields), first use
+  double2* nnC = nullptr;      // non-Newtonian coll temporaries (9 of coll), first use
+  double2* nnY = nullptr;      // their z-transform intermediates (9 fields), first use
   // granular transform temporaries (allocated on first use)
   double2* tY = nullptr;
   double* tP = nullptr;
@@ -490,10 +490,6 @@ void ensure_temps(opf_ctx* c) {
   c->tC = c->alloc<double2>(c->G.coll);
 }
 
-// Transforms of nf coll fields (stride coll) to / from physical fields
-// (stride N*Z*T) on device buffers for the plugins (tra_spec2phys /
-// tra_phys2spec, transform.fftw3.f90:65-147), one launch per stage with the
-// field as grid z; physical fields in the plugins' layout [n][z][theta].
 // one coll field to / from the planes Y of its z transform (nf fields)
 void launch_zfwd_one(opf_ctx* c, const double2* src, double2* Y, int nf) {
   launch(c, "zfwd1", c->fk.zfwd1, dim3(ztile_blocks(c, 1), 1, nf), dim3(c->fk.zn), c->fk.zfs, c->G, c->B, c->fk.t, src,
@@ -503,6 +499,11 @@ void launch_zbwd_one(opf_ctx* c, const double2* Y, double2* dst, int nf) {
   launch(c, "zbwd1", c->fk.zbwd1, dim3(ztile_blocks(c, 1), 1, nf), dim3(c->fk.zn), c->fk.zbs, c->G, c->B, c->fk.t, Y,
          dst, y_one(c), (size_t)c->G.coll);
 }
+// Transforms of nf coll fields (stride coll) to / from physical fields
+// (stride N*Z*T) on device buffers for the plugins (tra_spec2phys /
+// tra_phys2spec, transform.fftw3.f90:65-147), one launch per stage with the
+// field as grid z; physical fields in the plugins' layout [n][z][theta].  The
+// padding of the coll rows is left as it is (no kernel reads it).
 dim3 grid_lines(const opf_ctx* c, int nf) { return dim3((c->Z + 2 * c->fk.bt - 1) / (2 * c->fk.bt), c->N, nf); }
 void coll2phys_dev(opf_ctx* c, const double2* src, double* dst, int nf) {
   launch_zfwd_one(c, src, c->nnY, nf);
@@ -510,7 +511,6 @@ void coll2phys_dev(opf_ctx* c, const double2* src, double* dst, int nf) {
          (const double2*)c->nnY, dst, y_one(c), (size_t)c->N * c->Z * c->T);
 }
 void phys2coll_dev(opf_ctx* c, const double* src, double2* dst, int nf) {
-  HIPCHK(hipMemsetAsync(dst, 0, sizeof(double2) * c->G.coll * nf, c->stream));
   launch(c, "r2c_lines", c->fk.r2c, grid_lines(c, nf), dim3(c->fk.ln), c->fk.r2cs, c->G, c->B, c->fk.t, c->fk.bt, src,
          c->nnY, (size_t)c->N * c->Z * c->T, y_one(c));
   launch_zbwd_one(c, c->nnY, dst, nf);
@@ -524,8 +524,8 @@ NnPhys visc_fields(opf_ctx* c) {
   ensure_temps(c);
   const size_t np = (size_t)c->N * c->Z * c->T;
   if (!c->nnP) c->nnP = c->alloc<double>(16 * np);
-  if (!c->nnC) c->nnC = c->alloc<double2>(4 * c->G.coll);
-  if (!c->nnY) c->nnY = c->alloc<double2>(3 * y_one(c));
+  if (!c->nnC) c->nnC = c->alloc<double2>(9 * c->G.coll);
+  if (!c->nnY) c->nnY = c->alloc<double2>(9 * y_one(c));
   NnPhys P{};
   for (int i = 0; i < 9; ++i) P.S[i] = c->nnP + (size_t)i * np;
   P.nu = c->nnP + 9 * np;
@@ -534,28 +534,22 @@ NnPhys visc_fields(opf_ctx* c) {
   return P;
 }
 void visc_gradient(opf_ctx* c, int slot, const NnPhys& P) {
-  double2* c3 = c->nnC;
-  for (int row = 0; row < 3; ++row) {          // A(row, j), velocity-gradient rows
-    launch(c, "nn_grad", k_nn_grad, dim3((c->H + 63) / 64, c->N), dim3(64), 0, c->G, c->B, slot, row, c3);
-    coll2phys_dev(c, c3, P.S[row * 3], 3);
-  }
+  launch(c, "nn_grad", k_nn_grad, dim3((c->H + 63) / 64, c->N, 3), dim3(64), 0, c->G, c->B, slot, c->nnC);
+  coll2phys_dev(c, c->nnC, P.S[0], 9);   // A(row, j), S[0..8] one after another
 }
 void visc_derivatives(opf_ctx* c, int slot, const NnPhys& P) {
-  double2* c3 = c->nnC;
-  double2* nuc = c->nnC + 3 * c->G.coll;
+  double2* c6 = c->nnC;
+  double2* nuc = c->nnC + 6 * c->G.coll;
   const dim3 gh((c->H + 63) / 64, c->N), b64(64);
   phys2coll_dev(c, P.nu, nuc, 1);
-  launch(c, "nn_gradp", k_nn_gradp, gh, b64, 0, c->G, c->B, slot, (const double2*)nuc, c3);
-  coll2phys_dev(c, c3, P.g[0], 3);
-  launch(c, "nn_curlcurl", k_nn_curlcurl, gh, b64, 0, c->G, c->B, slot, c3);
-  coll2phys_dev(c, c3, P.q[0], 3);
+  launch(c, "nn_gradp", k_nn_gradp, gh, b64, 0, c->G, c->B, slot, (const double2*)nuc, c6);
+  launch(c, "nn_curlcurl", k_nn_curlcurl, gh, b64, 0, c->G, c->B, slot, c6 + 3 * c->G.coll);
+  coll2phys_dev(c, c6, P.g[0], 6);   // g[0..2] and q[0..2] one after another
 }
 void visc_add(opf_ctx* c, int slot, const NnPhys& P) {
   double2* c3 = c->nnC;
   phys2coll_dev(c, P.q[0], c3, 3);
-  for (int j = 0; j < 3; ++j)
-    launch(c, "nn_addN", k_nn_addN, dim3((c->H + 63) / 64, c->N, 1), dim3(64), 0, c->G, c->B, slot, j,
-           (const double2*)(c3 + (size_t)j * c->G.coll));
+  launch(c, "nn_addN", k_nn_addN, dim3((c->H + 63) / 64, c->N, 3), dim3(64), 0, c->G, c->B, slot, (const double2*)c3);
 }
 
 // util(2) of the non-Newtonian plugin for one slot: get_nu and

@@ -133,12 +133,12 @@ struct NnPhys {
   double* g[3];
   double* q[3];
 };
-__global__ void k_nn_grad(Geo G, Bufs B, int slot, int row, double2* __restrict__ out);
+__global__ void k_nn_grad(Geo G, Bufs B, int slot, double2* __restrict__ out);
 __global__ void k_nn_gradp(Geo G, Bufs B, int slot, const double2* __restrict__ p, double2* __restrict__ out);
 __global__ void k_nn_curlcurl(Geo G, Bufs B, int slot, double2* __restrict__ out);
 __global__ void k_nn_visc(NnPhys P, size_t np, double lam, double d1, double d2, double a);
 __global__ void k_nn_force(NnPhys P, size_t np, double nu_r, double Re);
-__global__ void k_nn_addN(Geo G, Bufs B, int slot, int comp, const double2* __restrict__ src);
+__global__ void k_nn_addN(Geo G, Bufs B, int slot, const double2* __restrict__ src);
 __global__ void k_les_prep(Geo G, Bufs B, int slot, int model, double Cs, double Aplus, double* D,
                            unsigned long long* numax);
 __global__ void k_les_visc(NnPhys P, size_t np, int N, int ZT, int model, double Cs, double dz, const double* D,

@@ -1046,12 +1046,17 @@ __global__ void k_symmetry(Geo G, Bufs B, int slot0, int gated) {
 // physical pieces per grid point; the transforms between them are the
 // single-field transforms of tra_coll2phys / tra_phys2coll.
 // ---------------------------------------------------------------------------
-// One row of the gradient tensor A of the slot's current iterate (get_nu,
+// The gradient tensor A of the slot's current iterate (get_nu,
 // nonnewtonian.f90:108-147): row 0 the radial derivatives by
 // var_coll_meshmult with dr(1), row 1 the theta terms (1/r)(d/dtheta u -
-// e_theta x u), row 2 the z derivatives; out holds the three components.
-// One thread per (h, n): grid x = harmonics / 64, y = N.
-__global__ void k_nn_grad(Geo G, Bufs B, int slot, int row, double2* __restrict__ out) {
+// e_theta x u), row 2 the z derivatives; out holds the three components of each
+// row.  One thread per (h, n): grid x = harmonics / 64, y = N, z = row.  The nine
+// fields then pass through each transform in one launch, which for few fields
+// takes little more than the launch itself ((48,48,24), z and theta: 6.1 and 7.0
+// us for three fields, 8.5 and 11.2 for six and nine).
+__global__ void k_nn_grad(Geo G, Bufs B, int slot, double2* __restrict__ out) {
+  const int row = blockIdx.z;
+  out += (size_t)row * 3 * G.coll;
   const int h = blockIdx.x * blockDim.x + threadIdx.x;
   const int n = blockIdx.y;
   if (h >= G.H) return;
@@ -1147,8 +1152,8 @@ __global__ void k_nn_curlcurl(Geo G, Bufs B, int slot, double2* __restrict__ out
   out[2 * G.coll + o] = qz;
 }
 
-// get_nu's algebra per grid point (nonnewtonian.f90:148-172): S = (A + A^T)/2
-// written back over A, strain rate sr = (2 S:S)^(1/2) and the Carreau-Yasuda
+// get_nu's algebra per grid point (nonnewtonian.f90:148-172): the upper half of
+// S = (A + A^T)/2 written back over A's, strain rate sr = (2 S:S)^(1/2) and the Carreau-Yasuda
 // viscosity nu = d1 + (1 - d1)(1 + (lam sr)^a)^d2.
 __global__ void k_nn_visc(NnPhys P, size_t np, double lam, double d1, double d2, double a) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1157,9 +1162,9 @@ __global__ void k_nn_visc(NnPhys P, size_t np, double lam, double d1, double d2,
   const double s12 = 0.5 * (S[1][i] + S[3][i]);
   const double s13 = 0.5 * (S[2][i] + S[6][i]);
   const double s23 = 0.5 * (S[5][i] + S[7][i]);
-  S[1][i] = s12; S[3][i] = s12;
-  S[2][i] = s13; S[6][i] = s13;
-  S[5][i] = s23; S[7][i] = s23;
+  S[1][i] = s12;
+  S[2][i] = s13;
+  S[5][i] = s23;
   const double s11 = S[0][i], s22 = S[4][i], s33 = S[8][i];
   double sr = s11 * s11 + s22 * s22 + s33 * s33 + 2.0 * (s12 * s12 + s13 * s13 + s23 * s23);
   sr = sqrt(2.0 * sr);
@@ -1172,9 +1177,12 @@ __global__ void k_nn_force(NnPhys P, size_t np, double nu_r, double Re) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
   const double nu_ = P.nu[i] - nu_r;
+  const double g[3] = {P.g[0][i], P.g[1][i], P.g[2][i]};
+  const double s01 = P.S[1][i], s02 = P.S[2][i], s12 = P.S[5][i];
+  const double S[9] = {P.S[0][i], s01, s02, s01, P.S[4][i], s12, s02, s12, P.S[8][i]};
   for (int c = 0; c < 3; ++c) {
     double q = nu_ * (-P.q[c][i]);
-    for (int j = 0; j < 3; ++j) q = q + P.g[j][i] * P.S[j * 3 + c][i] * 2.0;
+    for (int j = 0; j < 3; ++j) q = q + g[j] * S[j * 3 + c] * 2.0;
     if (c == 2) q = q + (nu_r - 1.0) * (-4.0);
     P.q[c][i] = q / Re;
   }
@@ -1310,9 +1318,11 @@ __global__ void k_les_force(NnPhys P, size_t np, Bufs B, int slot) {
   }
 }
 
-// N += N': one component added to the raw nonlinear terms of the slot's
-// current evaluation.
-__global__ void k_nn_addN(Geo G, Bufs B, int slot, int comp, const double2* __restrict__ src) {
+// N += N': added to the raw nonlinear terms of the slot's current evaluation.
+// grid: x = H/64, y = N, z = component.
+__global__ void k_nn_addN(Geo G, Bufs B, int slot, const double2* __restrict__ src) {
+  const int comp = blockIdx.z;
+  src += (size_t)comp * G.coll;
   const int h = blockIdx.x * blockDim.x + threadIdx.x;
   const int n = blockIdx.y;
   if (h >= G.H || n >= G.N) return;
