@@ -42,16 +42,22 @@ WORKLOADS = {
 }
 
 
+def factor_bytes(N, K, M):
+    """What a step launch reads of the solves: the 4 x 4 block inverses of four
+    matrices and the six influence vectors per (|k|, m) pair, and a 4 x 4 inverse
+    per harmonic."""
+    H = (2 * K - 1) * M - (K - 1)
+    return K * M * (4 * 128 * ((N + 3) // 4) + 48 * N) + 128 * H
+
+
 def alg_bytes(N, K, M):
     """Algorithmic (compulsory) bytes per launch of each kernel: every array
     the kernel must read or write once.  C = one complex coll field."""
     H = (2 * K - 1) * M - (K - 1)
-    P = K * M
     Z = 3 * K
     C = 16 * N * H
     Y = 16 * N * Z * M                       # one field of the z-transformed intermediates
-    # LU factors and pivots once per (|k|, m) pair, influence vectors and 4x4 inverses
-    F = 4 * P * (8 * 13 * N + 4 * N) + H * (48 * N + 128)
+    F = factor_bytes(N, K, M)
     return dict(C=C, F=F,
                 zfwd=6 * C + 6 * Y, theta=9 * Y, zbwd=3 * Y + 3 * C,
                 # the whole-plane evaluation of small grids: u, curl u in, N out
@@ -63,10 +69,10 @@ def alg_bytes(N, K, M):
 
 def alg_bytes_per_step(N, K, M, ncorr):
     """B_alg = (21 + 27 n_corr) C + (1 + n_corr) F, the two-phase compulsory
-    traffic model (factors once per +-k pair, influence vectors per harmonic)."""
+    traffic model (factors and influence vectors once per +-k pair)."""
     H = (2 * K - 1) * M - (K - 1)
     C = 16 * N * H
-    F = 4 * K * M * (8 * 13 * N + 4 * N) + H * (48 * N + 128)
+    F = factor_bytes(N, K, M)
     return (21 + 27 * ncorr) * C + (1 + ncorr) * F
 
 

@@ -4,9 +4,9 @@
 // device arrays of `capacity` slots.  The time loop of main.f90:18-46 runs as
 // a sequence of "iterations", each one nonlinear evaluation plus one
 // predictor or corrector (per slot, as the slot's control block says):
-//   k_zfwd -> k_theta -> k_zbwd -> k_step -> k_control
+//   k_zfwd -> k_theta -> k_zbwd -> k_step
 // (k_step ends with the curl for the next evaluation).  The corrector test
-// (tim_check_cgce) runs in k_control on the device, so the host only enqueues
+// (tim_check_cgce) runs in k_step's last workgroup on the device, so the host only enqueues
 // iterations and checks progress between chunks.
 #include <hip/hip_runtime.h>
 #include <dlfcn.h>
@@ -1110,7 +1110,7 @@ void run_plan(opf_ctx* c, const std::vector<int>& slots, const std::vector<int>&
       std::snprintf(msg, sizeof msg, "tim_check_cgce failure %d in slot %d at step %d", ctl[s].status, s, ctl[s].step);
       throw OpfError(OPF_ERR_CORRECTOR, msg);
     }
-  if (remaining > 0) {   // cannot happen while k_control keeps its corrector limit; never leave slots running
+  if (remaining > 0) {   // cannot happen while control_decide keeps its corrector limit; never leave slots running
     for (int s : p.slots) ctl[s].active = 0;
     write_ctl(c, ctl);
     throw OpfError(OPF_ERR_CORRECTOR, "time loop: steps left after the iteration budget");
