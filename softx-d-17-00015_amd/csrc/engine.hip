@@ -1000,34 +1000,11 @@ void run_enqueue(opf_ctx* c, const RunPlan& p, long iterations) {
 
 hipStream_t ctx_stream(opf_ctx* c) { return c->stream; }
 
-size_t state_rows(const opf_ctx* c) { return 3 * c->G.coll; }
+// slot's part of the backward intermediates: the planes of an idle slot pass
+// through it
+static double* slot_planes(opf_ctx* c, int slot) { return (double*)(c->B.Yb + (size_t)slot * c->N * c->G.ZQ * 3 * c->M); }
 
-void coll_to_rows(const opf_ctx* c, const double* const planes[6], double2* rows) {
-  for (int comp = 0; comp < 3; ++comp) {
-    double2* d = rows + (size_t)comp * c->G.coll;
-    const double* re = planes[2 * comp];
-    const double* im = planes[2 * comp + 1];
-    for (int n = 0; n < c->N; ++n) {
-      double2* row = d + (size_t)n * c->Hp;
-      for (int hh = 0; hh < c->H; ++hh) row[hh] = make_double2(re[(size_t)hh * c->N + n], im[(size_t)hh * c->N + n]);
-      for (int hh = c->H; hh < c->Hp; ++hh) row[hh] = make_double2(0.0, 0.0);
-    }
-  }
-}
-
-void rows_to_coll(const opf_ctx* c, const double2* rows, double* const planes[6]) {
-  for (int comp = 0; comp < 3; ++comp) {
-    const double2* d = rows + (size_t)comp * c->G.coll;
-    for (int hh = 0; hh < c->H; ++hh)
-      for (int n = 0; n < c->N; ++n) {
-        const double2 v = d[(size_t)n * c->Hp + hh];
-        planes[2 * comp][(size_t)hh * c->N + n] = v.x;
-        planes[2 * comp + 1][(size_t)hh * c->N + n] = v.y;
-      }
-  }
-}
-
-void admit_async(opf_ctx* c, int slot, double Re, double alpha, double dt, int ucur, const double2* rows,
+void admit_async(opf_ctx* c, int slot, double Re, double alpha, double dt, int ucur, const double* planes,
                  int nsteps, int corr_fixed) {
   check_slot(c, slot);
   if (!(dt > 0.0) || !(Re > 0.0) || alpha == 0.0) throw OpfError(OPF_ERR_ARG, "Re, dt must be > 0 and alpha != 0");
@@ -1047,8 +1024,10 @@ void admit_async(opf_ctx* c, int slot, double Re, double alpha, double dt, int u
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(c->B.prm + slot, &p, sizeof p, hipMemcpyHostToDevice, c->stream));
   launch_matrices(c, slot, 1, 0);
-  HIPCHK(hipMemcpyAsync(c->B.U[ucur] + (size_t)slot * 3 * c->G.coll, rows, sizeof(double2) * 3 * c->G.coll,
-                        hipMemcpyHostToDevice, c->stream));
+  double* dev = slot_planes(c, slot);
+  HIPCHK(hipMemcpyAsync(dev, planes, sizeof(double) * 6 * c->N * c->H, hipMemcpyHostToDevice, c->stream));
+  launch(c, "to_rows", k_planes_to_rows, grid_planes(c, 3), dim3(256), 0, c->G, (const double*)dev,
+         c->B.U[ucur] + (size_t)slot * 3 * c->G.coll);
   launch(c, "imposesym", k_imposesym, dim3((c->N + 63) / 64, 1, 1), dim3(64), 0, c->G, c->B, slot);
   hipLaunchKernelGGL(k_admit, dim3(1), dim3(1), 0, c->stream, c->B, slot, 1, nsteps, corr_fixed);
   HIPCHK(hipGetLastError());
@@ -1063,10 +1042,12 @@ void ctl_snapshot_async(opf_ctx* c, SlotCtl* out) {
   HIPCHK(hipMemcpyAsync(out, c->B.ctl, sizeof(SlotCtl) * c->cap, hipMemcpyDeviceToHost, c->stream));
 }
 
-void fetch_async(opf_ctx* c, int slot, int ucur, double2* rows) {
+void fetch_async(opf_ctx* c, int slot, int ucur, double* planes) {
   check_slot(c, slot);
-  HIPCHK(hipMemcpyAsync(rows, c->B.U[ucur] + (size_t)slot * 3 * c->G.coll, sizeof(double2) * 3 * c->G.coll,
-                        hipMemcpyDeviceToHost, c->stream));
+  double* dev = slot_planes(c, slot);
+  launch(c, "to_planes", k_rows_to_planes, grid_planes(c, 3), dim3(256), 0, c->G,
+         (const double2*)(c->B.U[ucur] + (size_t)slot * 3 * c->G.coll), dev);
+  HIPCHK(hipMemcpyAsync(planes, dev, sizeof(double) * 6 * c->N * c->H, hipMemcpyDeviceToHost, c->stream));
 }
 
 int run_remaining(opf_ctx* c, RunPlan& p) {

@@ -80,9 +80,9 @@ struct Block {
   std::vector<int> ucur;          // velocity buffer role of an idle slot
   std::vector<long> admit_seq;    // snapshots taken after its admission have seq >= this
   std::vector<hipEvent_t> fetched;
-  double2* in = nullptr;          // pinned state rows per slot (admission)
-  double2* out = nullptr;         // pinned state rows per slot (retirement)
-  size_t rows = 0;                // double2 per slot state
+  double* in = nullptr;           // pinned state planes per slot (admission)
+  double* out = nullptr;          // pinned state planes per slot (retirement)
+  size_t state = 0;               // doubles per slot state
   std::vector<Snapshot> ring;
   int ring_head = 0;              // oldest pending snapshot
   long seq = 0;                   // iterations enqueued
@@ -130,11 +130,6 @@ struct opf_server {
     return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   }
 
-  static void planes(const Class& c, double* base, double* p[6]) {
-    const size_t n = (size_t)c.N * c.H;
-    for (int i = 0; i < 6; ++i) p[i] = base + i * n;
-  }
-
   // ---- blocks ---------------------------------------------------------------
   Block* new_block(Class& c) {
     auto b = std::make_unique<Block>();
@@ -147,9 +142,9 @@ struct opf_server {
     b->ucur.assign(b->cap, 0);        // the role opf_ctx_create gives every slot
     b->admit_seq.assign(b->cap, 0);
     b->fetched.assign(b->cap, nullptr);
-    b->rows = opf::state_rows(b->ctx);
-    hipchk(hipHostMalloc((void**)&b->in, sizeof(double2) * b->rows * b->cap, hipHostMallocDefault), "pinned in");
-    hipchk(hipHostMalloc((void**)&b->out, sizeof(double2) * b->rows * b->cap, hipHostMallocDefault), "pinned out");
+    b->state = (size_t)6 * c.N * c.H;
+    hipchk(hipHostMalloc((void**)&b->in, sizeof(double) * b->state * b->cap, hipHostMallocDefault), "pinned in");
+    hipchk(hipHostMalloc((void**)&b->out, sizeof(double) * b->state * b->cap, hipHostMallocDefault), "pinned out");
     b->ring.resize(depth + 1);
     for (auto& s : b->ring) {
       hipchk(hipHostMalloc((void**)&s.host, sizeof(opf::SlotCtl) * b->cap, hipHostMallocDefault), "pinned ctl");
@@ -234,12 +229,10 @@ struct opf_server {
           c.queue.pop_front();
           r->t_admit = now();
         }
-        double* p[6];
-        planes(c, r->state.data(), p);
-        double2* rows = blk->in + (size_t)slot * blk->rows;
-        opf::coll_to_rows(blk->ctx, p, rows);
+        double* in = blk->in + (size_t)slot * blk->state;
+        std::memcpy(in, r->state.data(), sizeof(double) * blk->state);
         try {
-          opf::admit_async(blk->ctx, slot, r->Re, r->alpha, r->dt, blk->ucur[slot], rows, r->nsteps,
+          opf::admit_async(blk->ctx, slot, r->Re, r->alpha, r->dt, blk->ucur[slot], in, r->nsteps,
                            r->corr_fixed);
         } catch (const std::exception& e) {
           finish(r, OPF_ERR_ARG);
@@ -279,7 +272,7 @@ struct opf_server {
         } else if (!k.active && k.step >= k.target_steps) {
           b.ucur[s] = k.ucur;
           b.req[s]->t = k.t;
-          opf::fetch_async(b.ctx, s, k.ucur, b.out + (size_t)s * b.rows);
+          opf::fetch_async(b.ctx, s, k.ucur, b.out + (size_t)s * b.state);
           hipchk(hipEventRecord(b.fetched[s], opf::ctx_stream(b.ctx)), "fetch event");
           b.phase[s] = FETCHING;
         }
@@ -291,9 +284,7 @@ struct opf_server {
       if (q == hipErrorNotReady) continue;
       hipchk(q, "fetch event");
       ReqPtr r = b.req[s];
-      double* p[6];
-      planes(c, r->state.data(), p);
-      opf::rows_to_coll(b.ctx, b.out + (size_t)s * b.rows, p);
+      std::memcpy(r->state.data(), b.out + (size_t)s * b.state, sizeof(double) * b.state);
       b.req[s] = nullptr;
       b.phase[s] = FREE;
       --b.running;
