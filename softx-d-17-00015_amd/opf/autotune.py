@@ -29,6 +29,8 @@ WORKLOADS = [
     (48, 48, 24, 1, 3000.0, 1.25, 0.01, 100),
     (64, 64, 48, 1, 5300.0, 0.5, 0.005, 100),
     (96, 256, 128, 1, 5300.0, 0.4, 0.0025, 10),
+    (32, 24, 12, 8, 2400.0, 1.25, 0.01, 100),     # a server's blocks
+    (48, 48, 24, 4, 3000.0, 1.25, 0.01, 50),
     (32, 24, 12, 64, 2400.0, 1.25, 0.01, 40),
     (48, 48, 24, 32, 3000.0, 1.25, 0.01, 20),
     (64, 64, 48, 16, 5300.0, 0.5, 0.005, 10),
