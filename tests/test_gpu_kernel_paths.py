@@ -109,3 +109,54 @@ def test_step_with_a_replaced_factor_set(opf):
     ctx.vel_matrices(0, dt)
     after = ctx.lumesh_get(0, opf.LDZ)
     assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
+
+
+# theta lines of three passes whose sequence is not that of the z columns of
+# their length, with requests of more than 64 KiB of LDS (M = 192)
+@pytest.mark.parametrize("M", [128, 144, 162, 192, 216])
+def test_nonlinear_long_theta_sequences(opf, M):
+    _nonlinear_matches(opf, 10, 3, M)
+
+
+# narrow and odd tile requests: a last tile of one line or one column, an odd
+# number of z lines
+@pytest.mark.parametrize("K,M,tm,tz", [(9, 16, 5, 2), (27, 6, 5, 0), (16, 9, 1, 0), (12, 8, 7, 2)])
+def test_nonlinear_tiles(opf, K, M, tm, tz):
+    from opf import ic as icgen
+    res = []
+    for shape in ((0, 0), (tm, tz)):
+        ctx = opf.Context(10, K, M, tm=shape[0], tz=shape[1])
+        ctx.setup(0, 3000.0, 1.25, 0.01)
+        me = ctx.mesh()
+        ctx.put_state(0, *icgen.seeded_perturbation(me["r"], me["intrdr"], K, M, 1.25, 7, 1e-2))
+        ctx.transform(0)
+        ctx.nonlinear(0)
+        res.append(ctx.get_nonlinear(0))
+        ctx.close()
+    for c in range(3):
+        assert np.array_equal(res[0][c], res[1][c]), c
+
+
+# The plugins' batched transforms at odd numbers of z lines, at two and
+# three passes: one step with the
+# variable viscosity against the oracle, as close as the plugin's own test asks.
+@pytest.mark.parametrize("K,M", [(9, 9), (3, 4), (27, 8), (16, 32), (32, 3), (54, 6)])
+def test_viscosity_transform_lengths(opf, K, M):
+    from opf import ic as icgen
+    Re, alpha, dt = 2400.0, 1.25, 0.01
+    prm = dict(rho=1000.0, radius=0.01, mu_0=0.056, mu_inf=0.0056, lam_CY=3e-3, n_CY=0.6, a_CY=2.0)
+    ctx = opf.Context(10, K, M)
+    ctx.nonnewtonian(0, **prm)
+    ctx.setup(0, Re, alpha, dt)
+    me = ctx.mesh()
+    u = icgen.seeded_perturbation(me["r"], me["intrdr"], K, M, alpha, 3, 1e-2)
+    ctx.put_state(0, *u)
+    ctx.run(1)
+    got = ctx.get_state(0)
+    oc = O.Ctx(10, K, M, Re=Re, alpha=alpha, dt=dt)
+    oc.nonnewtonian = prm
+    oc.set_state(*u)
+    oc.run(1, ncorr_fixed=1)
+    for c, ref in enumerate((oc.ur, oc.ut, oc.uz)):
+        assert rel_err(got[c], ref) <= 1e-12, c
+    ctx.close()
