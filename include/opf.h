@@ -217,8 +217,9 @@ int opf_run(opf_ctx* ctx, int nsteps, int corr_fixed, int diag_every);
 int opf_run_slots(opf_ctx* ctx, const int* slots, int nslots, int nsteps, int corr_fixed,
                   int diag_every);
 
-/* tim_step, tim_t, failure status (0 ok), correctors of the last step,
- * tim_dterr of the last corrector, vel_Pr0. */
+/* tim_step, tim_t, failure status (0 ok; 1 dt -> 0, 2 too many its, 3 increasing
+ * error, 4 tim_dterr is a NaN), correctors of the last step, tim_dterr of the
+ * last corrector, vel_Pr0. */
 int opf_slot_status(opf_ctx* ctx, int slot, int* step, double* t, int* status, int* last_ncorr,
                     double* last_dterr, double* Pr0);
 /* Diagnostics records, oldest first, 10 doubles each:

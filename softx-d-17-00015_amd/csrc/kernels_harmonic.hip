@@ -86,6 +86,14 @@ __device__ __forceinline__ void eval_bc5(const double2* up, const double2* um, d
   BIm[3] = ((urIm * d + drIm) + (d * m_) * utRe) + a_ * uzN.x;
 }
 
+// max |du|^2 of a corrector as a bit pattern: the values are sums of squares, so
+// their patterns order as they do, and a NaN (its sign cleared) sorts above
+// them all, where fmax would drop it and count the corrector as converged
+__device__ __forceinline__ unsigned long long du_bits(double d, bool nan) {
+  return nan ? 0x7ff8000000000000ull : (unsigned long long)__double_as_longlong(d);
+}
+__device__ __forceinline__ unsigned long long du_max(unsigned long long a, unsigned long long b) { return a > b ? a : b; }
+
 __device__ __forceinline__ double pr0_of(const double2* uz0, size_t hs, int N, const double* dr1c) {
   // vel_Pr0 = dot_product(uz%Re(N-KL:N,0), dr1(:,1)) / (-2)  (velocity.f90:356-357)
   double s = 0.0;
@@ -98,7 +106,7 @@ __device__ __forceinline__ double pr0_of(const double2* uz0, size_t hs, int N, c
 // tim_check_cgce (timestep.f90:214-253), buffer roles, time and step counters
 // of one slot: one thread, on the slot's control block, after every
 // workgroup's part of the step.  Pr0 and Pr0_hpf are another workgroup's to
-// write.  dt2: max |du|^2 of a corrector; E, Ek0, Em0: var_coll_norm of a
+// write.  dt2: max |du|^2 of a corrector, a NaN if there was one; E, Ek0, Em0: var_coll_norm of a
 // diagnostics step.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void control_decide(SlotCtl* c, const SlotParams& prm, DiagRec* recs, bool diag_now,
@@ -666,19 +674,24 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
       }
     }
   }
-  double dmax = 0.0;
+  unsigned long long* WD = (unsigned long long*)(RED + 1);   // the waves' maxima
   if (corr) {
+    double dmax = 0.0;
+    bool nan = false;
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
       if (n0 + q * DN >= N || !S.valid) continue;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         const double dx = old[q][c].x - nu[q][c].x, dy = old[q][c].y - nu[q][c].y;
-        dmax = fmax(dmax, fma(dx, dx, dy * dy));
+        const double d = fma(dx, dx, dy * dy);
+        nan = nan || d != d;
+        dmax = fmax(dmax, d);
       }
     }
     for (int off = 32; off >= 1; off >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, off));
-    if ((tid & 63) == 0) RED[1 + wave] = dmax;
+    nan = __any(nan);
+    if ((tid & 63) == 0) WD[wave] = du_bits(dmax, nan);
   }
   __syncthreads();
 
@@ -694,10 +707,10 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   const int sub = grp % nsub;
   unsigned long long prev = 0ull, cnt = 0ull;
   if (tid == 0 && corr) {
+    unsigned long long wd = WD[0];
 #pragma unroll
-    for (int w = 1; w < THR / 64; ++w) dmax = fmax(dmax, RED[1 + w]);
-    prev = __hip_atomic_exchange(arr + 16 * ARRIVE_WORDS + grp, (unsigned long long)__double_as_longlong(dmax),
-                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int w = 1; w < THR / 64; ++w) wd = du_max(wd, WD[w]);
+    prev = __hip_atomic_exchange(arr + 16 * ARRIVE_WORDS + grp, wd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 #pragma unroll
   for (int q = 0; q < IT; ++q) {
@@ -750,8 +763,9 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   if (RED[0] == 0.0) return;
   DiagRec* recs = B.diag + (size_t)slot * ct.diag_cap;
   double* ws = (double*)V;   // [wave][3]
+  double dt2 = 0.0;
   if (corr) {
-    dmax = 0.0;
+    unsigned long long wd = 0ull;
     for (int i = tid; i < ST.ngroups; i += 4 * THR) {
       unsigned long long w4[4];
 #pragma unroll
@@ -759,15 +773,17 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
         w4[u] = __hip_atomic_load(arr + 16 * ARRIVE_WORDS + min(i + u * THR, ST.ngroups - 1), __ATOMIC_RELAXED,
                                   __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) dmax = fmax(dmax, __longlong_as_double((long long)w4[u]));
+      for (int u = 0; u < 4; ++u) wd = du_max(wd, w4[u]);
     }
-    for (int off = 32; off >= 1; off >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, off));
-    if ((tid & 63) == 0) ws[wave] = dmax;
+    for (int off = 32; off >= 1; off >>= 1) wd = du_max(wd, __shfl_xor(wd, off));
+    unsigned long long* wsd = (unsigned long long*)V;
+    if ((tid & 63) == 0) wsd[wave] = wd;
     __syncthreads();
-    for (int w = 1; w < THR / 64; ++w) dmax = fmax(dmax, ws[w]);
+    for (int w = 0; w < THR / 64; ++w) wd = du_max(wd, wsd[w]);
+    dt2 = __longlong_as_double((long long)wd);
   }
   if (!want_diag) {
-    if (tid == 0) control_decide(ctl, prm, recs, false, dmax, 0.0, 0.0, 0.0);
+    if (tid == 0) control_decide(ctl, prm, recs, false, dt2, 0.0, 0.0, 0.0);
     return;
   }
   // var_coll_norm (variables.f90:727-749) from the harmonics' partials
