@@ -124,6 +124,7 @@ struct opf_ctx {
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   double* dterrHost = nullptr;   // pinned: tim_dterr of the last host-driven call (first use)
   SlotParams* prmHost = nullptr; // pinned parameters of asynchronous admissions (first use)
+  int* luSingular = nullptr;     // a zero pivot of tim_lumesh_init's factors (first use)
   std::vector<int> lu_bc;        // BC of each factor set [slot][4] (tim_lumesh_invert's (0,0) rule)
   int device = 0;                // HIP device of the context
   // launch modes of the time loop: one iteration captured as a HIP graph
@@ -391,11 +392,13 @@ void launch_iteration(opf_ctx* c, int s0, int ns) {
 
 // The LAPACK-form factors of one factor set, for tim_lumesh_get and
 // tim_lumesh_invert: built from the matrix the set holds when they are asked
-// for (the time step does not read them).  Buffers on first use.
+// for (the time step does not read them).  Buffers on first use.  A zero pivot
+// is left in luSingular, which only tim_lumesh_init looks at.
 void lapack_factors(opf_ctx* c, int slot, int which) {
   if (!c->B.LU) c->B.LU = c->alloc<double>((size_t)c->cap * 4 * c->N * LUS * c->P);
   if (!c->B.PV) c->B.PV = c->alloc<unsigned char>((size_t)c->cap * 4 * c->N * c->P);
-  launch(c, "lapack_factor", k_lu_factor, dim3((c->P + 15) / 16), dim3(64), 0, c->G, c->B, slot, which);
+  if (!c->luSingular) c->luSingular = c->alloc<int>(1);
+  launch(c, "lapack_factor", k_lu_factor, dim3((c->P + 15) / 16), dim3(64), 0, c->G, c->B, slot, which, c->luSingular);
 }
 
 // n doubles per plane between the host's planes (null: skipped or zeros) and
@@ -1873,10 +1876,13 @@ extern "C" int opf_tim_lumesh_init(opf_ctx* c, int slot, int which, int PM, int 
     write_ctl(c, ctl);
     launch(c, "factor", k_block_factor, dim3((c->P + 31) / 32), dim3(64), 0, c->G, c->B, slot,
            LuSpec{which, PM, BC, c1, c2});
+    int singular = 0;
+    if (c->luSingular) HIPCHK(hipMemcpy(c->luSingular, &singular, sizeof(int), hipMemcpyHostToDevice));
     lapack_factors(c, slot, which);   // DGBTF2's own verdict on a singular matrix
     ctl = read_ctl(c);
     c->lu_bc[(size_t)slot * 4 + which] = BC;
-    if (ctl[slot].status != 0) {
+    HIPCHK(hipMemcpy(&singular, c->luSingular, sizeof(int), hipMemcpyDeviceToHost));
+    if (ctl[slot].status != 0 || singular) {
       ctl[slot].status = 0;
       write_ctl(c, ctl);
       throw OpfError(OPF_ERR_SINGULAR, "tim_lumesh_init");

@@ -115,7 +115,7 @@ __host__ __device__ constexpr int tile_m(int Z) { return FFT_TILE / Z; }
 __host__ __device__ constexpr int padded_len(int L) { return (L + (L - 1) / 16 + 1) | 1; }
 
 __global__ void k_block_factor(Geo G, Bufs B, int slot, LuSpec A);
-__global__ void k_lu_factor(Geo G, Bufs B, int slot, int mat);
+__global__ void k_lu_factor(Geo G, Bufs B, int slot, int mat, int* singular);
 using MatricesKern = void (*)(Geo, Bufs, int, int);
 MatricesKern matrices_kernel(int N);
 inline size_t matrices_smem(int N) { return (size_t)(10 * (N + 8) + 40 * (N + 4) + 48 * (KL + 1)) * sizeof(double); }

@@ -428,10 +428,11 @@ __global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot, Lu
 // ---------------------------------------------------------------------------
 // tim_lumesh_init (timestep.f90:67-96) + DGBTF2 of one matrix per pair in
 // LAPACK band layout, for tim_lumesh_get / tim_lumesh_invert (the time step
-// solves with block_factor's inverses).  Four lanes per system.
+// solves with block_factor's inverses).  Four lanes per system.  *singular is
+// set where a pivot is zero.
 // grid: x = pairs/16; 64 threads = 16 systems x 4 lanes.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot, int mat) {
+__global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot, int mat, int* singular) {
   constexpr int LPS = 4;              // lanes per system
   constexpr int SPW = 64 / LPS;       // systems per workgroup
   const int q = threadIdx.x % LPS, sl = threadIdx.x / LPS;
@@ -557,7 +558,7 @@ __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot, int m
     }
     if (!raw && piv == 0.0) {
       if (q == 0) pv[j] = (unsigned char)jp;
-      if (q == 0) atomicMax(&B.ctl[slot].status, 100 + mat);  // singular factor
+      if (q == 0) *singular = 1;
       return;
     }
     const int lim = j + KL + jp < N - 1 ? j + KL + jp : N - 1;
