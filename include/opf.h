@@ -76,7 +76,7 @@ int opf_ctx_dims(const opf_ctx* ctx, int* N, int* K, int* M, int* Mp, int* H, in
 /* Device bytes a context of this shape holds after opf_ctx_create
  * (admission control).  Allocated later, on first use: the shift tables
  * ((2K + M) * 16 bytes per slot), and for opf_tim_lumesh_get /
- * _invert / _init the LAPACK-form factors (4*K*M*129*N bytes per slot), and
+ * _invert / _init the LAPACK-form factors of the set (K*M*(129*N + 1) bytes), and
  * for opf_slot_nonnewtonian / opf_slot_les 16 physical fields of N*3K*3M doubles, 4 spectral fields and
  * 3 fields of N*3K*M complex values per context, and 4N + 1 words per slot. */
 size_t opf_ctx_bytes_needed(int N, int K, int M, int capacity);

@@ -124,6 +124,7 @@ struct opf_ctx {
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   double* dterrHost = nullptr;   // pinned: tim_dterr of the last host-driven call (first use)
   SlotParams* prmHost = nullptr; // pinned parameters of asynchronous admissions (first use)
+  std::vector<LuFactors> lu;     // LAPACK-form factors [slot][4] (first use)
   int* luSingular = nullptr;     // a zero pivot of tim_lumesh_init's factors (first use)
   std::vector<int> lu_bc;        // BC of each factor set [slot][4] (tim_lumesh_invert's (0,0) rule)
   int device = 0;                // HIP device of the context
@@ -392,13 +393,20 @@ void launch_iteration(opf_ctx* c, int s0, int ns) {
 
 // The LAPACK-form factors of one factor set, for tim_lumesh_get and
 // tim_lumesh_invert: built from the matrix the set holds when they are asked
-// for (the time step does not read them).  Buffers on first use.  A zero pivot
-// is left in luSingular, which only tim_lumesh_init looks at.
-void lapack_factors(opf_ctx* c, int slot, int which) {
-  if (!c->B.LU) c->B.LU = c->alloc<double>((size_t)c->cap * 4 * c->N * LUS * c->P);
-  if (!c->B.PV) c->B.PV = c->alloc<unsigned char>((size_t)c->cap * 4 * c->N * c->P);
+// for (the time step does not read them), where they are not there yet.  Buffers
+// per set on first use.  A zero pivot is left in luSingular, which only
+// tim_lumesh_init looks at.
+const LuFactors& lapack_factors(opf_ctx* c, int slot, int which) {
+  LuFactors& L = c->lu[(size_t)slot * 4 + which];
+  const size_t cols = (size_t)c->P * c->N, groups = (c->P + 15) / 16;
+  if (!L.F) {   // one buffer: the factors, the versions, the pivots
+    L.F = c->alloc<double>(cols * LUS + (groups + 1) / 2 + (cols + 7) / 8);
+    L.built = (unsigned*)(L.F + cols * LUS);
+    L.pv = (unsigned char*)(L.F + cols * LUS + (groups + 1) / 2);
+  }
   if (!c->luSingular) c->luSingular = c->alloc<int>(1);
-  launch(c, "lapack_factor", k_lu_factor, dim3((c->P + 15) / 16), dim3(64), 0, c->G, c->B, slot, which, c->luSingular);
+  launch(c, "lapack_factor", k_lu_factor, dim3((unsigned)groups), dim3(64), 0, c->G, c->B, L, slot, which, c->luSingular);
+  return L;
 }
 
 // n doubles per plane between the host's planes (null: skipped or zeros) and
@@ -732,6 +740,7 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   B.om = c->alloc<double2>(c3);
   B.SE = c->alloc<double>((size_t)cap * 4 * s.P * blk_count(N) * 16);
   B.spec = c->alloc<LuSpec>((size_t)cap * 4);
+  B.ver = c->alloc<unsigned>((size_t)cap * 4);
   B.Uinf = c->alloc<double>((size_t)cap * 6 * N * s.P);
   B.Ainv = c->alloc<double>((size_t)cap * 16 * s.H);
   B.Ui = c->alloc<double>((size_t)cap * N);
@@ -769,6 +778,7 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   write_ctl(c, ctl);
   c->occupied.assign(cap, 0);
   c->setup.assign(cap, 0);
+  c->lu.assign((size_t)cap * 4, LuFactors{});
   c->lu_bc.assign((size_t)cap * 4, 0);
   for (int i = 0; i < cap; ++i) c->lu_bc[(size_t)i * 4 + MAT_LNP] = 1;
   c->adapt.assign(cap, opf_ctx::Adapt{});
@@ -1817,14 +1827,13 @@ int opf_tim_lumesh_get(opf_ctx* c, int slot, int which, double* ab, int* ipiv) {
     if (which < 0 || which > 3) throw OpfError(OPF_ERR_ARG, "which must be 0..3");
     if (!c->setup[slot]) throw OpfError(OPF_ERR_STATE, "slot not set up");
     const int N = c->N, P = c->P, H = c->H;
-    lapack_factors(c, slot, which);
+    const LuFactors& L = lapack_factors(c, slot, which);
     // per-pair blocks [pair][n][LUS] and [pair][n]
     std::vector<double> F((size_t)P * N * LUS);
     std::vector<unsigned char> pv((size_t)P * N);
     HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(F.data(), lu_block(c->B, slot, which, 0, P, N), F.size() * sizeof(double),
-                     hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(pv.data(), pv_block(c->B, slot, which, 0, P, N), pv.size(), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(F.data(), L.F, F.size() * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(pv.data(), L.pv, pv.size(), hipMemcpyDeviceToHost));
     for (int hh = 0; hh < H; ++hh) {
       int k, m;
       if (hh < c->K) { m = 0; k = hh; }
@@ -1843,7 +1852,7 @@ int opf_tim_lumesh_get(opf_ctx* c, int slot, int which, double* ab, int* ipiv) {
 
 // tim_lumesh_invert on a host field: solved on the device, lane per harmonic.
 namespace opf {
-__global__ void k_lumesh_invert(Geo G, Bufs B, int slot, int which, int bc, double2* x);
+__global__ void k_lumesh_invert(Geo G, LuFactors L, int bc, double2* x);
 }
 
 extern "C" int opf_tim_lumesh_invert(opf_ctx* c, int slot, int which, int BC, double* bre, double* bim) {
@@ -1855,9 +1864,9 @@ extern "C" int opf_tim_lumesh_invert(opf_ctx* c, int slot, int which, int BC, do
     if (!bre || !bim) throw OpfError(OPF_ERR_ARG, "null field");
     const int bc = BC >= 0 ? BC : c->lu_bc[(size_t)slot * 4 + which];
     ensure_temps(c);
-    lapack_factors(c, slot, which);
+    const LuFactors& L = lapack_factors(c, slot, which);
     coll_to_dev(c, bre, bim, c->tC);
-    launch(c, "lumesh_invert", k_lumesh_invert, grid_h(c, 1), dim3(64), 0, c->G, c->B, slot, which, bc, c->tC);
+    launch(c, "lumesh_invert", k_lumesh_invert, grid_h(c, 1), dim3(64), 0, c->G, L, bc, c->tC);
     dev_to_coll(c, c->tC, bre, bim);
   });
 }

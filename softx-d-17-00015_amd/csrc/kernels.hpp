@@ -13,16 +13,24 @@ struct LuSpec {
   double c1, c2;
 };
 
+// LAPACK-form factors of one factor set (buffers on first use of
+// tim_lumesh_*): column n of pair p, LAPACK band row r at F[(p N + n) LUS + r],
+// pivot offset ipiv(n) - n at pv[p N + n].
+struct LuFactors {
+  double* F;
+  unsigned char* pv;
+  unsigned* built;   // per workgroup of k_lu_factor: the set's version that its factors are of
+};
+
 // All device arrays of one resolution class (slot-major).  Passed by value.
 struct Bufs {
   double2* U[3];        // velocity buffers [slot][3][N][Hp]; roles per slot in SlotCtl
   double2* Nraw[2];     // nonlinear terms without base-flow terms [slot][3][N][Hp]
   double2* om;          // curl of the current iterate [slot][3][N][Hp]
-  double* LU;           // LAPACK-form factors [slot][4 mats][P pairs][N columns][LUS] (first use of tim_lumesh_*)
-  unsigned char* PV;    // their pivot offsets ipiv(j)-j [slot][4][P][N]
   double* SE;           // block inverses (block_factor, solve.hpp) [slot][4 mats][P pairs][blk_count(N)][16],
                         // element (row, column) at 4 column + row
   LuSpec* spec;         // [slot][4] the matrix each factor set holds
+  unsigned* ver;        // [slot][4] its version: counts the set's rebuilds
   double* Uinf;         // influence vectors [slot][6][N][P]
   double* Ainv;         // inverted influence matrices [slot][16][H]
   double* Ui;           // flux correction vector [slot][N]
@@ -54,15 +62,6 @@ struct FftTiles {
   int tz;     // z lines per workgroup in the theta kernel
   FftPlan pz, pt;
 };
-
-// Factor blocks: matrix `mat` of pair p, column n, LAPACK band row r at
-// lu_block(...)[n*LUS + r]; pivot offset at pv_block(...)[n].
-__host__ __device__ inline double* lu_block(const Bufs& B, int slot, int mat, int p, int P, int N) {
-  return B.LU + (((size_t)(slot * 4 + mat) * P + p) * N) * LUS;
-}
-__host__ __device__ inline unsigned char* pv_block(const Bufs& B, int slot, int mat, int p, int P, int N) {
-  return B.PV + ((size_t)(slot * 4 + mat) * P + p) * N;
-}
 
 // Block elimination: blocks of four rows, the block where the two sides meet,
 // and the scale of a matrix' unknowns (solve.hpp).
@@ -115,7 +114,7 @@ __host__ __device__ constexpr int tile_m(int Z) { return FFT_TILE / Z; }
 __host__ __device__ constexpr int padded_len(int L) { return (L + (L - 1) / 16 + 1) | 1; }
 
 __global__ void k_block_factor(Geo G, Bufs B, int slot, LuSpec A);
-__global__ void k_lu_factor(Geo G, Bufs B, int slot, int mat, int* singular);
+__global__ void k_lu_factor(Geo G, Bufs B, LuFactors L, int slot, int mat, int* singular);
 using MatricesKern = void (*)(Geo, Bufs, int, int);
 MatricesKern matrices_kernel(int N);
 inline size_t matrices_smem(int N) { return (size_t)(10 * (N + 8) + 40 * (N + 4) + 48 * (KL + 1)) * sizeof(double); }

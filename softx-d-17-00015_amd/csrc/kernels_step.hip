@@ -256,6 +256,11 @@ __device__ __forceinline__ LuSpec matrix_spec(int mat, const SlotParams& prm) {
   return LuSpec{mat, pr || mat == MAT_LDZ ? 0 : (mat == MAT_LDP ? 1 : -1), pr ? 1 : 0, pr ? 0.0 : 1.0 / prm.dt,
                 pr ? 1.0 : -prm.implicit * prm.nu / prm.Re};
 }
+// the factor set A.mat now holds the matrix A
+__device__ __forceinline__ void hold(const Bufs& B, int slot, const LuSpec& A) {
+  B.spec[slot * 4 + A.mat] = A;
+  atomicAdd(&B.ver[slot * 4 + A.mat], 1u);
+}
 __device__ __forceinline__ void block_factor(const Geo& G, const Bufs& B, int slot, const LuSpec& A, int mat, int p,
                                              int side, double alpha, const double* T) {
   const int N = G.N, P = G.P, NB = blk_count(N);
@@ -418,7 +423,7 @@ __device__ __forceinline__ void block_factor(const Geo& G, const Bufs& B, int sl
 __global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot, LuSpec A) {
   __shared__ double T[10 * (MAXN + 8)];
   for (int i = threadIdx.x; i < 10 * (G.N + 8); i += 64) T[i] = G.mesh[MeshOff::make(G.N).lapT + i];
-  if (threadIdx.x == 0 && blockIdx.x == 0) B.spec[slot * 4 + A.mat] = A;
+  if (threadIdx.x == 0 && blockIdx.x == 0) hold(B, slot, A);
   __syncthreads();
   // spare lanes repeat the last pair
   block_factor(G, B, slot, A, A.mat, min((int)blockIdx.x * 32 + (int)(threadIdx.x >> 1), G.P - 1), threadIdx.x & 1,
@@ -429,17 +434,23 @@ __global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot, Lu
 // tim_lumesh_init (timestep.f90:67-96) + DGBTF2 of one matrix per pair in
 // LAPACK band layout, for tim_lumesh_get / tim_lumesh_invert (the time step
 // solves with block_factor's inverses).  Four lanes per system.  *singular is
-// set where a pivot is zero.
+// set where a pivot is zero.  A workgroup whose factors are of the set's present
+// version has nothing to do, so a host that solves with its own sets again and
+// again pays for the factors once per set; the version counts on the device,
+// where the matrices change (adaptive time step, LES).
 // grid: x = pairs/16; 64 threads = 16 systems x 4 lanes.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot, int mat, int* singular) {
+__global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, LuFactors L, int slot, int mat,
+                                                 int* singular) {
   constexpr int LPS = 4;              // lanes per system
   constexpr int SPW = 64 / LPS;       // systems per workgroup
   const int q = threadIdx.x % LPS, sl = threadIdx.x / LPS;
   const int p = blockIdx.x * SPW + sl;
+  const unsigned ver = B.ver[slot * 4 + mat];
+  if (L.built[blockIdx.x] == ver) return;
   // no barriers below: a lane may leave on its own
   if (p >= G.P) return;
-  const int N = G.N, P = G.P;
+  const int N = G.N;
   const int m = p / G.K, k = p % G.K;  // pair (|k|, m)
   const SlotParams prm = B.prm[slot];
   const MeshOff mo = MeshOff::make(N);
@@ -447,8 +458,8 @@ __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot, int m
   const LuSpec spec = B.spec[slot * 4 + mat];   // the matrix that the factor set holds
   const int PM = spec.PM, BC = spec.BC;
   const double c1 = spec.c1, c2 = spec.c2;
-  double* F = lu_block(B, slot, mat, p, P, N);
-  unsigned char* pv = pv_block(B, slot, mat, p, P, N);
+  double* F = L.F + (size_t)p * N * LUS;
+  unsigned char* pv = L.pv + (size_t)p * N;
   // The elimination at column j touches columns j .. j + KV only, so each
   // system keeps a window of KV + 1 band columns in LDS (column c in slot
   // c mod 9, the systems' values interleaved) instead of working on the
@@ -599,6 +610,7 @@ __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, int slot, int m
     lds_fence();   // every lane has read column j before its slot is refilled
     place(wj, jn, nx, j + WC < N);
   }
+  if (threadIdx.x == 0) L.built[blockIdx.x] = ver;
 }
 
 // ---------------------------------------------------------------------------
@@ -843,7 +855,7 @@ __global__ void __launch_bounds__(256) k_matrices_t(Geo G, Bufs B, int slot0, in
   if (wave == 0) {
     const int fm = lane >> 4, fp = (lane >> 1) & 7;
     const LuSpec A = matrix_spec(fm, prm);
-    if (p0 == 0 && (lane & 15) == 0) B.spec[slot * 4 + fm] = A;
+    if (p0 == 0 && (lane & 15) == 0) hold(B, slot, A);
     block_factor(G, B, slot, A, fm, p0 + min(fp, np - 1), lane & 1, prm.alpha, lap);   // spare lanes repeat the last pair
   }
   __syncthreads();
@@ -1429,19 +1441,19 @@ __global__ void k_imposesym(Geo G, Bufs B, int slot0) {
 }
 
 // tim_lumesh_invert (timestep.f90:102-123) of one coll field x[n][Hp] with
-// the slot's factor `which`; (0,0) of the pressure matrix gives zero.
-__global__ void k_lumesh_invert(Geo G, Bufs B, int slot, int which, int bc, double2* x) {
+// the factors L; (0,0) of the pressure matrix gives zero.
+__global__ void k_lumesh_invert(Geo G, LuFactors L, int bc, double2* x) {
   const int h = blockIdx.x * blockDim.x + threadIdx.x;
   if (h >= G.H) return;
   int k, m;
   harmonic_km(h, G.K, k, m);
-  const int N = G.N, P = G.P;
+  const int N = G.N;
   const int p = m * G.K + (k < 0 ? -k : k);
   if (bc == 1 && k == 0 && m == 0) {   // the (0,0) pressure system is singular: b = 0
     for (int n = 0; n < N; ++n) x[(size_t)n * G.Hp + h] = make_double2(0.0, 0.0);
     return;
   }
-  lu_solve<double2>(lu_block(B, slot, which, p, P, N), pv_block(B, slot, which, p, P, N), x + h, G.Hp, N);
+  lu_solve<double2>(L.F + (size_t)p * N * LUS, L.pv + (size_t)p * N, x + h, G.Hp, N);
 }
 
 }  // namespace opf

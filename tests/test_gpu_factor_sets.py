@@ -17,6 +17,72 @@ def opf():
     return pkg
 
 
+def _field(rng, N, H):
+    b = rng.standard_normal((N, H)) + 1j * rng.standard_normal((N, H))
+    b[0] = b[-1] = 0.0
+    return b
+
+
+def test_factors_are_built_once_per_set(opf):
+    """tim_lumesh_invert factors a set when it is first used and not again until
+    the set changes: a repeated solve spends on the factors no more than half of
+    what the first did (the launch finds nothing to do), with the same result,
+    and the factors of one set take the memory of one set."""
+    N, K, M = 48, 32, 24
+    ctx = opf.Context(N, K, M, capacity=3)
+    ctx.setup(0, RE, ALPHA, DT)
+    H = ctx.H
+    b = _field(np.random.default_rng(1), N, H)
+    ctx.coll2phys(b)                       # the transforms' buffers
+    bytes0 = _bytes(ctx)
+    times, xs = [], []
+    for _ in range(3):
+        ctx.kernel_timing(True)
+        xs.append(ctx.lumesh_invert(0, opf.LDZ, b))
+        times.append(ctx.kernel_time("lapack_factor")[0])
+        ctx.kernel_timing(False)
+    assert np.array_equal(xs[0], xs[1]) and np.array_equal(xs[0], xs[2])
+    assert max(times[1:]) <= 0.5 * times[0], times
+    assert _bytes(ctx) - bytes0 <= K * M * 129 * N + 8192
+    # a change of the set is seen
+    ctx.vel_matrices(0, 2.0 * DT)
+    oc = O.Ctx(N, K, M, Re=RE, alpha=ALPHA, dt=2.0 * DT)
+    ref = oc.lumesh_invert(oc.lumesh_init(0, 0, 1.0 / (2.0 * DT), -0.51 / RE), b)
+    assert rel_err(ctx.lumesh_invert(0, opf.LDZ, b), ref) <= 1e-12
+
+
+def _bytes(ctx):
+    import ctypes as C
+    n = C.c_size_t()
+    opf_int = [C.c_int() for _ in range(6)]
+    ctx.lib.opf_ctx_dims(ctx.h, *[C.byref(d) for d in opf_int], C.byref(n))
+    return n.value
+
+
+def test_factors_follow_the_device_loop(opf):
+    """The factors that tim_lumesh_get returns are those of the matrices as the
+    device loop left them (adaptive time step), also where they were asked for
+    before."""
+    N, K, M = 16, 6, 4
+    from opf import ic
+    me = opf.host_mesh(N)
+    u = ic.seeded_perturbation(me["r"], me["intrdr"], K, M, ALPHA, 3, 1e-3)
+    ctx = opf.Context(N, K, M)
+    ctx.adaptive(0)
+    ctx.setup(0, RE, ALPHA, DT)
+    before = ctx.lumesh_get(0, opf.LDZ)[0]
+    ctx.put_state(0, *u)
+    ctx.run(4)
+    dt = ctx.timestep(0)["dt"]
+    assert dt != DT
+    got = ctx.lumesh_get(0, opf.LDZ)
+    fresh = opf.Context(N, K, M)
+    fresh.setup(0, RE, ALPHA, dt)
+    ref = fresh.lumesh_get(0, opf.LDZ)
+    assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
+    assert not np.array_equal(got[0], before)
+
+
 def test_reading_a_singular_set_leaves_the_slot_alone(opf):
     """A set that tim_lumesh_init reported singular can be read and solved with
     without marking the slot's run as failed."""
