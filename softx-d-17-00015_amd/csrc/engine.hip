@@ -125,7 +125,9 @@ struct opf_ctx {
   double* dterrHost = nullptr;   // pinned: tim_dterr of the last host-driven call (first use)
   SlotParams* prmHost = nullptr; // pinned parameters of asynchronous admissions (first use)
   std::vector<LuFactors> lu;     // LAPACK-form factors [slot][4] (first use)
-  int* luSingular = nullptr;     // a zero pivot of tim_lumesh_init's factors (first use)
+  int* luVerdict = nullptr;      // tim_lumesh_init: a zero pivot; blocks that cannot represent the set (first use)
+  std::vector<int> lu_unsafe;    // the latter per factor set [slot][4]
+  int n_unsafe = 0;              // and how many
   std::vector<int> lu_bc;        // BC of each factor set [slot][4] (tim_lumesh_invert's (0,0) rule)
   int device = 0;                // HIP device of the context
   // launch modes of the time loop: one iteration captured as a HIP graph
@@ -138,11 +140,11 @@ struct opf_ctx {
   int* smapDev = nullptr;        // compacted slot list on the device [cap]
   std::vector<int> smapHost;     // its host copy (what the device holds)
   struct GraphKey {
-    int s0 = -1, ns = 0, symm = 0, adapt = 0, iters = 0;
+    int s0 = -1, ns = 0, symm = 0, adapt = 0, banded = 0, iters = 0;
     const int* smap = nullptr;
     bool operator==(const GraphKey& o) const {
-      return s0 == o.s0 && ns == o.ns && symm == o.symm && adapt == o.adapt && iters == o.iters &&
-             smap == o.smap;
+      return s0 == o.s0 && ns == o.ns && symm == o.symm && adapt == o.adapt && banded == o.banded &&
+             iters == o.iters && smap == o.smap;
     }
   } gkey;
   hipGraphExec_t gexec = nullptr;
@@ -353,7 +355,18 @@ void launch_eval(opf_ctx* c, int s0, int ns) {
   launch_back(c, s0, ns);
 }
 
+void set_unsafe(opf_ctx* c, int slot, int which, int unsafe) {
+  int& u = c->lu_unsafe[(size_t)slot * 4 + which];
+  c->n_unsafe += unsafe - u;
+  u = unsafe;
+}
 void launch_step(opf_ctx* c, int s0, int ns) {
+  if (c->n_unsafe > 0) {   // a slot holds a set that needs the banded LU
+    const StepTiles st{1, c->P, step_smem(c->N, 1)};
+    launch(c, "step", step_kernel_banded(), dim3(8 * ((c->P + 7) / 8), 1, ns), dim3(step_threads(1)), st.smem, c->G, c->B,
+           st, s0);
+    return;
+  }
   const int per = (c->st.ngroups + 7) / 8;   // XCD-aware order inside the kernel
   launch(c, "step", step_kernel(c->N, c->st.gp), dim3(8 * per, 1, ns), dim3(step_threads(c->st.gp)), c->st.smem, c->G, c->B,
          c->st, s0);
@@ -394,7 +407,7 @@ void launch_iteration(opf_ctx* c, int s0, int ns) {
 // The LAPACK-form factors of one factor set, for tim_lumesh_get and
 // tim_lumesh_invert: built from the matrix the set holds when they are asked
 // for (the time step does not read them), where they are not there yet.  Buffers
-// per set on first use.  A zero pivot is left in luSingular, which only
+// per set on first use.  A zero pivot is left in luVerdict, which only
 // tim_lumesh_init looks at.
 const LuFactors& lapack_factors(opf_ctx* c, int slot, int which) {
   LuFactors& L = c->lu[(size_t)slot * 4 + which];
@@ -403,9 +416,10 @@ const LuFactors& lapack_factors(opf_ctx* c, int slot, int which) {
     L.F = c->alloc<double>(cols * LUS + (groups + 1) / 2 + (cols + 7) / 8);
     L.built = (unsigned*)(L.F + cols * LUS);
     L.pv = (unsigned char*)(L.F + cols * LUS + (groups + 1) / 2);
+    HIPCHK(hipMemcpy(c->B.lu + (size_t)slot * 4 + which, &L, sizeof L, hipMemcpyHostToDevice));
   }
-  if (!c->luSingular) c->luSingular = c->alloc<int>(1);
-  launch(c, "lapack_factor", k_lu_factor, dim3((unsigned)groups), dim3(64), 0, c->G, c->B, L, slot, which, c->luSingular);
+  if (!c->luVerdict) c->luVerdict = c->alloc<int>(2);
+  launch(c, "lapack_factor", k_lu_factor, dim3((unsigned)groups), dim3(64), 0, c->G, c->B, L, slot, which, c->luVerdict);
   return L;
 }
 
@@ -741,6 +755,8 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   B.SE = c->alloc<double>((size_t)cap * 4 * s.P * blk_count(N) * 16);
   B.spec = c->alloc<LuSpec>((size_t)cap * 4);
   B.ver = c->alloc<unsigned>((size_t)cap * 4);
+  B.lu = c->alloc<LuFactors>((size_t)cap * 4);
+  B.banded = c->alloc<int>(cap);
   B.Uinf = c->alloc<double>((size_t)cap * 6 * N * s.P);
   B.Ainv = c->alloc<double>((size_t)cap * 16 * s.H);
   B.Ui = c->alloc<double>((size_t)cap * N);
@@ -779,6 +795,7 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   c->occupied.assign(cap, 0);
   c->setup.assign(cap, 0);
   c->lu.assign((size_t)cap * 4, LuFactors{});
+  c->lu_unsafe.assign((size_t)cap * 4, 0);
   c->lu_bc.assign((size_t)cap * 4, 0);
   for (int i = 0; i < cap; ++i) c->lu_bc[(size_t)i * 4 + MAT_LNP] = 1;
   c->adapt.assign(cap, opf_ctx::Adapt{});
@@ -824,6 +841,7 @@ void slot_setup(opf_ctx* c, int slot, double Re, double alpha, double dt, double
   ctl[slot].status = 0;
   write_ctl(c, ctl);
   launch_matrices(c, slot, 1, 0);
+  for (int q = 0; q < 4; ++q) set_unsafe(c, slot, q, 0);
   ctl = read_ctl(c);
   if (ctl[slot].status != 0) {
     const int st = ctl[slot].status;
@@ -923,6 +941,7 @@ void enqueue_iterations(opf_ctx* c, int s0, int ns, long iterations) {
   key.ns = ns;
   key.symm = c->n_symm > 0;
   key.adapt = c->n_adaptive > 0;
+  key.banded = c->n_unsafe > 0;
   key.smap = c->B.smap;
   key.iters = gi;
   if (!c->gexec || !(key == c->gkey)) {
@@ -1883,19 +1902,25 @@ extern "C" int opf_tim_lumesh_init(opf_ctx* c, int slot, int which, int PM, int 
     auto ctl = read_ctl(c);
     ctl[slot].status = 0;
     write_ctl(c, ctl);
+    int verdict[2] = {0, 0};
+    if (!c->luVerdict) c->luVerdict = c->alloc<int>(2);
+    HIPCHK(hipMemcpy(c->luVerdict, verdict, sizeof verdict, hipMemcpyHostToDevice));
     launch(c, "factor", k_block_factor, dim3((c->P + 31) / 32), dim3(64), 0, c->G, c->B, slot,
-           LuSpec{which, PM, BC, c1, c2});
-    int singular = 0;
-    if (c->luSingular) HIPCHK(hipMemcpy(c->luSingular, &singular, sizeof(int), hipMemcpyHostToDevice));
+           LuSpec{which, PM, BC, c1, c2}, c->luVerdict + 1);
     lapack_factors(c, slot, which);   // DGBTF2's own verdict on a singular matrix
-    ctl = read_ctl(c);
+    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(hipMemcpy(verdict, c->luVerdict, sizeof verdict, hipMemcpyDeviceToHost));
     c->lu_bc[(size_t)slot * 4 + which] = BC;
-    HIPCHK(hipMemcpy(&singular, c->luSingular, sizeof(int), hipMemcpyDeviceToHost));
-    if (ctl[slot].status != 0 || singular) {
-      ctl[slot].status = 0;
-      write_ctl(c, ctl);
-      throw OpfError(OPF_ERR_SINGULAR, "tim_lumesh_init");
-    }
+    if (verdict[0]) throw OpfError(OPF_ERR_SINGULAR, "tim_lumesh_init");
+    // a set that needs row interchanges across blocks: the slot's steps solve
+    // with the LAPACK-form factors of all four sets
+    set_unsafe(c, slot, which, verdict[1]);
+    const int* unsafe = &c->lu_unsafe[(size_t)slot * 4];
+    const int banded = unsafe[0] | unsafe[1] | unsafe[2] | unsafe[3];
+    if (banded)
+      for (int q = 0; q < 4; ++q) lapack_factors(c, slot, q);
+    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(hipMemcpy(c->B.banded + slot, &banded, sizeof banded, hipMemcpyHostToDevice));
   });
 }
 

@@ -31,6 +31,8 @@ struct Bufs {
                         // element (row, column) at 4 column + row
   LuSpec* spec;         // [slot][4] the matrix each factor set holds
   unsigned* ver;        // [slot][4] its version: counts the set's rebuilds
+  LuFactors* lu;        // [slot][4] its LAPACK-form factors
+  int* banded;          // [slot] the step solves with those (a set needs row interchanges)
   double* Uinf;         // influence vectors [slot][6][N][P]
   double* Ainv;         // inverted influence matrices [slot][16][H]
   double* Ui;           // flux correction vector [slot][N]
@@ -113,7 +115,7 @@ __host__ __device__ constexpr int tile_m(int Z) { return FFT_TILE / Z; }
 
 __host__ __device__ constexpr int padded_len(int L) { return (L + (L - 1) / 16 + 1) | 1; }
 
-__global__ void k_block_factor(Geo G, Bufs B, int slot, LuSpec A);
+__global__ void k_block_factor(Geo G, Bufs B, int slot, LuSpec A, int* unsafe);
 __global__ void k_lu_factor(Geo G, Bufs B, LuFactors L, int slot, int mat, int* singular);
 using MatricesKern = void (*)(Geo, Bufs, int, int);
 MatricesKern matrices_kernel(int N);
@@ -153,6 +155,7 @@ __global__ void k_norm_sum(Geo G, const double* b, double* out);
 // the fused step kernel for N radial points and gp pairs per workgroup
 using StepKern = void (*)(Geo, Bufs, StepTiles, int);
 StepKern step_kernel(int N, int gp);
+StepKern step_kernel_banded();   // one pair per workgroup, any N: also for slots marked banded
 
 // transforms: kernels specialised to the radix plans of (Z, T), chosen once
 // per context by fft_kernels (run-time plans for other lengths)

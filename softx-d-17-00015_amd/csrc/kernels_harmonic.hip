@@ -194,7 +194,8 @@ __device__ __forceinline__ void control_decide(SlotCtl* c, const SlotParams& prm
 
 // IT: (radial point, harmonic) items per thread in the parallel stages,
 // N * 2 * GP <= IT * THR; THR: threads of the workgroup; SM >= blk_mid(N).
-template <int GP, int IT, int THR, int SM>
+// BAND: slots marked banded are solved with the LAPACK-form factors.
+template <int GP, int IT, int THR, int SM, bool BAND>
 __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const StepTiles& ST, int slot0) {
   const int slot = slot_of(B, slot0);
   SlotCtl* ctl = &B.ctl[slot];
@@ -424,6 +425,19 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   const bool solver = wave < GP;
   const int ps = p0 + min(wave, np - 1);   // a missing pair of the last group repeats a factor on zeros
   const int lhs = wave + GP * (bl.col >> 1);
+  const bool banded = BAND && B.banded[slot] != 0;
+  // the fields f0 .. f0 + nf - 1 of V with the sets m0 .. on lanes of their own
+  auto band_solve = [&](int f0, int nf, int m0) {
+    const int lane = tid & 63, f = lane >> 1, l = wave + GP * (lane & 1);
+    if (f >= nf) return;
+    double2* x = V + (f0 + f) * VC + l;
+    if (B.spec[slot * 4 + m0 + f].BC == 1 && ps == 0) {   // singular (timestep.f90:84): zero
+      for (int n = 0; n < N; ++n) x[n * GH] = make_double2(0.0, 0.0);
+      return;
+    }
+    const LuFactors L = B.lu[slot * 4 + m0 + f];
+    lu_solve<double2>(L.F + (size_t)ps * N * LUS, L.pv + (size_t)ps * N, x, GH, N);
+  };
   BlkE<SM, 1> EP;
   if (solver) blk_load(EP, 0, G, B, slot, B.spec[slot * 4 + MAT_LNP], MAT_LNP, ps, bl);
   __syncthreads();
@@ -509,10 +523,11 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
 
   // ---- stage 3: pressure solve with LNp (tim_lumesh_invert(1,...)) -------
   // (harmonics without a mode or with none to solve hold zeros and stay so)
-  if (solver) {
+  if (solver && !banded) {
     double* const x[1] = {(double*)(V + 2 * VC + lhs) + (bl.col & 1)};
     blk_solve(EP, N, bl, LT, x, 2 * GH);
   }
+  if (BAND && solver && banded) band_solve(2, 1, MAT_LNP);
   BlkE<SM, 2> EH;
   if (solver) {
     blk_load(EH, 0, G, B, slot, B.spec[slot * 4 + MAT_LDP + bl.mi], MAT_LDP + bl.mi, ps, bl);
@@ -593,7 +608,8 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   if (solver) {
     double* xp = (double*)(V + lhs) + (bl.col & 1);
     double* const x[2] = {xp + (bl.mi ? 2 * VC : 0), xp + 4 * VC};
-    blk_solve(EH, N, bl, LT, x, 2 * GH);
+    if (!banded) blk_solve(EH, N, bl, LT, x, 2 * GH);
+    else if (BAND) band_solve(0, 3, MAT_LDP);
     if (!EARLY) influence_loads();
   }
   __syncthreads();
@@ -818,10 +834,10 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
 
 }  // namespace
 
-template <int GP, int IT, int THR, int SM, int WPE>
+template <int GP, int IT, int THR, int SM, int WPE, bool BAND = false>
 __global__ void __launch_bounds__(THR) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_step_t(Geo G, Bufs B, StepTiles ST, int slot0) {
-  step_body<GP, IT, THR, SM>(G, B, ST, slot0);
+  step_body<GP, IT, THR, SM, BAND>(G, B, ST, slot0);
 }
 
 StepKern step_kernel(int N, int gp) {
@@ -834,5 +850,6 @@ StepKern step_kernel(int N, int gp) {
   static const StepKern g4[] = {k_step_t<4, 1, 256, 4, 3>, k_step_t<4, 2, 256, 8, 3>, k_step_t<4, 3, 256, 12, 2>};
   return gp == 1 ? g1[r] : gp == 2 ? g2[r] : g4[r];
 }
+StepKern step_kernel_banded() { return k_step_t<1, 2, 128, 16, 2, true>; }
 
 }  // namespace opf

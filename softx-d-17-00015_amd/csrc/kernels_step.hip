@@ -58,90 +58,6 @@ __device__ __forceinline__ double2 band_row(const double* band, int N, int n,
 }
 
 // ---------------------------------------------------------------------------
-// banded LU solve (LAPACK DGBTRS 'N', KL = KU = 4), one system per lane.
-// F: factor of this lane's matrix, column n at F[n*LUS] with the 13 rows of
-// LAPACK band storage AB(1:13, n) (rows 9..12 hold the multipliers); pv:
-// pivot offsets ipiv(j)-j; x: vector with stride xs, solved in place.  T is
-// double or double2 (real and imaginary parts solved with the same factor,
-// as tim_lumesh_invert does with two dgbtrs calls).
-// ---------------------------------------------------------------------------
-template <typename T> struct VT;
-template <> struct VT<double> {
-  __device__ static double zero() { return 0.0; }
-  __device__ static void axpy(double& y, double a, double t) { y = y + a * t; }
-  __device__ static double neg(double v) { return -v; }
-  __device__ static double div(double v, double d) { return v / d; }
-  __device__ static void sub_mul(double& y, double t, double a) { y = y - t * a; }
-};
-template <> struct VT<double2> {
-  __device__ static double2 zero() { return make_double2(0.0, 0.0); }
-  __device__ static void axpy(double2& y, double a, double2 t) {
-    y.x = y.x + a * t.x;
-    y.y = y.y + a * t.y;
-  }
-  __device__ static double2 neg(double2 v) { return make_double2(-v.x, -v.y); }
-  __device__ static double2 div(double2 v, double d) { return make_double2(v.x / d, v.y / d); }
-  __device__ static void sub_mul(double2& y, double2 t, double a) {
-    y.x = y.x - t.x * a;
-    y.y = y.y - t.y * a;
-  }
-};
-
-template <typename T>
-__device__ void lu_solve(const double* F, const unsigned char* pv, T* x, size_t xs, int N) {
-  using V = VT<T>;
-  // L solve with row interchanges: window w[i] = b(j+i)
-  T w[5];
-#pragma unroll
-  for (int i = 0; i < 5; ++i) w[i] = i < N ? x[i * xs] : V::zero();
-  for (int j = 0; j < N - 1; ++j) {
-    const int off = pv[j];
-    const T a0 = w[0];
-    T s = w[0];
-    s = off == 1 ? w[1] : s;
-    s = off == 2 ? w[2] : s;
-    s = off == 3 ? w[3] : s;
-    s = off == 4 ? w[4] : s;
-    w[0] = s;
-    w[1] = off == 1 ? a0 : w[1];
-    w[2] = off == 2 ? a0 : w[2];
-    w[3] = off == 3 ? a0 : w[3];
-    w[4] = off == 4 ? a0 : w[4];
-    const T t = V::neg(w[0]);
-    const int lm = N - 1 - j < KL ? N - 1 - j : KL;
-    const double* Fj = F + (size_t)j * LUS;
-#pragma unroll
-    for (int i = 1; i <= KL; ++i)
-      if (i <= lm) V::axpy(w[i], Fj[8 + i], t);
-    x[j * xs] = w[0];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = w[i + 1];
-    w[4] = j + 5 < N ? x[(j + 5) * xs] : V::zero();
-  }
-  // U solve (DTBSV upper, 8 superdiagonals): window v[q] = x(j-8+q)
-  T v[9];
-  const int jN = N - 1;
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int idx = jN - 8 + q;
-    v[q] = idx >= 0 ? x[idx * xs] : V::zero();
-  }
-  v[8] = w[0];
-  for (int j = N - 1; j >= 0; --j) {
-    const double* Fj = F + (size_t)j * LUS;
-    v[8] = V::div(v[8], Fj[8]);
-    const T t = v[8];
-    x[j * xs] = t;
-#pragma unroll
-    for (int d = 1; d <= 8; ++d)
-      if (j - d >= 0) V::sub_mul(v[8 - d], t, Fj[8 - d]);
-#pragma unroll
-    for (int q = 8; q >= 1; --q) v[q] = v[q - 1];
-    v[0] = j - 9 >= 0 ? x[(j - 9) * xs] : V::zero();
-  }
-}
-
-// ---------------------------------------------------------------------------
 // wall boundary residuals of the influence method (vel_evalBC,
 // velocity.f90:262-298) for one harmonic; inputs are the last KL+1 radial
 // values of u+, u-, uz.
@@ -245,11 +161,23 @@ __device__ __forceinline__ double diag_d(double r2inv, int Mp, int m, double alp
 // and, for the block where the sides meet, both sides' terms subtracted.  The
 // 4 x 4 inverses interchange rows; between blocks nothing is interchanged (the
 // boundary rows, whose scale differs from the interior's, sit in the outermost
-// blocks; against 80-bit arithmetic the solves are as accurate as with the
-// banded LU and partial pivoting, error ratio 0.3 to 1.1 over N = 9 .. 128).
+// blocks; against 80-bit arithmetic the solves are about as accurate as with the
+// banded LU and partial pivoting: error ratio 0.3 to 1.8 in the geometric mean
+// over N = 9 .. 128, single systems 30 times better or worse).
 // A lane's chain is N / 8 blocks of a few hundred instructions, which bounds it.
 // T: MeshOff::lapT in LDS.
+// The matrices of vel_matrices are definite and their Schur complements stay
+// near their diagonal blocks (row sums of the subtracted terms up to 0.7 of the
+// block's own).  A matrix that a caller gives tim_lumesh_init need not be: where
+// a leading block is singular, or nearly, the elimination has nothing to divide
+// by.  CHECK sets *unsafe where a subtracted term exceeds BLK_GROWTH times the
+// block's own row; the step then solves that slot with the banded LU.  Why the
+// line lies there: over indefinite matrices with c1 near such points, against
+// 80-bit arithmetic, the block elimination's error is 0.7 to 0.9 of the banded
+// LU's in the geometric mean with terms up to 10 times the row, 1.7 at 10 to 30,
+// 4 at 30 to 100, 130 at 300 to 1000, and it grows with the square from there.
 // ---------------------------------------------------------------------------
+constexpr double BLK_GROWTH = 10.0;
 // the matrices of vel_matrices (velocity.f90:85-100)
 __device__ __forceinline__ LuSpec matrix_spec(int mat, const SlotParams& prm) {
   const bool pr = mat == MAT_LNP;
@@ -261,8 +189,9 @@ __device__ __forceinline__ void hold(const Bufs& B, int slot, const LuSpec& A) {
   B.spec[slot * 4 + A.mat] = A;
   atomicAdd(&B.ver[slot * 4 + A.mat], 1u);
 }
+template <bool CHECK>
 __device__ __forceinline__ void block_factor(const Geo& G, const Bufs& B, int slot, const LuSpec& A, int mat, int p,
-                                             int side, double alpha, const double* T) {
+                                             int side, double alpha, const double* T, int* unsafe) {
   const int N = G.N, P = G.P, NB = blk_count(N);
   const MeshOff mo = MeshOff::make(N);
   const double* me = G.mesh;
@@ -355,7 +284,10 @@ __device__ __forceinline__ void block_factor(const Geo& G, const Bufs& B, int sl
         }
       }
     }
-    if (singular && !raw) atomicMax(&B.ctl[slot].status, 100 + mat);
+    if (singular && !raw) {
+      if (CHECK) *unsafe = 1;
+      else atomicMax(&B.ctl[slot].status, 100 + mat);
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -369,6 +301,25 @@ __device__ __forceinline__ void block_factor(const Geo& G, const Bufs& B, int sl
         *(double2*)(out + t * 16 + 4 * j + i) =
             raw ? make_double2(0.0, 0.0) : make_double2(sc * E[i][j], sc * E[i + 1][j]);
   };
+  // D -= U; a row whose term dwarfs it loses that many digits
+  auto subtract = [&](double (&D)[4][4], const double (&U)[4][4]) {
+    if (CHECK && !raw) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        double u = 0.0, d = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          u = u + fabs(U[i][j]);
+          d = d + fabs(D[i][j]);
+        }
+        if (!(u <= BLK_GROWTH * d)) *unsafe = 1;   // a NaN, after a singular block, also
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) D[i][j] = D[i][j] - U[i][j];
+  };
   const int nm = blk_mid(N);
   const int steps = side ? NB - 1 - nm : nm, dt = side ? -1 : 1;
   double D[4][4], U[4][4];   // the next block's matrix; the terms to subtract from it
@@ -381,10 +332,7 @@ __device__ __forceinline__ void block_factor(const Geo& G, const Bufs& B, int sl
   for (int s = 0; s < nm; ++s) {
     if (s >= steps) break;
     diagonal(t, D);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) D[i][j] = D[i][j] - U[i][j];
+    subtract(D, U);
     invert(D);
     store(t, D);
     double C[4][4], Y[4][4];
@@ -414,20 +362,21 @@ __device__ __forceinline__ void block_factor(const Geo& G, const Bufs& B, int sl
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) D[i][j] = D[i][j] - (U[i][j] + __shfl_xor(U[i][j], 1));
+    for (int j = 0; j < 4; ++j) U[i][j] = U[i][j] + __shfl_xor(U[i][j], 1);
+  subtract(D, U);
   invert(D);
   if (side == 0) store(nm, D);
 }
 
 // one factor set of its own matrix (tim_lumesh_init).  grid: x = pairs / 32; 64 threads.
-__global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot, LuSpec A) {
+__global__ void __launch_bounds__(64) k_block_factor(Geo G, Bufs B, int slot, LuSpec A, int* unsafe) {
   __shared__ double T[10 * (MAXN + 8)];
   for (int i = threadIdx.x; i < 10 * (G.N + 8); i += 64) T[i] = G.mesh[MeshOff::make(G.N).lapT + i];
   if (threadIdx.x == 0 && blockIdx.x == 0) hold(B, slot, A);
   __syncthreads();
   // spare lanes repeat the last pair
-  block_factor(G, B, slot, A, A.mat, min((int)blockIdx.x * 32 + (int)(threadIdx.x >> 1), G.P - 1), threadIdx.x & 1,
-               B.prm[slot].alpha, T);
+  block_factor<true>(G, B, slot, A, A.mat, min((int)blockIdx.x * 32 + (int)(threadIdx.x >> 1), G.P - 1),
+                     threadIdx.x & 1, B.prm[slot].alpha, T, unsafe);
 }
 
 // ---------------------------------------------------------------------------
@@ -856,7 +805,9 @@ __global__ void __launch_bounds__(256) k_matrices_t(Geo G, Bufs B, int slot0, in
     const int fm = lane >> 4, fp = (lane >> 1) & 7;
     const LuSpec A = matrix_spec(fm, prm);
     if (p0 == 0 && (lane & 15) == 0) hold(B, slot, A);
-    block_factor(G, B, slot, A, fm, p0 + min(fp, np - 1), lane & 1, prm.alpha, lap);   // spare lanes repeat the last pair
+    if (p0 == 0 && lane == 0) B.banded[slot] = 0;
+    // spare lanes repeat the last pair
+    block_factor<false>(G, B, slot, A, fm, p0 + min(fp, np - 1), lane & 1, prm.alpha, lap, nullptr);
   }
   __syncthreads();
   const BlkLane l = BlkLane::make(lane);

@@ -26,6 +26,10 @@
 // of blocks, N / 8 pairs, and its code is short: a wave runs it once per launch,
 // at the rate at which instructions arrive rather than execute.  (An
 // elimination row by row took 90 to 105 ns a row in straight-line code.)
+//
+// lu_solve at the end is that elimination, with LAPACK's factors and row
+// interchanges: tim_lumesh_invert's, and the step kernel's for a slot one of
+// whose sets the blocks cannot represent (block_factor).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -167,6 +171,98 @@ __device__ __forceinline__ void blk_solve(BlkE<SM, NG>& R, int N, const BlkLane&
         for (int g = 0; g < NG; ++g) x[g][rowof(i)] = c[g] * R.rs[g];
       }
     }
+}
+
+// ---------------------------------------------------------------------------
+// banded LU solve (LAPACK DGBTRS 'N', KL = KU = 4), one system per lane.
+// F: factor of this lane's matrix, column n at F[n*LUS] with the 13 rows of
+// LAPACK band storage AB(1:13, n) (rows 9..12 hold the multipliers); pv:
+// pivot offsets ipiv(j)-j; x: vector with stride xs, solved in place.  T is
+// double or double2 (real and imaginary parts solved with the same factor,
+// as tim_lumesh_invert does with two dgbtrs calls).
+// ---------------------------------------------------------------------------
+template <typename T> struct VT;
+template <> struct VT<double> {
+  __device__ static double zero() { return 0.0; }
+  __device__ static void axpy(double& y, double a, double t) {
+#pragma clang fp contract(off)
+    y = y + a * t;
+  }
+  __device__ static double neg(double v) { return -v; }
+  __device__ static double div(double v, double d) { return v / d; }
+  __device__ static void sub_mul(double& y, double t, double a) {
+#pragma clang fp contract(off)
+    y = y - t * a;
+  }
+};
+template <> struct VT<double2> {
+  __device__ static double2 zero() { return make_double2(0.0, 0.0); }
+  __device__ static void axpy(double2& y, double a, double2 t) {
+#pragma clang fp contract(off)
+    y.x = y.x + a * t.x;
+    y.y = y.y + a * t.y;
+  }
+  __device__ static double2 neg(double2 v) { return make_double2(-v.x, -v.y); }
+  __device__ static double2 div(double2 v, double d) { return make_double2(v.x / d, v.y / d); }
+  __device__ static void sub_mul(double2& y, double2 t, double a) {
+#pragma clang fp contract(off)
+    y.x = y.x - t.x * a;
+    y.y = y.y - t.y * a;
+  }
+};
+
+template <typename T>
+__device__ void lu_solve(const double* F, const unsigned char* pv, T* x, size_t xs, int N) {
+  using V = VT<T>;
+  // L solve with row interchanges: window w[i] = b(j+i)
+  T w[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) w[i] = i < N ? x[i * xs] : V::zero();
+  for (int j = 0; j < N - 1; ++j) {
+    const int off = pv[j];
+    const T a0 = w[0];
+    T s = w[0];
+    s = off == 1 ? w[1] : s;
+    s = off == 2 ? w[2] : s;
+    s = off == 3 ? w[3] : s;
+    s = off == 4 ? w[4] : s;
+    w[0] = s;
+    w[1] = off == 1 ? a0 : w[1];
+    w[2] = off == 2 ? a0 : w[2];
+    w[3] = off == 3 ? a0 : w[3];
+    w[4] = off == 4 ? a0 : w[4];
+    const T t = V::neg(w[0]);
+    const int lm = N - 1 - j < KL ? N - 1 - j : KL;
+    const double* Fj = F + (size_t)j * LUS;
+#pragma unroll
+    for (int i = 1; i <= KL; ++i)
+      if (i <= lm) V::axpy(w[i], Fj[8 + i], t);
+    x[j * xs] = w[0];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = w[i + 1];
+    w[4] = j + 5 < N ? x[(j + 5) * xs] : V::zero();
+  }
+  // U solve (DTBSV upper, 8 superdiagonals): window v[q] = x(j-8+q)
+  T v[9];
+  const int jN = N - 1;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int idx = jN - 8 + q;
+    v[q] = idx >= 0 ? x[idx * xs] : V::zero();
+  }
+  v[8] = w[0];
+  for (int j = N - 1; j >= 0; --j) {
+    const double* Fj = F + (size_t)j * LUS;
+    v[8] = V::div(v[8], Fj[8]);
+    const T t = v[8];
+    x[j * xs] = t;
+#pragma unroll
+    for (int d = 1; d <= 8; ++d)
+      if (j - d >= 0) V::sub_mul(v[8 - d], t, Fj[8 - d]);
+#pragma unroll
+    for (int q = 8; q >= 1; --q) v[q] = v[q - 1];
+    v[0] = j - 9 >= 0 ? x[(j - 9) * xs] : V::zero();
+  }
 }
 
 }  // namespace opf

@@ -96,3 +96,46 @@ def test_reading_a_singular_set_leaves_the_slot_alone(opf):
     assert ctx.status(0)["status"] == 0
     ctx.lumesh_invert(0, opf.LDM, np.zeros((N, ctx.H), complex))
     assert ctx.status(0)["status"] == 0
+
+
+# c1 that make a leading principal block (rows 0 .. 3 or 0 .. 7) of one pair's
+# matrix c1 + c2 Lap (c2 = -3e-4, PM = 0, N = 20, alpha = 1.25) singular to a few
+# 1e-14, while all whole matrices are regular (condition below 4e5): an
+# elimination by blocks of four rows has nothing to divide by there.
+@pytest.mark.parametrize("pairs", [1, 2, 4])
+@pytest.mark.parametrize("c1", [-0.23272778313654063, -0.14513836407775046, -0.11507417760238585,
+                                -0.35203654575952653])
+def test_step_with_a_set_whose_leading_block_is_singular(opf, c1, pairs):
+    """tim_lumesh_init takes such a set, and the time step solves with it as
+    closely as tim_lumesh_invert does, while the context's other slots go on as
+    without it; then vel_matrices takes it back."""
+    from opf import ic
+    N, K, M, c2 = 20, 4, 3, -3e-4
+    ctx = opf.Context(N, K, M, capacity=2, pairs=pairs)
+    me = ctx.mesh()
+    u = ic.seeded_perturbation(me["r"], me["intrdr"], K, M, ALPHA, 3, 1e-2)
+    for s in (0, 1):
+        ctx.setup(s, RE, ALPHA, DT)
+        ctx.put_state(s, *u)
+    ctx.run(1, corr_fixed=1)
+    plain = ctx.get_state(0)
+    ctx.lumesh_init(0, opf.LDZ, 0, 0, c1, c2)
+    for s in (0, 1):
+        ctx.put_state(s, *u)
+    ctx.run(1, corr_fixed=1)
+    got = ctx.get_state(0)
+    for a, b in zip(ctx.get_state(1), plain):
+        assert np.array_equal(a, b)
+    oc = O.Ctx(N, K, M, Re=RE, alpha=ALPHA, dt=DT)
+    oc.LDz = oc.lumesh_init(0, 0, c1, c2)
+    oc.set_state(*u)
+    oc.run(1, ncorr_fixed=1)
+    # the condition of the matrices, 4e5, times the rounding of the right-hand
+    # sides, a few 1e-16
+    for c, ref in enumerate((oc.ur, oc.ut, oc.uz)):
+        assert rel_err(got[c], ref) <= 1e-9, c
+    ctx.vel_matrices(0, DT)
+    ctx.put_state(0, *u)
+    ctx.run(1, corr_fixed=1, slots=[0])
+    for a, b in zip(ctx.get_state(0), plain):
+        assert np.array_equal(a, b)
