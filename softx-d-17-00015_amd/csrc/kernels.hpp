@@ -69,7 +69,10 @@ struct FftTiles {
 // and the scale of a matrix' unknowns (solve.hpp).
 __host__ __device__ constexpr int blk_count(int N) { return (N + 3) / 4; }
 __host__ __device__ constexpr int blk_mid(int N) { return blk_count(N) / 2; }
-__host__ __device__ inline double blk_scale(double c2) { return c2 != 0.0 ? c2 : 1e-300; }
+// The scale is c2; without a Laplacian (c2 = 0, d_implicit = 0) a stand-in so
+// small that the couplings drop out of every sum, and so far from the smallest
+// double that the scaled unknowns keep their digits.
+__host__ __device__ inline double blk_scale(double c2) { return c2 != 0.0 ? c2 : 1e-100; }
 
 // curl of one harmonic at one radial point (var_coll_curl,
 // variables.f90:408-436) from u, the radial derivatives d1 of u_z and d2 of

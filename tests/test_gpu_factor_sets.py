@@ -139,3 +139,23 @@ def test_step_with_a_set_whose_leading_block_is_singular(opf, c1, pairs):
     ctx.run(1, corr_fixed=1, slots=[0])
     for a, b in zip(ctx.get_state(0), plain):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("amp", [1.0, 1e-10, 1e-20])
+def test_explicit_step_of_small_states(opf, amp):
+    """d_implicit = 0 (the matrices of the velocity are 1/dt I with the boundary
+    rows) at any size of the state: the solves lose no digits to underflow."""
+    from opf import ic
+    N, K, M, dt = 20, 4, 3, 1e-4
+    ctx = opf.Context(N, K, M)
+    ctx.setup(0, RE, ALPHA, dt, implicit=0.0)
+    me = ctx.mesh()
+    u = [amp * f for f in ic.seeded_perturbation(me["r"], me["intrdr"], K, M, ALPHA, 3, 1e-2)]
+    ctx.put_state(0, *u)
+    ctx.run(2, corr_fixed=1)
+    got = ctx.get_state(0)
+    oc = O.Ctx(N, K, M, Re=RE, alpha=ALPHA, dt=dt, implicit=0.0)
+    oc.set_state(*u)
+    oc.run(2, ncorr_fixed=1)
+    for c, ref in enumerate((oc.ur, oc.ut, oc.uz)):
+        assert rel_err(got[c], ref) <= 1e-12, (amp, c)
