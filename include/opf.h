@@ -382,7 +382,9 @@ int opf_launch_mode(opf_ctx* ctx, int graph, int compact, int streams, int* grap
 
 /* Launch shapes in use (no reference counterpart): pairs per workgroup of the
  * step kernel, m columns per z-transform workgroup, z-lines per theta
- * workgroup. */
+ * workgroup.  The last two are at most what the kernels of the transform
+ * lengths hold, also where opf_ctx_create_tiles was asked for more, and can be
+ * passed back to it. */
 int opf_tile_config(const opf_ctx* ctx, int* pairs, int* tm, int* tz);
 
 /* Launch shape of the fused step kernel chosen at opf_create: (|k|, m)

@@ -675,11 +675,14 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
     // the default width) from the caller or the table
     const int tm = tm_req > 0 ? tm_req : tuned.tm;
     const int tz = tz_req > 0 ? tz_req : tuned.tz;
+    const int tz_run = fft_kernels(c->tiles.pz, c->tiles.pt, c->tiles, M).t.tz;   // the width that runs by default
     if (tm > 0) {
       if (tm > c->tiles.tm) throw OpfError(OPF_ERR_ARG, "z tile wider than the kernels hold");
       c->tiles.tm = tm;
     }
-    if (tz > 0 && tz != c->tiles.tz) {
+    if (tz > 0 && tz != c->tiles.tz && tz == tz_run) {
+      c->tiles.tz = tz;
+    } else if (tz > 0 && tz != c->tiles.tz) {
       // the theta kernel transforms N_z of z-lines 2q and 2q + 1 together; an
       // even tile keeps those partners (and so the rounding) of the default
       if (tz > c->tiles.tz) throw OpfError(OPF_ERR_ARG, "theta tile wider than the kernels hold");
@@ -1957,8 +1960,8 @@ extern "C" int opf_tile_config(const opf_ctx* c, int* pairs, int* tm, int* tz) {
   return guard([&] {
     if (!c) throw OpfError(OPF_ERR_ARG, "null context");
     if (pairs) *pairs = c->st.gp;
-    if (tm) *tm = c->tiles.tm;
-    if (tz) *tz = c->tiles.tz;
+    if (tm) *tm = c->fk.t.tm;   // what the launches use: at most what the kernels of the length hold
+    if (tz) *tz = c->fk.t.tz;
   });
 }
 

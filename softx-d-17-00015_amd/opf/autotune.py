@@ -88,10 +88,23 @@ def tune(wl, log=print):
     probe.close()
     cache = {}
 
+    def runs_as(shape):
+        """The shape that runs when `shape` is asked for: wider tiles than the
+        kernels of a length hold, and widths that split M unevenly, run as others."""
+        ctx = Context(N, K, M, capacity=1, pairs=shape[0], tm=shape[1], tz=shape[2])
+        try:
+            return ctx.tile_config() + tuple(shape[3:])
+        finally:
+            ctx.close()
+
     def cost(shape):
         if shape not in cache:
             try:
-                cache[shape] = time_shape(wl, shape, states)[0]
+                same = runs_as(shape)
+                if same != shape and same in cache:
+                    cache[shape] = cache[same]
+                    return cache[shape]
+                cache[shape] = cache[same] = time_shape(wl, shape, states)[0]
             except Exception as e:              # noqa: BLE001  (a shape the device cannot take)
                 log(f"  {shape}: rejected ({e})")
                 cache[shape] = float("inf")

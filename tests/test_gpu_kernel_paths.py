@@ -160,3 +160,19 @@ def test_viscosity_transform_lengths(opf, K, M):
     for c, ref in enumerate((oc.ur, oc.ut, oc.uz)):
         assert rel_err(got[c], ref) <= 1e-12, c
     ctx.close()
+
+
+# requests beyond what the kernels of the lengths hold (3K = 144: 8 columns; 3M =
+# 48, 72: 8 lines, 432: 2 where the run-time plans hold one) and widths that
+# split M unevenly
+@pytest.mark.parametrize("K,M,tm,tz,runs", [(48, 16, 14, 14, (8, 8)), (48, 16, 7, 6, (6, 6)), (48, 16, 1, 2, (1, 2)),
+                                            (48, 24, 13, 9, (8, 8)), (48, 24, 5, 0, (5, 8)), (3, 144, 0, 0, (14, 2)),
+                                            (3, 144, 20, 1, (14, 2))])
+def test_tile_config_names_the_tiles_that_run(opf, K, M, tm, tz, runs):
+    """opf_tile_config gives the widths that the launches use, and a context made
+    with those gives them again."""
+    for _ in range(2):
+        ctx = opf.Context(10, K, M, tm=tm, tz=tz)
+        assert ctx.tile_config()[1:] == runs
+        ctx.close()
+        tm, tz = runs
