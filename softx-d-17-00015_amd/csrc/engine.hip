@@ -416,7 +416,7 @@ const LuFactors& lapack_factors(opf_ctx* c, int slot, int which) {
     L.F = c->alloc<double>(cols * LUS + (groups + 1) / 2 + (cols + 7) / 8);
     L.built = (unsigned*)(L.F + cols * LUS);
     L.pv = (unsigned char*)(L.F + cols * LUS + (groups + 1) / 2);
-    HIPCHK(hipMemcpy(c->B.lu + (size_t)slot * 4 + which, &L, sizeof L, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(&c->B.sets[(size_t)slot * 4 + which].lu, &L, sizeof L, hipMemcpyHostToDevice));
   }
   if (!c->luVerdict) c->luVerdict = c->alloc<int>(2);
   launch(c, "lapack_factor", k_lu_factor, dim3((unsigned)groups), dim3(64), 0, c->G, c->B, L, slot, which, c->luVerdict);
@@ -757,8 +757,7 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   B.om = c->alloc<double2>(c3);
   B.SE = c->alloc<double>((size_t)cap * 4 * s.P * blk_count(N) * 16);
   B.spec = c->alloc<LuSpec>((size_t)cap * 4);
-  B.ver = c->alloc<unsigned>((size_t)cap * 4);
-  B.lu = c->alloc<LuFactors>((size_t)cap * 4);
+  B.sets = c->alloc<FactorSet>((size_t)cap * 4);
   B.banded = c->alloc<int>(cap);
   B.Uinf = c->alloc<double>((size_t)cap * 6 * N * s.P);
   B.Ainv = c->alloc<double>((size_t)cap * 16 * s.H);

@@ -21,18 +21,22 @@ struct LuFactors {
   unsigned char* pv;
   unsigned* built;   // per workgroup of k_lu_factor: the set's version that its factors are of
 };
+struct FactorSet {
+  LuFactors lu;
+  unsigned ver;      // counts the set's rebuilds
+  int pad;
+};
 
 // All device arrays of one resolution class (slot-major).  Passed by value.
 struct Bufs {
   double2* U[3];        // velocity buffers [slot][3][N][Hp]; roles per slot in SlotCtl
   double2* Nraw[2];     // nonlinear terms without base-flow terms [slot][3][N][Hp]
   double2* om;          // curl of the current iterate [slot][3][N][Hp]
+  FactorSet* sets;      // [slot][4 mats]
+  int* banded;          // [slot] the step solves with the sets' LAPACK-form factors (one needs row interchanges)
   double* SE;           // block inverses (block_factor, solve.hpp) [slot][4 mats][P pairs][blk_count(N)][16],
                         // element (row, column) at 4 column + row
   LuSpec* spec;         // [slot][4] the matrix each factor set holds
-  unsigned* ver;        // [slot][4] its version: counts the set's rebuilds
-  LuFactors* lu;        // [slot][4] its LAPACK-form factors
-  int* banded;          // [slot] the step solves with those (a set needs row interchanges)
   double* Uinf;         // influence vectors [slot][6][N][P]
   double* Ainv;         // inverted influence matrices [slot][16][H]
   double* Ui;           // flux correction vector [slot][N]

@@ -192,6 +192,22 @@ __device__ __forceinline__ void control_decide(SlotCtl* c, const SlotParams& prm
   }
 }
 
+// The systems of the sets m0 .. m0 + nf - 1 of pair p with their LAPACK-form
+// factors, in place, a lane per system: the fields f0 .. of V (VC double2 apart,
+// V at the pair's harmonic +k; -k is gp further), rows 2 gp double2 apart.
+__device__ void band_solve(const Geo& G, const Bufs& B, int slot, int f0, int nf, int m0, int p, double2* V, int VC,
+                           int gp, int lane) {
+  const int f = lane >> 1, N = G.N;
+  if (f >= nf) return;
+  double2* x = V + (f0 + f) * VC + gp * (lane & 1);
+  if (B.spec[slot * 4 + m0 + f].BC == 1 && p == 0) {   // singular (timestep.f90:84): zero
+    for (int n = 0; n < N; ++n) x[n * 2 * gp] = make_double2(0.0, 0.0);
+    return;
+  }
+  const LuFactors L = B.sets[slot * 4 + m0 + f].lu;
+  lu_solve<double2>(L.F + (size_t)p * N * LUS, L.pv + (size_t)p * N, x, 2 * gp, N);
+}
+
 // IT: (radial point, harmonic) items per thread in the parallel stages,
 // N * 2 * GP <= IT * THR; THR: threads of the workgroup; SM >= blk_mid(N).
 // BAND: slots marked banded are solved with the LAPACK-form factors.
@@ -425,19 +441,6 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   const bool solver = wave < GP;
   const int ps = p0 + min(wave, np - 1);   // a missing pair of the last group repeats a factor on zeros
   const int lhs = wave + GP * (bl.col >> 1);
-  const bool banded = BAND && B.banded[slot] != 0;
-  // the fields f0 .. f0 + nf - 1 of V with the sets m0 .. on lanes of their own
-  auto band_solve = [&](int f0, int nf, int m0) {
-    const int lane = tid & 63, f = lane >> 1, l = wave + GP * (lane & 1);
-    if (f >= nf) return;
-    double2* x = V + (f0 + f) * VC + l;
-    if (B.spec[slot * 4 + m0 + f].BC == 1 && ps == 0) {   // singular (timestep.f90:84): zero
-      for (int n = 0; n < N; ++n) x[n * GH] = make_double2(0.0, 0.0);
-      return;
-    }
-    const LuFactors L = B.lu[slot * 4 + m0 + f];
-    lu_solve<double2>(L.F + (size_t)ps * N * LUS, L.pv + (size_t)ps * N, x, GH, N);
-  };
   BlkE<SM, 1> EP;
   if (solver) blk_load(EP, 0, G, B, slot, B.spec[slot * 4 + MAT_LNP], MAT_LNP, ps, bl);
   __syncthreads();
@@ -523,11 +526,11 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
 
   // ---- stage 3: pressure solve with LNp (tim_lumesh_invert(1,...)) -------
   // (harmonics without a mode or with none to solve hold zeros and stay so)
-  if (solver && !banded) {
+  if (solver) {
     double* const x[1] = {(double*)(V + 2 * VC + lhs) + (bl.col & 1)};
-    blk_solve(EP, N, bl, LT, x, 2 * GH);
+    if (!BAND || !B.banded[slot]) blk_solve(EP, N, bl, LT, x, 2 * GH);
+    else band_solve(G, B, slot, 2, 1, MAT_LNP, ps, V + wave, VC, GP, tid & 63);
   }
-  if (BAND && solver && banded) band_solve(2, 1, MAT_LNP);
   BlkE<SM, 2> EH;
   if (solver) {
     blk_load(EH, 0, G, B, slot, B.spec[slot * 4 + MAT_LDP + bl.mi], MAT_LDP + bl.mi, ps, bl);
@@ -608,8 +611,8 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   if (solver) {
     double* xp = (double*)(V + lhs) + (bl.col & 1);
     double* const x[2] = {xp + (bl.mi ? 2 * VC : 0), xp + 4 * VC};
-    if (!banded) blk_solve(EH, N, bl, LT, x, 2 * GH);
-    else if (BAND) band_solve(0, 3, MAT_LDP);
+    if (!BAND || !B.banded[slot]) blk_solve(EH, N, bl, LT, x, 2 * GH);
+    else band_solve(G, B, slot, 0, 3, MAT_LDP, ps, V + wave, VC, GP, tid & 63);
     if (!EARLY) influence_loads();
   }
   __syncthreads();

@@ -187,7 +187,7 @@ __device__ __forceinline__ LuSpec matrix_spec(int mat, const SlotParams& prm) {
 // the factor set A.mat now holds the matrix A
 __device__ __forceinline__ void hold(const Bufs& B, int slot, const LuSpec& A) {
   B.spec[slot * 4 + A.mat] = A;
-  atomicAdd(&B.ver[slot * 4 + A.mat], 1u);
+  atomicAdd(&B.sets[slot * 4 + A.mat].ver, 1u);
 }
 template <bool CHECK>
 __device__ __forceinline__ void block_factor(const Geo& G, const Bufs& B, int slot, const LuSpec& A, int mat, int p,
@@ -395,7 +395,7 @@ __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, LuFactors L, in
   constexpr int SPW = 64 / LPS;       // systems per workgroup
   const int q = threadIdx.x % LPS, sl = threadIdx.x / LPS;
   const int p = blockIdx.x * SPW + sl;
-  const unsigned ver = B.ver[slot * 4 + mat];
+  const unsigned ver = B.sets[slot * 4 + mat].ver;
   if (L.built[blockIdx.x] == ver) return;
   // no barriers below: a lane may leave on its own
   if (p >= G.P) return;
