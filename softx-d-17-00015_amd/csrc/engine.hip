@@ -756,9 +756,14 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   for (int i = 0; i < 2; ++i) B.Nraw[i] = c->alloc<double2>(c3);
   B.om = c->alloc<double2>(c3);
   B.SE = c->alloc<double>((size_t)cap * 4 * s.P * blk_count(N) * 16);
-  B.spec = c->alloc<LuSpec>((size_t)cap * 4);
-  B.sets = c->alloc<FactorSet>((size_t)cap * 4);
-  B.banded = c->alloc<int>(cap);
+  struct SlotSets {   // one buffer: an allocation takes about 0.1 ms
+    FactorSet sets[4];
+    LuSpec spec[4];
+    int banded, pad;
+  };
+  B.sets = (FactorSet*)c->alloc<SlotSets>(cap);
+  B.spec = (LuSpec*)(B.sets + (size_t)cap * 4);
+  B.banded = (int*)(B.spec + (size_t)cap * 4);
   B.Uinf = c->alloc<double>((size_t)cap * 6 * N * s.P);
   B.Ainv = c->alloc<double>((size_t)cap * 16 * s.H);
   B.Ui = c->alloc<double>((size_t)cap * N);
