@@ -134,7 +134,7 @@ struct opf_ctx {
   // and replayed; iterations of a run's tail over the list of slots still
   // active (compaction)
   int use_graph = 0, use_compact = 1;   // use_graph: iterations per captured graph (0: eager)
-  int use_streams = 2;           // streams a run's slots are split over (1 or 2; table or 2)
+  int use_streams = 2;           // streams a run's slots are split over (1 or 2; table or choose_streams)
   hipStream_t stream2 = nullptr; // the second stream of a split run (first use)
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   int* smapDev = nullptr;        // compacted slot list on the device [cap]
@@ -221,7 +221,10 @@ FftTiles choose_tiles(int Z, int T, int M) {
 // Rows: N K M min_capacity pairs tm tz graph [measured figures]; '#' starts
 // a comment; graph = iterations per captured HIP graph (0: eager launches).
 // A context takes the row of its (N, K, M) with the largest min_capacity not
-// above its capacity.
+// above its capacity; a zero leaves that shape to the built-in choice.  The tuner
+// lets a row hold below twice the capacity it was measured at and follows it
+// with one of zeros from there: the shapes depend on how full the slots make the
+// chip.
 struct Tuned {
   int gp = 0, tm = 0, tz = 0, graph = 0, streams = 0;
 };
@@ -287,6 +290,15 @@ StepTiles choose_step_tiles(int N, int P, int cap, int ncu, int gp_req, size_t l
   if (t.smem > lds_max) throw OpfError(OPF_ERR_ARG, "step kernel tiles do not fit in LDS");
   return t;
 }
+
+// Streams of a run over many slots: two where the slots have more than four step
+// workgroups per CU, so that either half fills the chip; one where the halves
+// would only leave it emptier.  Time with one stream over two, and workgroups per
+// CU: (16,6,4) 16 and 256 slots 0.67, 0.75 and 1.03, 6; (24,16,8) 16, 32 and 64
+// slots 0.85, 2; 0.94, 4 and 1.02, 8; (32,24,12) 8 and 16 slots 0.93, 2.3 and
+// 1.13, 4.5; (64,32,24) 4 and 8 slots 0.98, 3 and 1.04, 6; (48,48,24) 4 slots 1.05,
+// 4.5; (64,64,48) 4 slots 1.04, 12.
+int choose_streams(const StepTiles& st, int cap, int ncu) { return (long long)st.ngroups * cap > 4LL * ncu ? 2 : 1; }
 
 void check_slot(opf_ctx* c, int slot) {
   if (!c) throw OpfError(OPF_ERR_ARG, "null context");
@@ -669,7 +681,6 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   c->tiles = choose_tiles(c->Z, c->T, M);
   const Tuned tuned = lookup_tuning(N, K, M, cap);
   c->use_graph = tuned.graph;
-  c->use_streams = tuned.streams > 0 ? tuned.streams : 2;
   {
     // narrower transform tiles than the defaults (the kernels hold at most
     // the default width) from the caller or the table
@@ -699,6 +710,7 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
     HIPCHK(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     const int gp = gp_req > 0 ? gp_req : (e1 ? std::atoi(e1) : tuned.gp);
     c->st = choose_step_tiles(N, c->P, cap, ncu, gp, (size_t)lds);
+    c->use_streams = tuned.streams > 0 ? tuned.streams : choose_streams(c->st, cap, ncu);
     if (c->st.smem > 64 * 1024)   // dynamic LDS beyond 64 KiB is requested per kernel
       HIPCHK(hipFuncSetAttribute((const void*)step_kernel(N, c->st.gp), hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)c->st.smem));

@@ -29,8 +29,6 @@ WORKLOADS = [
     (48, 48, 24, 1, 3000.0, 1.25, 0.01, 100),
     (64, 64, 48, 1, 5300.0, 0.5, 0.005, 100),
     (96, 256, 128, 1, 5300.0, 0.4, 0.0025, 10),
-    (32, 24, 12, 8, 2400.0, 1.25, 0.01, 100),     # a server's blocks
-    (48, 48, 24, 4, 3000.0, 1.25, 0.01, 50),
     (32, 24, 12, 64, 2400.0, 1.25, 0.01, 40),
     (48, 48, 24, 32, 3000.0, 1.25, 0.01, 20),
     (64, 64, 48, 16, 5300.0, 0.5, 0.005, 10),
@@ -77,7 +75,7 @@ def tune(wl, log=print):
     os.environ["OPF_TUNING"] = "none"       # the built-in shape, not an older table's
     states = _states(N, K, M, alpha, cap, host_mesh(N))
     probe = Context(N, K, M, capacity=cap)
-    base = probe.tile_config() + (0, 2 if cap >= 4 else 1)
+    base = probe.tile_config() + (0, probe.launch_mode()["streams"])
     # a grid whose evaluation is the whole-plane kernel has no transform
     # tiles to choose
     probe.setup(0, Re, alpha, dt)
@@ -153,10 +151,14 @@ def main(argv=None):
     with open(args.out, "w") as f:
         f.write("# launch shapes of the time step chosen by opf/autotune.py (python -m opf.autotune)\n")
         f.write(f"# measured {datetime.date.today().isoformat()} on one MI355X (gfx950); opf_ctx_create takes the\n")
-        f.write("# row of its (N, K, M) with the largest min_capacity not above its capacity\n")
+        f.write("# row of its (N, K, M) with the largest min_capacity not above its capacity; zeros leave a\n")
+        f.write("# shape to the built-in choice, from twice the capacity that the row before was measured at\n")
         f.write("# N K M min_capacity pairs tm tz graph streams us_per_state_step default_us_per_state_step\n")
+        keys = {key for key, *_ in rows}
         for (N, K, M, cap), (p, tm, tz, g, ns), c, c0 in sorted(rows):
             f.write(f"{N} {K} {M} {cap} {p} {tm} {tz} {g} {ns} {c * 1e6:.3f} {c0 * 1e6:.3f}\n")
+            if (N, K, M, 2 * cap) not in keys:
+                f.write(f"{N} {K} {M} {2 * cap} 0 0 0 0 0\n")
     print(f"wrote {args.out}", flush=True)
     return 0
 

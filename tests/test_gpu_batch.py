@@ -225,3 +225,23 @@ def test_ensemble_512_states():
         assert np.array_equal(alone.diag(0), ctx.diag(s)), s
         alone.close()
     ctx.close()
+
+
+def test_tuned_shapes_hold_where_they_were_measured(monkeypatch):
+    """A row of the committed table holds below twice the capacity it was measured
+    at; beyond, contexts have the built-in shapes, whose number of streams
+    follows how full the slots make the chip (256 CUs)."""
+    import opf
+    for (n, k, m, cap, streams) in ((48, 48, 24, 2, 1), (48, 48, 24, 4, 2), (32, 24, 12, 8, 1), (32, 24, 12, 16, 2),
+                                    (64, 64, 48, 4, 2), (24, 16, 8, 32, 1)):
+        shapes = []
+        for table in (None, "none"):
+            if table:
+                monkeypatch.setenv("OPF_TUNING", table)
+            else:
+                monkeypatch.delenv("OPF_TUNING", raising=False)
+            with opf.Context(n, k, m, capacity=cap) as ctx:
+                mode = ctx.launch_mode()
+                shapes.append((ctx.tile_config(), mode["graph"], mode["streams"]))
+        assert shapes[0] == shapes[1], (n, k, m, cap)
+        assert shapes[1][2] == streams, (n, k, m, cap)
