@@ -384,11 +384,13 @@ void launch_step(opf_ctx* c, int s0, int ns) {
          c->st, s0);
 }
 
-// vel_matrices for slots s0 .. s0+ns-1 (gate: k_matrices_t)
-void launch_matrices(opf_ctx* c, int s0, int ns, int gate) {
-  launch(c, "matrices", matrices_kernel(c->N), dim3((c->P + 7) / 8, 1, ns), dim3(256), matrices_smem(c->N), c->G, c->B,
+// vel_matrices for slots s0 .. s0+ns-1 of B, c->B unless the launch is of a slot
+// whatever list c->B.smap holds (gate: k_matrices_t)
+void launch_matrices(opf_ctx* c, int s0, int ns, int gate, const Bufs& B) {
+  launch(c, "matrices", matrices_kernel(c->N), dim3((c->P + 7) / 8, 1, ns), dim3(256), matrices_smem(c->N), c->G, B,
          s0, gate);
 }
+void launch_matrices(opf_ctx* c, int s0, int ns, int gate) { launch_matrices(c, s0, ns, gate, c->B); }
 
 // One iteration.  With adaptive slots, the predictor's evaluation is
 // followed by vel_maxtstep + tim_new_tstep and, where dt changed,
@@ -605,8 +607,6 @@ void launch_nonnewtonian(opf_ctx* c, int slot) {
   visc_add(c, slot, P);
 }
 
-void launch_matrices(opf_ctx* c, int s0, int ns, int gate);
-
 // util(2) of the LES plugin for one slot (LES.f90:100-320): get_nu with the
 // slot's eddy-viscosity model, update_nu_r before a predictor (vel_matrices
 // on the device where vel_nu changed), update_nonlin_terms.
@@ -624,7 +624,9 @@ void launch_les(opf_ctx* c, int slot) {
   launch(c, "les_visc", k_les_visc, gp, b256, 0, P, np, c->N, c->Z * c->T, q.model, q.Cs, dz, (const double*)D,
          c->lesMax + slot);
   launch(c, "les_nur", k_les_nur, dim3(1), dim3(1), 0, c->B, slot, (const unsigned long long*)c->lesMax);
-  launch_matrices(c, slot, 1, 1);
+  Bufs B = c->B;
+  B.smap = nullptr;   // `slot` is a slot, also in a compacted iteration
+  launch_matrices(c, slot, 1, 1, B);
   visc_derivatives(c, slot, P);
   launch(c, "les_force", k_les_force, gp, b256, 0, P, np, c->B, slot);
   visc_add(c, slot, P);

@@ -289,3 +289,32 @@ def test_viscosity_plugins_match_reference_plugin_runs(name):
     rs = g["series"]
     assert np.max(np.abs(d[:, 2] - rs[:, 2]) / rs[:, 2]) <= 1e-10
     assert np.all(d[:, 8] == 1)
+
+
+def test_les_slots_of_different_lengths_do_not_disturb_each_other():
+    """Two LES slots with 2 and 9 steps in one call, beside a slot without a
+    plugin: each ends with the bits of a run of its own, vel_nu's refactored
+    matrices included."""
+    import opf
+    N, K, M, Re, alpha, dt = 16, 6, 4, 2400.0, 1.25, 0.01
+    states = [_seeded(N, K, M, 1, alpha, 11 + s, e) for s, e in enumerate((1e-2, 3e-2, 1e-3))]
+    ndts = (2, 9, 5)
+
+    def les(ctx, slot, s):
+        if s < 2:
+            ctx.les(slot, model=1, C_s=0.1, filter=1, A_plus=25.0)
+
+    ctx = opf.Context(N, K, M, capacity=3)
+    for s in range(3):
+        ctx.setup(s, Re, alpha, dt)
+        les(ctx, s, s)
+        ctx.put_state(s, *states[s])
+    ctx.steporbit([0, 1, 2], ndts, [n * dt for n in ndts], 0.0, 0.0)
+    for s in range(3):
+        one = opf.Context(N, K, M)
+        one.setup(0, Re, alpha, dt)
+        les(one, 0, s)
+        one.put_state(0, *states[s])
+        one.steporbit([0], ndts[s], ndts[s] * dt, 0.0, 0.0)
+        for a, b in zip(ctx.get_state(s)[:3], one.get_state(0)[:3]):
+            assert np.array_equal(a, b), s
