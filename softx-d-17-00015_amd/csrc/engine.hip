@@ -207,7 +207,7 @@ FftTiles choose_tiles(int Z, int T, int M) {
   t.pt = make_plan(T);
   // a workgroup transforms at most FFT_TILE complex values: tm columns of
   // length Z, or 3*tz packed lines of length T
-  if (Z > FFT_TILE || 3 * T > FFT_TILE) throw OpfError(OPF_ERR_ARG, "transform length too large for the FFT tiles");
+  if (Z > FFT_TILE || T > THETA_MAX) throw OpfError(OPF_ERR_ARG, "transform length too large for the FFT tiles");
   t.tm = std::max(1, std::min(M, tile_m(Z)));
   t.tz = std::max(1, std::min(Z, FFT_TILE / (3 * T)));
   if (t.tz == 1 && Z >= 2 && 2 * T <= THETA_ITEMS) t.tz = 2;   // long theta lines

@@ -107,6 +107,7 @@ __host__ __device__ constexpr size_t step_lds_doubles(int N, int gp) {
 
 constexpr int FFT_THREADS = 256;
 constexpr int FFT_TILE = 2048;   // complex values per transform workgroup (all its lines)
+constexpr int THETA_MAX = FFT_TILE / 3;   // longest theta line: its three packed transforms fill a tile
 // items (line, theta point) one theta workgroup holds in registers: FFT_TILE / 3
 // rounded up to whole rounds of FFT_THREADS (768).  Lines of 3M > FFT_TILE / 2
 // would leave one line per workgroup under FFT_TILE; they take two lines

@@ -1515,7 +1515,8 @@ struct LenKerns {
   int ln, bt;   // threads and transforms (two lines each) of the line kernels
   size_t zfs, zbs, ts, c2rs, r2cs;
 };
-// passes (first, middle or 1, last) of the z kernels and of the theta kernel
+// passes (first, middle or 1, last) of the z kernels and of the theta kernel (up
+// to the longest theta line that contexts take)
 template <int ZF, int ZM, int ZL, int TF = ZF, int TM = ZM, int TL = ZL>
 LenKerns kerns_of() {
   static_assert(TF * TM * TL == ZF * ZM * ZL, "one length");
@@ -1526,22 +1527,24 @@ LenKerns kerns_of() {
   k.L = ZF * ZM * ZL;
   k.zfwd = k_zfwd_t<ZF, ZM, ZL>;
   k.zbwd = k_zbwd_t<ZF, ZM, ZL>;
-  k.theta = k_theta_t<TF, TM, TL>;
   k.zfwd1 = k_zfwd_one_t<ZF, ZM, ZL>;
   k.zbwd1 = k_zbwd_one_t<ZF, ZM, ZL>;
-  k.c2r = k_c2r_lines_t<TF, TM, TL>;
-  k.r2c = k_r2c_lines_t<TF, TM, TL>;
   k.zn = ZT::NT;
   k.tm = ZT::TM;
-  k.tn = TT::NT;
-  k.tz = TT::TZ;
-  k.ln = LT::NT;
-  k.bt = LT::TM;
   k.zfs = ZT::smem_f;
   k.zbs = ZT::smem_b;
-  k.ts = TT::smem;
-  k.c2rs = LT::smem_b;
-  k.r2cs = LT::smem_b + (size_t)LT::TM * ((2 * (k.L / 3) - 1) | 1) * sizeof(double2);
+  if constexpr (TF * TM * TL <= THETA_MAX) {
+    k.theta = k_theta_t<TF, TM, TL>;
+    k.c2r = k_c2r_lines_t<TF, TM, TL>;
+    k.r2c = k_r2c_lines_t<TF, TM, TL>;
+    k.tn = TT::NT;
+    k.tz = TT::TZ;
+    k.ln = LT::NT;
+    k.bt = LT::TM;
+    k.ts = TT::smem;
+    k.c2rs = LT::smem_b;
+    k.r2cs = LT::smem_b + (size_t)LT::TM * ((2 * (k.L / 3) - 1) | 1) * sizeof(double2);
+  }
   return k;
 }
 }  // namespace
@@ -1609,7 +1612,7 @@ FftKerns fft_kernels(const FftPlan& pz, const FftPlan& pt, const FftTiles& t, in
     const int w = std::min(t.tm, z->tm), g = (M + w - 1) / w;
     k.t.tm = (M + g - 1) / g;
   }
-  if (const LenKerns* z = find(pt.L)) {
+  if (const LenKerns* z = find(pt.L); z && z->theta) {
     k.theta = z->theta;
     k.c2r = z->c2r;
     k.r2c = z->r2c;
