@@ -290,6 +290,7 @@ struct Seq {
   static constexpr int L = F * MID * LA, JF = L / F, JM = L / MID, JL = L / LA;
   static constexpr int P1 = F | 1, P2 = (F * MID) | 1, PL = MID > 1 ? P2 : P1;
   static constexpr int SIZE = JF * P1 > (MID > 1 ? LA * P2 : 0) ? JF * P1 : LA * P2;
+  static_assert(JF * P1 <= SIZE && LA * PL <= SIZE && F <= P1 && JL <= PL, "each pass' table within the transform's part");
 };
 // the smallest size >= n with size % 8 == r: the distance of two transforms in
 // LDS, such that the lanes of a few transforms share no bank
@@ -877,8 +878,14 @@ struct PlaneTile {
   static constexpr int DS = S::SIZE | 1, DI = I::SIZE | 1, DO = (2 * M - 1) | 1;
   static constexpr int NTR = Z + Z / 2, OUT = NTR * DI;
   static constexpr int mx(int a, int b) { return a > b ? a : b; }
-  static constexpr int BUF = mx(mx(6 * M * mx(DZ, DY), 3 * Z * DS), mx(OUT, 3 * M * DZ) + NTR * DO);
+  // the retained bins stand behind both the tables of the transforms back that
+  // they are read from and the z columns that they are read into
+  static constexpr int BINS = mx(OUT, 3 * M * DZ);
+  static constexpr int BUF = mx(mx(6 * M * mx(DZ, DY), 3 * Z * DS), BINS + NTR * DO);
   static constexpr size_t smem = (size_t)(BUF + Z + TT) * sizeof(double2);
+  static_assert(BINS >= NTR * DI && BINS >= 3 * M * DZ && BUF >= 3 * Z * DS && BUF >= 6 * M * DY && 2 * M - 1 <= DO,
+                "the tables of a stage");
+  static_assert(smem <= 160 * 1024, "the LDS of a CU");
 };
 template <int ZF, int ZL, int TF, int TL>
 __global__ void __launch_bounds__(PLANE_THREADS) k_plane_t(Geo G, Bufs B, FftTiles, int slot0) {
@@ -988,7 +995,7 @@ __global__ void __launch_bounds__(PLANE_THREADS) k_plane_t(Geo G, Bufs B, FftTil
   if ((B.prm[slot].adaptive && c->mode == MODE_PRED) || c->host_driven) plane_maxima<NT, true>(mr, mt, mz, mx, G.N);
   else if (tid < 3) mx[(size_t)tid * G.N] = 0ull;
   __syncthreads();
-  double2* out = buf + C::mx(C::OUT, 3 * M * C::DZ);
+  double2* out = buf + C::BINS;
   constexpr int N5 = C::NTR * I::JL;
 #pragma unroll
   for (int q0 = 0; q0 < N5; q0 += NT) {

@@ -55,8 +55,8 @@ struct BlkLane {
 struct BlkSweep {
   int NB, S, d;        // blocks; steps of either side; 1: side 1 has one block less (its step 0 is empty)
   int t0, dt;          // block of step i: t0 + i dt (step 0 of an empty first step clamped by the callers)
-  __device__ static BlkSweep make(int N, int side) {
-    BlkSweep s;
+  __host__ __device__ static constexpr BlkSweep make(int N, int side) {
+    BlkSweep s{};
     s.NB = blk_count(N);
     s.S = blk_mid(N);
     s.d = 1 - (s.NB & 1);
@@ -64,8 +64,37 @@ struct BlkSweep {
     s.dt = side ? -1 : 1;
     return s;
   }
-  __device__ __forceinline__ int first(int side) const { return side ? NB - 1 : 0; }
+  __host__ __device__ __forceinline__ constexpr int first(int side) const { return side ? NB - 1 : 0; }
 };
+
+// The sweeps take every block once, the middle one last, and stay within the
+// table (rows 0 .. N + 7) and the right-hand sides (rows 0 .. N + 3), for every N
+// of a context.
+constexpr bool blk_sweeps_cover() {
+  for (int N = 9; N <= MAXN; ++N) {
+    bool seen[blk_count(MAXN)] = {};
+    const int mid = blk_mid(N);
+    for (int side = 0; side < 2; ++side) {
+      const BlkSweep w = BlkSweep::make(N, side);
+      if (w.S != mid || 4 * w.NB + 4 > N + 8) return false;
+      for (int i = 0; i < w.S; ++i) {
+        const int t = w.t0 + i * w.dt;
+        const int f = t + w.dt;   // table rows 4 f .. of the forward sweep, 4 t .. of the backward one
+        if (f < 0 || f > w.NB || t < 0 || t > w.NB) return false;
+        const bool empty = side && w.d && i == 0;
+        if (empty != (t == w.NB)) return false;
+        if (empty) continue;
+        if (seen[t] || t == mid) return false;
+        seen[t] = true;
+        if (i == w.S - 1 && f != mid) return false;
+      }
+    }
+    for (int t = 0; t < blk_count(N); ++t)
+      if (seen[t] == (t == mid)) return false;
+  }
+  return true;
+}
+static_assert(blk_sweeps_cover(), "blocks of the two sides");
 
 // The inverses of NG groups of two matrices: steps 0 .. S-1, then the middle
 // block in e[g][SM].  SM >= S.
