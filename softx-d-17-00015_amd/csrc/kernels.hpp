@@ -154,9 +154,8 @@ __global__ void k_les_visc(NnPhys P, size_t np, int N, int ZT, int model, double
                            unsigned long long* numax_slot);
 __global__ void k_les_nur(Bufs B, int slot, const unsigned long long* numax);
 __global__ void k_les_force(NnPhys P, size_t np, Bufs B, int slot);
-__global__ void k_add_coll(Geo G, double2* dst, const double2* src);
 __global__ void k_rows_to_planes(Geo G, const double2* rows, double* planes);
-__global__ void k_planes_to_rows(Geo G, const double* planes, double2* rows);
+template <bool ADD> __global__ void k_planes_to_rows(Geo G, const double* planes, double2* rows);
 // var_coll_norm of a field in the coll layout: per-harmonic partials b[H], then [E, Ek, Em]
 __global__ void k_norm_harm(Geo G, const SlotParams* prm, const double* re, const double* im, double* b);
 __global__ void k_norm_sum(Geo G, const double* b, double* out);

@@ -563,19 +563,6 @@ __global__ void __launch_bounds__(64) k_lu_factor(Geo G, Bufs B, LuFactors L, in
 }
 
 // ---------------------------------------------------------------------------
-// dst += src on one coll component (harmonics 0..H-1 of every radial row):
-// forcing terms added to vel_N* by var_null(2) hooks.  grid: x = H/64, y = N.
-// ---------------------------------------------------------------------------
-__global__ void k_add_coll(Geo G, double2* dst, const double2* src) {
-  const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n = blockIdx.y;
-  if (h >= G.H || n >= G.N) return;
-  const size_t o = (size_t)n * G.Hp + h;
-  const double2 a = dst[o], b = src[o];
-  dst[o] = make_double2(a.x + b.x, a.y + b.y);
-}
-
-// ---------------------------------------------------------------------------
 // Device rows u[comp][n][Hp] <-> the reference's coll planes, of a component
 // re[h][n] then im[h][n] (r fastest), through LDS tiles of 32 x 32 so that both
 // sides move whole lines.  The host's loops over both layouts took 100 ms for
@@ -601,6 +588,8 @@ __global__ void __launch_bounds__(256) k_rows_to_planes(Geo G, const double2* __
       planes[nh + o] = v.y;
     }
 }
+// ADD: onto the rows (forcing added to vel_N* by var_null(2) hooks), of the H harmonics
+template <bool ADD>
 __global__ void __launch_bounds__(256) k_planes_to_rows(Geo G, const double* __restrict__ planes,
                                                         double2* __restrict__ rows) {
   __shared__ double2 t[32][33];
@@ -615,8 +604,15 @@ __global__ void __launch_bounds__(256) k_planes_to_rows(Geo G, const double* __r
   }
   __syncthreads();
   for (int i = hi; i < 32; i += 8)
-    if (n0 + i < G.N && h0 + lo < G.Hp) rows[(size_t)(n0 + i) * G.Hp + h0 + lo] = t[i][lo];
+    if (n0 + i < G.N && h0 + lo < (ADD ? G.H : G.Hp)) {
+      double2 v = t[i][lo];
+      double2* r = rows + (size_t)(n0 + i) * G.Hp + h0 + lo;
+      if (ADD) v = make_double2(r->x + v.x, r->y + v.y);
+      *r = v;
+    }
 }
+template __global__ void k_planes_to_rows<false>(Geo, const double*, double2*);
+template __global__ void k_planes_to_rows<true>(Geo, const double*, double2*);
 
 // ---------------------------------------------------------------------------
 // var_coll_norm (variables.f90:718-751) of a field in the reference's coll

@@ -103,3 +103,33 @@ def test_load_onto_other_resolution_matches_host_reading_and_oracle(tmp_path):
     O.Ctx.imposesym0(*want)
     for c in range(3):
         assert np.array_equal(ud[c], want[c]), c
+
+
+# states of 6 N H doubles just below and above one pinned piece (4 MiB), a field
+# of one component around it, small and odd sizes
+@pytest.mark.parametrize("N,K,M", [(9, 3, 2), (33, 6, 4), (62, 27, 27), (63, 27, 27), (117, 32, 36), (104, 36, 36)])
+def test_fields_to_and_from_the_device_keep_their_bits(N, K, M):
+    """put_state / get_state, get_nonlinear after add_nonlinear of a field onto
+    zero terms, and a transform there and back, at either side of the size up to
+    which the kernels read and write the pinned planes themselves."""
+    import opf
+    rng = np.random.default_rng(N)
+    ctx = opf.Context(N, K, M)
+    ctx.setup(0, 2400.0, 1.25, 0.01)
+    u = [rng.standard_normal((N, ctx.H)) + 1j * rng.standard_normal((N, ctx.H)) for _ in range(3)]
+    u[0][:, 0] = 0.0                       # vel_imposesym's conditions on harmonic (0, 0)
+    for f in u[1:]:
+        f[:, 0] = f[:, 0].real
+    ctx.put_state(0, *u)
+    for a, b in zip(ctx.get_state(0), u):
+        assert np.array_equal(a, b)
+    before = ctx.get_nonlinear(0)          # no evaluation yet: the base-flow terms alone
+    add = [np.round(rng.standard_normal((N, ctx.H)) * 8.0) + 0j for _ in range(3)]
+    ctx.add_nonlinear(0, *add)
+    for a, b, d in zip(ctx.get_nonlinear(0), before, add):
+        # the base-flow terms, a few hundred, are summed onto zero and onto whole numbers
+        assert np.abs(a - (b + d)).max() <= 1e-12
+    for a, b in zip(ctx.get_state(0), u):
+        assert np.array_equal(a, b)
+    back = ctx.phys2coll(ctx.coll2phys(u[2]))
+    assert np.abs(back - u[2]).max() <= 1e-12 * np.abs(u[2]).max()
