@@ -125,7 +125,9 @@ struct opf_ctx {
   double* dterrHost = nullptr;   // pinned: tim_dterr of the last host-driven call (first use)
   SlotParams* prmHost = nullptr; // pinned parameters of asynchronous admissions (first use)
   std::vector<LuFactors> lu;     // LAPACK-form factors [slot][4] (first use)
-  int* luVerdict = nullptr;      // tim_lumesh_init: a zero pivot; blocks that cannot represent the set (first use)
+  int* luVerdict = nullptr;      // tim_lumesh_init: a zero pivot; blocks that cannot represent the set (pinned, first use)
+  long mat_gen = 1;              // counts the launches that may change a factor set
+  std::vector<long> lu_gen;      // its value when the factors of a set [slot][4] were last asked for
   std::vector<int> lu_unsafe;    // the latter per factor set [slot][4]
   int n_unsafe = 0;              // and how many
   std::vector<int> lu_bc;        // BC of each factor set [slot][4] (tim_lumesh_invert's (0,0) rule)
@@ -387,6 +389,7 @@ void launch_step(opf_ctx* c, int s0, int ns) {
 // vel_matrices for slots s0 .. s0+ns-1 of B, c->B unless the launch is of a slot
 // whatever list c->B.smap holds (gate: k_matrices_t)
 void launch_matrices(opf_ctx* c, int s0, int ns, int gate, const Bufs& B) {
+  ++c->mat_gen;
   launch(c, "matrices", matrices_kernel(c->N), dim3((c->P + 7) / 8, 1, ns), dim3(256), matrices_smem(c->N), c->G, B,
          s0, gate);
 }
@@ -418,6 +421,14 @@ void launch_iteration(opf_ctx* c, int s0, int ns) {
   launch_step(c, s0, ns);
 }
 
+int* lu_verdict(opf_ctx* c) {
+  if (!c->luVerdict) {
+    HIPCHK(hipHostMalloc((void**)&c->luVerdict, 2 * sizeof(int), hipHostMallocDefault));
+    c->luVerdict[0] = c->luVerdict[1] = 0;
+  }
+  return c->luVerdict;
+}
+
 // The LAPACK-form factors of one factor set, for tim_lumesh_get and
 // tim_lumesh_invert: built from the matrix the set holds when they are asked
 // for (the time step does not read them), where they are not there yet.  Buffers
@@ -432,8 +443,12 @@ const LuFactors& lapack_factors(opf_ctx* c, int slot, int which) {
     L.pv = (unsigned char*)(L.F + cols * LUS + (groups + 1) / 2);
     HIPCHK(hipMemcpy(&c->B.sets[(size_t)slot * 4 + which].lu, &L, sizeof L, hipMemcpyHostToDevice));
   }
-  if (!c->luVerdict) c->luVerdict = c->alloc<int>(2);
-  launch(c, "lapack_factor", k_lu_factor, dim3((unsigned)groups), dim3(64), 0, c->G, c->B, L, slot, which, c->luVerdict);
+  long& gen = c->lu_gen[(size_t)slot * 4 + which];
+  if (gen != c->mat_gen) {   // no launch since then may have changed the set
+    launch(c, "lapack_factor", k_lu_factor, dim3((unsigned)groups), dim3(64), 0, c->G, c->B, L, slot, which,
+           lu_verdict(c));
+    gen = c->mat_gen;
+  }
   return L;
 }
 
@@ -841,6 +856,7 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   c->occupied.assign(cap, 0);
   c->setup.assign(cap, 0);
   c->lu.assign((size_t)cap * 4, LuFactors{});
+  c->lu_gen.assign((size_t)cap * 4, 0);
   c->lu_unsafe.assign((size_t)cap * 4, 0);
   c->lu_bc.assign((size_t)cap * 4, 0);
   for (int i = 0; i < cap; ++i) c->lu_bc[(size_t)i * 4 + MAT_LNP] = 1;
@@ -1015,6 +1031,7 @@ void enqueue_iterations(opf_ctx* c, int s0, int ns, long iterations) {
     ++c->graph_captures;
   }
   const long reps = iterations / gi;
+  ++c->mat_gen;   // replays launch what their capture did
   for (long i = 0; i < reps; ++i) HIPCHK(hipGraphLaunch(c->gexec, c->stream));
   for (long i = reps * gi; i < iterations; ++i) launch_iteration(c, s0, ns);
   c->graph_launches += reps;
@@ -1296,6 +1313,7 @@ int opf_ctx_destroy(opf_ctx* c) {
   if (c->stream2) (void)hipStreamDestroy(c->stream2);
   if (c->prmHost) (void)hipHostFree(c->prmHost);
   if (c->dterrHost) (void)hipHostFree(c->dterrHost);
+  if (c->luVerdict) (void)hipHostFree(c->luVerdict);
   for (int b = 0; b < 2; ++b) {
     if (c->stage[b]) (void)hipHostFree(c->stage[b]);
     if (c->stage_ev[b]) (void)hipEventDestroy(c->stage_ev[b]);
@@ -1888,9 +1906,9 @@ int opf_tim_lumesh_get(opf_ctx* c, int slot, int which, double* ab, int* ipiv) {
     // per-pair blocks [pair][n][LUS] and [pair][n]
     std::vector<double> F((size_t)P * N * LUS);
     std::vector<unsigned char> pv((size_t)P * N);
+    HIPCHK(hipMemcpyAsync(F.data(), L.F, F.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(pv.data(), L.pv, pv.size(), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(F.data(), L.F, F.size() * sizeof(double), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(pv.data(), L.pv, pv.size(), hipMemcpyDeviceToHost));
     for (int hh = 0; hh < H; ++hh) {
       int k, m;
       if (hh < c->K) { m = 0; k = hh; }
@@ -1938,23 +1956,26 @@ extern "C" int opf_tim_lumesh_init(opf_ctx* c, int slot, int which, int PM, int 
     if (PM < -1 || PM > 1 || BC < 0 || BC > 1) throw OpfError(OPF_ERR_ARG, "PM must be -1, 0, 1 and BC 0 or 1");
     if (!c->setup[slot]) throw OpfError(OPF_ERR_STATE, "slot not set up (alpha unknown)");
     auto ctl = read_ctl(c);
-    ctl[slot].status = 0;
-    write_ctl(c, ctl);
-    int verdict[2] = {0, 0};
-    if (!c->luVerdict) c->luVerdict = c->alloc<int>(2);
-    HIPCHK(hipMemcpy(c->luVerdict, verdict, sizeof verdict, hipMemcpyHostToDevice));
+    if (ctl[slot].status != 0) {
+      ctl[slot].status = 0;
+      write_ctl(c, ctl);
+    }
+    ++c->mat_gen;
+    int* verdict = lu_verdict(c);
+    verdict[0] = verdict[1] = 0;
     launch(c, "factor", k_block_factor, dim3((c->P + 31) / 32), dim3(64), 0, c->G, c->B, slot,
-           LuSpec{which, PM, BC, c1, c2}, c->luVerdict + 1);
+           LuSpec{which, PM, BC, c1, c2}, verdict + 1);
     lapack_factors(c, slot, which);   // DGBTF2's own verdict on a singular matrix
     HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(verdict, c->luVerdict, sizeof verdict, hipMemcpyDeviceToHost));
     c->lu_bc[(size_t)slot * 4 + which] = BC;
     if (verdict[0]) throw OpfError(OPF_ERR_SINGULAR, "tim_lumesh_init");
     // a set that needs row interchanges across blocks: the slot's steps solve
     // with the LAPACK-form factors of all four sets
-    set_unsafe(c, slot, which, verdict[1]);
     const int* unsafe = &c->lu_unsafe[(size_t)slot * 4];
+    const int before = unsafe[0] | unsafe[1] | unsafe[2] | unsafe[3];
+    set_unsafe(c, slot, which, verdict[1]);
     const int banded = unsafe[0] | unsafe[1] | unsafe[2] | unsafe[3];
+    if (!banded && !before) return;
     if (banded)
       for (int q = 0; q < 4; ++q) lapack_factors(c, slot, q);
     HIPCHK(hipStreamSynchronize(c->stream));
