@@ -1850,8 +1850,7 @@ int opf_get_phys(opf_ctx* c, int slot, int which, double* phys) {
     launch_zfwd_one(c, src, c->tY, 1);
     launch(c, "c2r", k_theta_c2r, dim3((c->Z + 1) / 2, c->N, 1), dim3(FFT_THREADS),
            (padded_len(c->T) + c->T) * sizeof(double2), c->G, c->B, t, (const double2*)c->tY, c->tP);
-    HIPCHK(hipMemcpyAsync(phys, c->tP, sizeof(double) * c->N * c->Z * c->T, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    planes_to_host(c, c->tP, &phys, 1, (size_t)c->N * c->Z * c->T);
   });
 }
 
@@ -1877,8 +1876,7 @@ int opf_tra_coll2phys(opf_ctx* c, const double* cre, const double* cim, double* 
     launch_zfwd_one(c, c->tC, c->tY, 1);
     launch(c, "c2r", k_theta_c2r, dim3((c->Z + 1) / 2, c->N, 1), dim3(FFT_THREADS), (padded_len(c->T) + c->T) * sizeof(double2), c->G,
            c->B, t, (const double2*)c->tY, c->tP);
-    HIPCHK(hipMemcpyAsync(phys, c->tP, sizeof(double) * c->N * c->Z * c->T, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    planes_to_host(c, c->tP, &phys, 1, (size_t)c->N * c->Z * c->T);
   });
 }
 
@@ -1886,7 +1884,7 @@ int opf_tra_phys2coll(opf_ctx* c, const double* phys, double* cre, double* cim) 
   return guard([&] {
     if (!c || !phys) throw OpfError(OPF_ERR_ARG, "null argument");
     ensure_temps(c);
-    HIPCHK(hipMemcpyAsync(c->tP, phys, sizeof(double) * c->N * c->Z * c->T, hipMemcpyHostToDevice, c->stream));
+    planes_to_dev(c, c->tP, &phys, 1, (size_t)c->N * c->Z * c->T);
     const FftTiles& t = c->tiles;
     HIPCHK(hipMemsetAsync(c->tC, 0, sizeof(double2) * c->G.coll, c->stream));
     launch(c, "r2c", k_theta_r2c, dim3((c->Z + 1) / 2, c->N, 1), dim3(FFT_THREADS), (padded_len(c->T) + c->T) * sizeof(double2), c->G,

@@ -597,10 +597,17 @@ __global__ void __launch_bounds__(256) k_planes_to_rows(Geo G, const double* __r
   const size_t nh = (size_t)G.N * G.H;
   rows += blockIdx.z * G.coll;
   planes += blockIdx.z * 2 * nh;
-  for (int i = hi; i < 32; i += 8) {
-    const size_t o = (size_t)(h0 + i) * G.N + n0 + lo;
-    const bool in = n0 + lo < G.N && h0 + i < G.H;
-    t[lo][i] = in ? make_double2(planes[o], planes[nh + o]) : make_double2(0.0, 0.0);
+  double re[4], im[4];   // all loads in one batch: the planes may be host memory
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const size_t o = (size_t)min(h0 + hi + 8 * q, G.H - 1) * G.N + min(n0 + lo, G.N - 1);
+    re[q] = planes[o];
+    im[q] = planes[nh + o];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int i = hi + 8 * q;
+    t[lo][i] = n0 + lo < G.N && h0 + i < G.H ? make_double2(re[q], im[q]) : make_double2(0.0, 0.0);
   }
   __syncthreads();
   for (int i = hi; i < 32; i += 8)
