@@ -77,8 +77,10 @@ int opf_ctx_dims(const opf_ctx* ctx, int* N, int* K, int* M, int* Mp, int* H, in
  * (admission control).  Allocated later, on first use: the shift tables
  * ((2K + M) * 16 bytes per slot), and for opf_tim_lumesh_get /
  * _invert / _init the LAPACK-form factors of the set (K*M*(129*N + 1) bytes), and
- * for opf_slot_nonnewtonian / opf_slot_les 16 physical fields of N*3K*3M doubles, 4 spectral fields and
- * 3 fields of N*3K*M complex values per context, and 4N + 1 words per slot. */
+ * for opf_slot_nonnewtonian / opf_slot_les 16 physical fields of N*3K*3M doubles, 9 spectral fields (N*Hp
+ * complex values, Hp = H rounded up to 64) and 9 fields of N*Z*M complex values (Z = 3K rounded up to 4) per
+ * context, with the granular transforms' one of each kind (also opf_get_phys, opf_tra_*), and 4N + 1 words
+ * per slot. */
 size_t opf_ctx_bytes_needed(int N, int K, int M, int capacity);
 
 /* mes_D of meshs.f90:48-58: r(1:N), intrdr(1:N), dr0(1:5,0:4), dr1(1:5,0:4)

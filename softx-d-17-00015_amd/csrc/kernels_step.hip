@@ -15,10 +15,10 @@
 #include "kernels.hpp"
 #include "solve.hpp"
 
-// Products and sums are rounded separately, as in the reference's Fortran
-// (built for x86-64 without FMA): the ill-conditioned Neumann pressure solve
-// then reproduces the reference's rounding instead of amplifying the
-// difference a fused multiply-add makes.
+// Sums round as they are written: separately, as in the reference's Fortran
+// (built for x86-64 without FMA), in the LAPACK-form factors, the 4x4 inverses,
+// the shifts and the norms, which then agree with it to the last bit or nearly;
+// fused where fma() stands, in the block elimination and the curl.
 #pragma clang fp contract(off)
 
 namespace opf {
