@@ -85,7 +85,8 @@ struct opf_ctx {
   Bufs B{};
   Geo G{};
   FftTiles tiles{};
-  StepTiles st{};
+  StepTiles st{};              // launches of several slots
+  StepTiles st1{};             // and of one, which leaves the chip emptier
 
   FftKerns fk{};
   PlaneKern plane = nullptr;   // whole-plane evaluation, where the grid has one
@@ -125,9 +126,9 @@ struct opf_ctx {
   double* dterrHost = nullptr;   // pinned: tim_dterr of the last host-driven call (first use)
   SlotParams* prmHost = nullptr; // pinned parameters of asynchronous admissions (first use)
   std::vector<LuFactors> lu;     // LAPACK-form factors [slot][4] (first use)
-  int* luVerdict = nullptr;      // tim_lumesh_init: a zero pivot; blocks that cannot represent the set (pinned, first use)
   long mat_gen = 1;              // counts the launches that may change a factor set
   std::vector<long> lu_gen;      // its value when the factors of a set [slot][4] were last asked for
+  int* luVerdict = nullptr;      // tim_lumesh_init: a zero pivot; blocks that cannot represent the set (pinned, first use)
   std::vector<int> lu_unsafe;    // the latter per factor set [slot][4]
   int n_unsafe = 0;              // and how many
   std::vector<int> lu_bc;        // BC of each factor set [slot][4] (tim_lumesh_invert's (0,0) rule)
@@ -381,9 +382,9 @@ void launch_step(opf_ctx* c, int s0, int ns) {
            st, s0);
     return;
   }
-  const int per = (c->st.ngroups + 7) / 8;   // XCD-aware order inside the kernel
-  launch(c, "step", step_kernel(c->N, c->st.gp), dim3(8 * per, 1, ns), dim3(step_threads(c->st.gp)), c->st.smem, c->G, c->B,
-         c->st, s0);
+  const StepTiles& st = ns == 1 ? c->st1 : c->st;
+  const int per = (st.ngroups + 7) / 8;   // XCD-aware order inside the kernel
+  launch(c, "step", step_kernel(c->N, st.gp), dim3(8 * per, 1, ns), dim3(step_threads(st.gp)), st.smem, c->G, c->B, st, s0);
 }
 
 // vel_matrices for slots s0 .. s0+ns-1 of B, c->B unless the launch is of a slot
@@ -750,12 +751,14 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
     c->device = dev;
     HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     HIPCHK(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    const int gp = gp_req > 0 ? gp_req : (e1 ? std::atoi(e1) : tuned.gp);
-    c->st = choose_step_tiles(N, c->P, cap, ncu, gp, (size_t)lds);
+    const int gp = gp_req > 0 ? gp_req : e1 ? std::atoi(e1) : 0;
+    c->st = choose_step_tiles(N, c->P, cap, ncu, gp > 0 ? gp : tuned.gp, (size_t)lds);
+    c->st1 = choose_step_tiles(N, c->P, 1, ncu, gp > 0 ? gp : lookup_tuning(N, K, M, 1).gp, (size_t)lds);
     c->use_streams = tuned.streams > 0 ? tuned.streams : choose_streams(c->st, cap, ncu);
-    if (c->st.smem > 64 * 1024)   // dynamic LDS beyond 64 KiB is requested per kernel
-      HIPCHK(hipFuncSetAttribute((const void*)step_kernel(N, c->st.gp), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)c->st.smem));
+    for (const StepTiles* t : {&c->st, &c->st1})
+      if (t->smem > 64 * 1024)   // dynamic LDS beyond 64 KiB is requested per kernel
+        HIPCHK(hipFuncSetAttribute((const void*)step_kernel(N, t->gp), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)t->smem));
     // the whole-plane evaluation where the grid has one and its LDS fits
     // (OPF_PLANE=0: the three transform kernels instead)
     const char* e2 = std::getenv("OPF_PLANE");
