@@ -816,11 +816,9 @@ void create(opf_ctx* c, int N, int K, int M, int Mp, int cap, const double* r, i
   struct SlotSets {   // one buffer: an allocation takes about 0.1 ms
     FactorSet sets[4];
     LuSpec spec[4];
-    int banded, pad;
   };
   B.sets = (FactorSet*)c->alloc<SlotSets>(cap);
   B.spec = (LuSpec*)(B.sets + (size_t)cap * 4);
-  B.banded = (int*)(B.spec + (size_t)cap * 4);
   B.Uinf = c->alloc<double>((size_t)cap * 6 * N * s.P);
   B.Ainv = c->alloc<double>((size_t)cap * 16 * s.H);
   B.Ui = c->alloc<double>((size_t)cap * N);
@@ -1980,7 +1978,7 @@ extern "C" int opf_tim_lumesh_init(opf_ctx* c, int slot, int which, int PM, int 
     if (banded)
       for (int q = 0; q < 4; ++q) lapack_factors(c, slot, q);
     HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(c->B.banded + slot, &banded, sizeof banded, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(&c->B.sets[(size_t)slot * 4].banded, &banded, sizeof banded, hipMemcpyHostToDevice));
   });
 }
 

@@ -24,7 +24,7 @@ struct LuFactors {
 struct FactorSet {
   LuFactors lu;
   unsigned ver;      // counts the set's rebuilds
-  int pad;
+  int banded;        // of a slot's first set: its steps solve with the LAPACK-form factors (a set needs row interchanges)
 };
 
 // All device arrays of one resolution class (slot-major).  Passed by value.
@@ -33,7 +33,6 @@ struct Bufs {
   double2* Nraw[2];     // nonlinear terms without base-flow terms [slot][3][N][Hp]
   double2* om;          // curl of the current iterate [slot][3][N][Hp]
   FactorSet* sets;      // [slot][4 mats]
-  int* banded;          // [slot] the step solves with the sets' LAPACK-form factors (one needs row interchanges)
   double* SE;           // block inverses (block_factor, solve.hpp) [slot][4 mats][P pairs][blk_count(N)][16],
                         // element (row, column) at 4 column + row
   LuSpec* spec;         // [slot][4] the matrix each factor set holds

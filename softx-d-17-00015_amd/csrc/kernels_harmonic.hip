@@ -528,7 +528,7 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   // (harmonics without a mode or with none to solve hold zeros and stay so)
   if (solver) {
     double* const x[1] = {(double*)(V + 2 * VC + lhs) + (bl.col & 1)};
-    if (!BAND || !B.banded[slot]) blk_solve(EP, N, bl, LT, x, 2 * GH);
+    if (!BAND || !B.sets[slot * 4].banded) blk_solve(EP, N, bl, LT, x, 2 * GH);
     else band_solve(G, B, slot, 2, 1, MAT_LNP, ps, V + wave, VC, GP, tid & 63);
   }
   BlkE<SM, 2> EH;
@@ -611,7 +611,7 @@ __device__ __forceinline__ void step_body(const Geo& G, const Bufs& B, const Ste
   if (solver) {
     double* xp = (double*)(V + lhs) + (bl.col & 1);
     double* const x[2] = {xp + (bl.mi ? 2 * VC : 0), xp + 4 * VC};
-    if (!BAND || !B.banded[slot]) blk_solve(EH, N, bl, LT, x, 2 * GH);
+    if (!BAND || !B.sets[slot * 4].banded) blk_solve(EH, N, bl, LT, x, 2 * GH);
     else band_solve(G, B, slot, 0, 3, MAT_LDP, ps, V + wave, VC, GP, tid & 63);
     if (!EARLY) influence_loads();
   }

@@ -808,7 +808,7 @@ __global__ void __launch_bounds__(256) k_matrices_t(Geo G, Bufs B, int slot0, in
     const int fm = lane >> 4, fp = (lane >> 1) & 7;
     const LuSpec A = matrix_spec(fm, prm);
     if (p0 == 0 && (lane & 15) == 0) hold(B, slot, A);
-    if (p0 == 0 && lane == 0) B.banded[slot] = 0;
+    if (p0 == 0 && lane == 0) B.sets[slot * 4].banded = 0;
     // spare lanes repeat the last pair
     block_factor<false>(G, B, slot, A, fm, p0 + min(fp, np - 1), lane & 1, prm.alpha, lap, nullptr);
   }
